@@ -195,7 +195,7 @@ struct PcgState {     // device-resident scalars of the PCG iteration
   int32_t breakdown_k;
   int32_t maxiter;
   int32_t converged;  // 1 if ||r_k|| <= rtol ||b||
-  int32_t pad;
+  int32_t aborted;    // 1 if a resident launch gave up waiting (grid_exchange.hpp)
 };
 
 struct NewtonStats {  // device-resident FP64 norms of one Newton step
@@ -352,6 +352,13 @@ struct Ctx {
   int pcg_pred[2][kPredSlots] = {{-1, -1, -1, -1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1, -1, -1, -1}};
   bool pcg_predict = true;
 
+  // one-launch PCG of small models (resident_solve.hip): the grid exchange's
+  // slots; epochs in use so far; the longest wait in ticks of the 100 MHz clock (ONSAS_RESIDENT_TICKS)
+  bool pcg_resident = false;  // ONSAS_PCG_RESIDENT=0 turns it off (read at finalize)
+  unsigned long long* d_gslots = nullptr;
+  uint32_t gslot_epoch = 1;
+  long long gslot_ticks = 20000000;  // 0.2 s
+
   // aggregation multigrid preconditioner (built on its first use)
   Amg amg;
 
@@ -424,6 +431,11 @@ int launch_residual(Ctx* c);                                    // d_res, partia
 // device by the factor minimising ||b - a K x0||
 int launch_pcg_solve(Ctx* c, const double* b_dev, bool forcing, int* iters, double* relres,
                      int* converged, int* breakdown, const void* x0 = nullptr, int expect = -1);
+// ---- resident_solve.hip ----
+bool pcg_resident_fits(const Ctx* c);
+int pcg_resident_alloc(Ctx* c);                                 // at finalize
+int launch_pcg_resident(Ctx* c);                                // after the init kernels
+
 double linear_rtol(const Ctx* c);                               // configured / default rtol
 int reset_forcing(Ctx* c);                                      // new load step
 int launch_gmres_solve(Ctx* c, const double* b_dev, int* iters, double* relres, int* converged);

@@ -324,6 +324,7 @@ __global__ __launch_bounds__(NT) void k_pcg_init_finalize(const double* __restri
     st->breakdown_k = -1;
     st->maxiter = maxiter;
     st->converged = 0;
+    st->aborted = 0;
   }
 }
 
@@ -1001,6 +1002,16 @@ int build_pcg_graph(Ctx* c, int slot, int iters) {
   return ONSAS_OK;
 }
 
+// most iterations of a solve that runs as one launch (a bound on its time)
+constexpr int kMaxResidentIters = 100000;
+
+void pcg_result(const PcgState& ps, int* iters, double* relres, int* converged, int* breakdown) {
+  *iters = ps.breakdown ? ps.breakdown_k : ps.iters;
+  *converged = ps.converged;
+  *breakdown = ps.breakdown;
+  *relres = ps.bb > 0 ? std::sqrt(ps.rr_last / ps.bb) : 0.0;
+}
+
 template <typename KT>
 int pcg_solve_t(Ctx* c, const double* b_dev, bool forcing, const void* x0, int expect, int* iters,
                 double* relres, int* converged, int* breakdown) {
@@ -1026,34 +1037,57 @@ int pcg_solve_t(Ctx* c, const double* b_dev, bool forcing, const void* x0, int e
   // d0 = D^-1 r_0 / theta into the finest level's d0
   void* amg_d0 = nullptr;
   const KT d0_scale = amg ? (KT)amg_fine_smoother(c, &amg_d0) : KT(1);
-  if (x0) {
-    // warm start: t = K x0 (into q, free until the first iteration), the scale
-    // a minimising ||b - a t||, then x = a x0 and r = b - a t
-    const int64_t rstride = c->ell_rounds ? 64 * c->nslices : 64;
-    hipLaunchKernelGGL(k_spmv_sell<KT>, dim3(grid_for(c->nslices, 4)), dim3(256), 0, s,
-                       c->d_sell_ptr, c->d_slice_rounds, rstride, c->d_sell_col,
-                       (const KT*)c->d_Ksell, (const KT*)x0, (KT*)c->d_pq, c->nslices, c->nn);
-    hipLaunchKernelGGL(k_warm_dots<KT>, dim3(np), dim3(NT), 0, s, b_dev, c->d_fixmask,
-                       (const KT*)c->d_pq, part(c, kPartPQ), part(c, kPartRZ1), np, c->chunk, c->nn);
-    hipLaunchKernelGGL(k_warm_init<KT>, dim3(np), dim3(NT), 0, s, b_dev, c->d_fixmask,
-                       (const KT*)x0, (const KT*)c->d_pq, part(c, kPartPQ), part(c, kPartRZ1),
-                       (const KT*)c->d_Dinv, d0_scale, (KT*)c->d_px, (KT*)c->d_pr,
-                       amg ? (KT*)amg_d0 : (KT*)c->d_pz, part(c, kPartRZ0), part(c, kPartRR),
-                       part(c, kPartBB), np, c->chunk, c->nn);
-  } else if (amg) {
-    hipLaunchKernelGGL(k_pcg_init_r<KT>, dim3(np), dim3(NT), 0, s, b_dev, c->d_fixmask,
-                       (KT*)c->d_px, (KT*)c->d_pr, part(c, kPartRR), part(c, kPartBB),
-                       (const KT*)c->d_Dinv, d0_scale, (KT*)amg_d0, np, c->chunk, c->nn);
-  } else {
-    hipLaunchKernelGGL(k_pcg_init<KT>, dim3(np), dim3(NT), 0, s, b_dev, c->d_fixmask,
-                       (const KT*)c->d_Dinv, (KT*)c->d_px, (KT*)c->d_pr, (KT*)c->d_pz,
-                       part(c, kPartRZ0), part(c, kPartRR), part(c, kPartBB), np, c->chunk, c->nn);
-  }
+  auto init_vectors = [&]() {
+    if (x0) {
+      // warm start: t = K x0 (into q, free until the first iteration), the scale
+      // a minimising ||b - a t||, then x = a x0 and r = b - a t
+      const int64_t rstride = c->ell_rounds ? 64 * c->nslices : 64;
+      hipLaunchKernelGGL(k_spmv_sell<KT>, dim3(grid_for(c->nslices, 4)), dim3(256), 0, s,
+                         c->d_sell_ptr, c->d_slice_rounds, rstride, c->d_sell_col,
+                         (const KT*)c->d_Ksell, (const KT*)x0, (KT*)c->d_pq, c->nslices, c->nn);
+      hipLaunchKernelGGL(k_warm_dots<KT>, dim3(np), dim3(NT), 0, s, b_dev, c->d_fixmask,
+                         (const KT*)c->d_pq, part(c, kPartPQ), part(c, kPartRZ1), np, c->chunk, c->nn);
+      hipLaunchKernelGGL(k_warm_init<KT>, dim3(np), dim3(NT), 0, s, b_dev, c->d_fixmask,
+                         (const KT*)x0, (const KT*)c->d_pq, part(c, kPartPQ), part(c, kPartRZ1),
+                         (const KT*)c->d_Dinv, d0_scale, (KT*)c->d_px, (KT*)c->d_pr,
+                         amg ? (KT*)amg_d0 : (KT*)c->d_pz, part(c, kPartRZ0), part(c, kPartRR),
+                         part(c, kPartBB), np, c->chunk, c->nn);
+    } else if (amg) {
+      hipLaunchKernelGGL(k_pcg_init_r<KT>, dim3(np), dim3(NT), 0, s, b_dev, c->d_fixmask,
+                         (KT*)c->d_px, (KT*)c->d_pr, part(c, kPartRR), part(c, kPartBB),
+                         (const KT*)c->d_Dinv, d0_scale, (KT*)amg_d0, np, c->chunk, c->nn);
+    } else {
+      hipLaunchKernelGGL(k_pcg_init<KT>, dim3(np), dim3(NT), 0, s, b_dev, c->d_fixmask,
+                         (const KT*)c->d_Dinv, (KT*)c->d_px, (KT*)c->d_pr, (KT*)c->d_pz,
+                         part(c, kPartRZ0), part(c, kPartRR), part(c, kPartBB), np, c->chunk, c->nn);
+    }
+  };
+  init_vectors();
   const bool f = forcing && c->lin.forcing;
   hipLaunchKernelGGL(k_pcg_init_finalize, dim3(1), dim3(NT), 0, s, part(c, kPartBB),
                      part(c, kPartF2), &c->d_sc->pcg, &c->d_sc->nwt, rtol, maxiter, np, f ? 1 : 0,
                      c->lin.newton_tol, c->lin.eta_max > 0 ? c->lin.eta_max : 0.1,
                      c->lin.eta_first > 0 ? c->lin.eta_first : 1e-3, kForcingGuard);
+  if (c->pcg_resident && !amg && maxiter <= kMaxResidentIters) {
+    ONSAS_TRY(launch_pcg_resident(c));
+    ONSAS_HIP_TRY(c, hipMemcpyAsync(&c->h_sc->pcg, &c->d_sc->pcg, sizeof(PcgState),
+                                    hipMemcpyDeviceToHost, s));
+    ONSAS_HIP_TRY(c, hipStreamSynchronize(s));
+    PcgState& ps = c->h_sc->pcg;
+    c->gslot_epoch += (ps.aborted ? (uint32_t)maxiter : (uint32_t)ps.k) + 2;
+    if (!ps.aborted) {
+      pcg_result(ps, iters, relres, converged, breakdown);
+      return ONSAS_OK;
+    }
+    // a wait expired (the GPU was too busy to hold the whole grid): this solve
+    // starts again on the kernels below, which the context keeps to from here
+    c->pcg_resident = false;
+    ps.k = ps.done = ps.iters = ps.breakdown = ps.converged = ps.aborted = 0;
+    ps.breakdown_k = -1;
+    ps.rr_last = ps.bb;
+    ONSAS_HIP_TRY(c, hipMemcpyAsync(&c->d_sc->pcg, &ps, sizeof(PcgState), hipMemcpyHostToDevice, s));
+    init_vectors();
+  }
   if (amg) {
     // a (warm) start that already meets the tolerance stops in the prologue of
     // the cycle's first fine-level product, before the preconditioner
@@ -1159,11 +1193,7 @@ int pcg_solve_t(Ctx* c, const double* b_dev, bool forcing, const void* x0, int e
     first = false;
     if (ps.done || ps.breakdown) break;
   }
-  const PcgState& ps = c->h_sc->pcg;
-  *iters = ps.breakdown ? ps.breakdown_k : ps.iters;
-  *converged = ps.converged;
-  *breakdown = ps.breakdown;
-  *relres = ps.bb > 0 ? std::sqrt(ps.rr_last / ps.bb) : 0.0;
+  pcg_result(c->h_sc->pcg, iters, relres, converged, breakdown);
   return ONSAS_OK;
 }
 
