@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "../../include/onsas_hip.h"
+#include "grid_exchange.hpp"
 #include "host_setup.hpp"
 
 namespace onsas {
@@ -352,10 +353,11 @@ struct Ctx {
   int pcg_pred[2][kPredSlots] = {{-1, -1, -1, -1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1, -1, -1, -1}};
   bool pcg_predict = true;
 
-  // one-launch PCG of small models (resident_solve.hip): the grid exchange's
+  // one-launch PCG and GMRES of small models (resident_solve.hip): the exchange's
   // slots; epochs in use so far; the longest wait in ticks of the 100 MHz clock (ONSAS_RESIDENT_TICKS)
   bool pcg_resident = false;  // ONSAS_PCG_RESIDENT=0 turns it off (read at finalize)
-  unsigned long long* d_gslots = nullptr;
+  unsigned long long* d_gslots = nullptr;    // the tail of d_part's allocation
+  unsigned long long* d_gmslots = nullptr;  // the same for GMRES (on its first use)
   uint32_t gslot_epoch = 1;
   long long gslot_ticks = 20000000;  // 0.2 s
 
@@ -433,8 +435,12 @@ int launch_pcg_solve(Ctx* c, const double* b_dev, bool forcing, int* iters, doub
                      int* converged, int* breakdown, const void* x0 = nullptr, int expect = -1);
 // ---- resident_solve.hip ----
 bool pcg_resident_fits(const Ctx* c);
-int pcg_resident_alloc(Ctx* c);                                 // at finalize
+void pcg_resident_setup(Ctx* c);                                // at finalize
 int launch_pcg_resident(Ctx* c);                                // after the init kernels
+int launch_gmres_resident(Ctx* c, const double* b_dev, int m, int maxiter, double rtol, bool* ran,
+                          int* iters, double* relres, int* converged);
+// most iterations of a solve that runs as one launch (a bound on its time)
+constexpr int kMaxResidentIters = 100000;
 
 double linear_rtol(const Ctx* c);                               // configured / default rtol
 int reset_forcing(Ctx* c);                                      // new load step

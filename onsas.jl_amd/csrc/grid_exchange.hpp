@@ -30,6 +30,7 @@
 namespace onsas {
 
 constexpr int kMaxGridWg = 128;  // workgroups of a resident launch (two polled slots per lane)
+constexpr size_t kGridSlotWords = 6 * kMaxGridWg;  // the PCG's slots: a one- and a two-value sum
 
 template <typename T>
 __device__ inline T agent_load(const T* p) {
@@ -79,6 +80,37 @@ __device__ inline void wg_sum(double (&v)[NV], double* sh) {
   wg_total<NV, T>(v, sh);
 }
 
+// One value of a slot: its two words once both carry the epoch; false once the
+// launch is aborted.
+template <int NW>
+__device__ inline bool poll_words(const unsigned long long* s, uint32_t epoch, const GridSlots& gs,
+                                  unsigned long long (&w)[NW]) {
+  long long t0 = 0;
+  for (uint32_t spin = 0;; ++spin) {
+    bool ready = true;
+#pragma unroll
+    for (int q = 0; q < NW; ++q) w[q] = agent_load(s + q);
+#pragma unroll
+    for (int q = 0; q < NW; ++q) ready = ready && (uint32_t)(w[q] >> 32) == epoch;
+    if (ready) return true;
+    if ((spin & 63u) == 0) {
+      const long long now = wall_clock64();
+      if (spin == 0) t0 = now;
+      if (now - t0 > gs.limit || agent_load(gs.abort) != 0) {
+        agent_store(gs.abort, 1);
+        return false;
+      }
+    }
+  }
+}
+__device__ inline double words_value(unsigned long long hi, unsigned long long lo) {
+  return __longlong_as_double((long long)((hi << 32) | (lo & 0xffffffffull)));
+}
+__device__ inline unsigned long long value_word(double p, uint32_t epoch, bool low) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(p);
+  return ((unsigned long long)epoch << 32) | (low ? (b & 0xffffffffull) : (b >> 32));
+}
+
 // Sum over all workgroups of the launch; false once the launch is aborted (the
 // same answer for every thread of the workgroup).  sh: NV * (T / 64 + 1) + 1
 // doubles.  With DRAIN the caller's stores are visible to every workgroup that
@@ -90,43 +122,22 @@ __device__ inline bool grid_sum(double (&v)[NV], const GridSlots& gs, uint32_t e
   if (threadIdx.x < 64) {
     wg_total<NV, T>(v, sh);
     const int lane = threadIdx.x;
-    const unsigned long long tag = (unsigned long long)epoch << 32;
     unsigned long long* mine = gs.words + (size_t)(2 * NV) * blockIdx.x;
     if (lane < 2 * NV) {
       double p = v[0];
 #pragma unroll
       for (int q = 1; q < NV; ++q) p = (lane >> 1) == q ? v[q] : p;
-      const unsigned long long b = (unsigned long long)__double_as_longlong(p);
-      agent_store(mine + lane, tag | ((lane & 1) ? (b & 0xffffffffull) : (b >> 32)));
+      agent_store(mine + lane, value_word(p, epoch, lane & 1));
     }
     bool ok = true;
     double acc[NV];
 #pragma unroll
     for (int q = 0; q < NV; ++q) acc[q] = 0;
-    for (int g = lane; g < gs.nwg; g += 64) {
-      const unsigned long long* s = gs.words + (size_t)(2 * NV) * g;
+    for (int g = lane; ok && g < gs.nwg; g += 64) {
       unsigned long long w[2 * NV];
-      long long t0 = 0;
-      for (uint32_t spin = 0;; ++spin) {
-        bool ready = true;
+      ok = poll_words<2 * NV>(gs.words + (size_t)(2 * NV) * g, epoch, gs, w);
 #pragma unroll
-        for (int q = 0; q < 2 * NV; ++q) w[q] = agent_load(s + q);
-#pragma unroll
-        for (int q = 0; q < 2 * NV; ++q) ready = ready && (uint32_t)(w[q] >> 32) == epoch;
-        if (ready) break;
-        if ((spin & 63u) == 0) {
-          const long long now = wall_clock64();
-          if (spin == 0) t0 = now;
-          if (now - t0 > gs.limit || agent_load(gs.abort) != 0) {
-            agent_store(gs.abort, 1);
-            ok = false;
-            break;
-          }
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < NV; ++q)
-        acc[q] += __longlong_as_double((long long)((w[2 * q] << 32) | (w[2 * q + 1] & 0xffffffffull)));
+      for (int q = 0; q < NV; ++q) acc[q] += words_value(w[2 * q], w[2 * q + 1]);
     }
     ok = __all(ok);
 #pragma unroll

@@ -1,6 +1,7 @@
-// resident_solve.hip -- block-Jacobi PCG of small and mid-size models as one
-// launch.  gfx950, wave64.
+// resident_solve.hip -- block-Jacobi PCG and GMRES of small and mid-size models,
+// each solve one launch.  gfx950, wave64.
 //
+// PCG.
 // The two-kernel iteration (k_pcg_A, k_pcg_B) of a model of a few thousand nodes
 // is bound by kernel boundaries: 8.2 + 4.7 us of kernel time and 1.5 us of gaps
 // an iteration at 1,680 nodes in FP32, where the bytes take 0.2 us.  Here the
@@ -12,6 +13,7 @@
 // The recurrences, the stop and breakdown rules and the scalars are those of
 // k_pcg_A / k_pcg_B (p = z + beta p, q = K z + beta q); only the order of the
 // sums differs.
+#include <cmath>
 #include <cstdlib>
 
 #include "engine.hpp"
@@ -171,6 +173,297 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs<KT> a) {
   }
 }
 
+// Restarted GMRES(m) with right block-Jacobi preconditioning (K D^-1 y = b,
+// x = D^-1 y), classical Gram-Schmidt twice, as gmres_solve_t in
+// solver_kernels.hip, whose iteration is some ten launches and three host round
+// trips: 157 us at 720 nodes in FP64, and 14.5 us here (289 -> 27 ms for the two
+// load steps of a 9 x 8 x 7 box).  A workgroup holds R = T / L rows: the
+// tangent in registers, the basis V of its 3 R dofs and the working vector w in
+// LDS, the Hessenberg column and its rotations in LDS (every workgroup computes
+// the same ones).  An iteration is three grid exchanges: the dot products of
+// each Gram-Schmidt pass (a value per basis vector, four threads a value), and
+// |w| together with t = D^-1 w of the next product, which is published before w
+// is scaled: K D^-1 v = K t / |w|.
+constexpr int kGmresThreads = 256;
+constexpr int kGmresMax = 60;    // most basis vectors of the resident kernel (four threads each)
+constexpr int kGmresSlot = 128;  // words of a workgroup's slot: 64 values
+
+template <typename KT>
+struct GmresArgs {
+  const int32_t* sell_ptr;
+  const int32_t* slice_rounds;
+  int64_t rstride;
+  const int32_t* scol;
+  const KT* sval;
+  const KT* Dinv;
+  const double* b;
+  const uint8_t* mask;
+  KT* x;
+  KT* t;  // D^-1 w, read by the neighbouring workgroups
+  PcgState* st;
+  unsigned long long* slots;  // two regions of kMaxGridWg slots, used in turn
+  uint32_t base;
+  long long limit;
+  int64_t nn;
+  int m, maxiter;
+  double rtol;
+};
+
+// LDS of one workgroup: packed triangle of R, two coefficient columns, rotations,
+// right-hand side, solution, four scalars; then w and the m + 1 basis vectors,
+// each padded by 4 values so that four threads of 16 vectors hit distinct banks
+inline size_t gmres_lds(int m, int rows, size_t kt) {
+  return sizeof(double) * ((size_t)m * (m + 1) / 2 + 6 * 64 + 4) +
+         kt * (size_t)(m + 2) * (3 * rows + 4);
+}
+
+template <typename KT, int L, int NB>
+__global__ __launch_bounds__(kGmresThreads) void k_gmres_resident(GmresArgs<KT> a) {
+  constexpr int T = kGmresThreads, R = T / L, DN = 3 * R, S = DN + 4;
+  extern __shared__ double lds[];
+  const int m = a.m;
+  double* Rm = lds;  // column j at j (j + 1) / 2
+  double* h1 = Rm + m * (m + 1) / 2;
+  double *h2 = h1 + 64, *cs = h2 + 64, *sn = cs + 64, *gv = sn + 64, *yv = gv + 64, *sc = yv + 64;
+  KT* w = (KT*)(sc + 4);
+  KT* V = w + S;
+  const int t = threadIdx.x;
+  const int lane = t & 63;
+  const int ph = t % L, lrow = t / L;
+  const int64_t i = (int64_t)blockIdx.x * R + lrow;
+  const bool row = i < a.nn;
+  // a thread's dof (t < DN)
+  const bool isd = t < DN;
+  const int comp = t % 3, n0 = t - comp;
+  const int64_t dof = (int64_t)blockIdx.x * DN + t;
+  const bool live = isd && dof < 3 * a.nn;
+  const bool freed = live && !((a.mask[live ? dof / 3 : 0] >> comp) & 1u);
+  const double bd = freed ? a.b[dof] : 0.0;
+  KT d0 = 0, d1 = 0, d2 = 0, xs = 0;
+  if (live) {
+    const KT* D = a.Dinv + 9 * (dof / 3) + 3 * comp;
+    d0 = D[0];
+    d1 = D[1];
+    d2 = D[2];
+  }
+  KT v[NB][9];
+  uint32_t cj[NB];
+  {
+    const int64_t s = row ? i >> 6 : 0;
+    const int32_t b0 = a.sell_ptr[s], rounds = a.slice_rounds[s];
+    const int l = (int)(i & 63);
+#pragma unroll
+    for (int q = 0; q < NB; ++q) {
+      const int mr = ph + L * q;
+      const bool has = row && mr < rounds;
+      const int64_t b = b0 + a.rstride * (has ? mr : 0);
+      cj[q] = has ? 3u * (uint32_t)sizeof(KT) * (uint32_t)a.scol[b + l] : 0u;
+#pragma unroll
+      for (int e = 0; e < 9; ++e) v[q][e] = has ? a.sval[9 * b + 64 * e + l] : KT(0);
+    }
+  }
+  GridSlots gs{a.slots, (int)gridDim.x, &a.st->aborted, a.limit};
+  uint32_t ep = a.base;
+  auto region = [&](uint32_t e) { return a.slots + (size_t)(e & 1u) * kMaxGridWg * kGmresSlot; };
+
+  // w = scale K y, y shared through device memory
+  auto product = [&](const KT* y, double scale) {
+    KT yj[NB][3];
+#pragma unroll
+    for (int q = 0; q < NB; ++q)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) yj[q][c] = agent_load((const KT*)((const char*)y + cj[q]) + c);
+    KT a0 = 0, a1 = 0, a2 = 0;
+#pragma unroll
+    for (int q = 0; q < NB; ++q) {
+      a0 += v[q][0] * yj[q][0] + v[q][1] * yj[q][1] + v[q][2] * yj[q][2];
+      a1 += v[q][3] * yj[q][0] + v[q][4] * yj[q][1] + v[q][5] * yj[q][2];
+      a2 += v[q][6] * yj[q][0] + v[q][7] * yj[q][1] + v[q][8] * yj[q][2];
+    }
+    a0 = group_sum<L>(a0);
+    a1 = group_sum<L>(a1);
+    a2 = group_sum<L>(a2);
+    __syncthreads();  // the last readers of w are done
+    if (ph < 3) {
+      const KT ac = ph == 0 ? a0 : (ph == 1 ? a1 : a2);
+      w[3 * lrow + ph] = (KT)((double)ac * scale);
+    }
+    __syncthreads();
+  };
+  // |w|^2 over the launch, with t = D^-1 w published before it; `between` runs on
+  // the last wave while the first one waits for the other workgroups
+  auto norm_publish = [&](double& n2, auto between) -> bool {
+    ++ep;
+    if (live) agent_store(a.t + dof, d0 * w[n0] + d1 * w[n0 + 1] + d2 * w[n0 + 2]);
+    double p = 0;
+    if (t < 64) {
+      for (int d = lane; d < DN; d += 64) p += (double)w[d] * (double)w[d];
+      p = wave_sum(p);
+    }
+    stores_done();
+    __syncthreads();
+    if (t < 64) {
+      unsigned long long* reg = region(ep);
+      if (lane < 2) agent_store(reg + (size_t)kGmresSlot * blockIdx.x + lane, value_word(p, ep, lane & 1));
+      bool ok = true;
+      double acc = 0;
+      for (int g = lane; ok && g < gs.nwg; g += 64) {
+        unsigned long long wd[2];
+        ok = poll_words<2>(reg + (size_t)kGmresSlot * g, ep, gs, wd);
+        acc += words_value(wd[0], wd[1]);
+      }
+      ok = __all(ok);
+      acc = wave_sum(acc);
+      if (lane == 0) {
+        sc[0] = acc;
+        sc[1] = ok ? 1.0 : 0.0;
+      }
+    } else if (t >= T - 64) {
+      between();
+    }
+    __syncthreads();
+    n2 = sc[0];
+    return sc[1] != 0.0;
+  };
+  // h[0 .. nv) = V' w over the launch
+  auto dots = [&](int nv, double* h) -> bool {
+    ++ep;
+    const int q = t >> 2, seg = t & 3;
+    double acc = 0;
+    if (q < nv) {
+      const KT* vq = V + q * S;
+      for (int d = seg; d < DN; d += 4) acc += (double)vq[d] * (double)w[d];
+    }
+    acc = group_sum<4>(acc);
+    unsigned long long* reg = region(ep);
+    bool ok = true;
+    double sum = 0;
+    if (q < nv) {
+      if (seg < 2)
+        agent_store(reg + (size_t)kGmresSlot * blockIdx.x + 2 * q + seg, value_word(acc, ep, seg));
+      for (int g = seg; ok && g < gs.nwg; g += 4) {
+        unsigned long long wd[2];
+        ok = poll_words<2>(reg + (size_t)kGmresSlot * g + 2 * q, ep, gs, wd);
+        sum += words_value(wd[0], wd[1]);
+      }
+    }
+    sum = group_sum<4>(sum);
+    if (q < nv && seg == 0) h[q] = sum;
+    return __syncthreads_and(ok);
+  };
+  auto subtract = [&](int nv, const double* h) {
+    if (isd) {
+      double s = 0;
+      for (int q = 0; q < nv; ++q) s += h[q] * (double)V[q * S + t];
+      w[t] = (KT)((double)w[t] - s);
+    }
+    __syncthreads();
+  };
+
+  double beta0 = -1, beta = 0, n2 = 0;
+  int total = 0;
+  for (bool first = true;; first = false) {
+    // r = b - K x on the free dofs
+    KT rv = freed ? (KT)bd : KT(0);
+    if (!first) {
+      if (live) agent_store(a.x + dof, xs);
+      stores_done();
+      __syncthreads();
+      // the exchange that makes x visible (its value is not used)
+      ++ep;
+      if (t < 64) {
+        unsigned long long* reg = region(ep);
+        if (lane < 2) agent_store(reg + (size_t)kGmresSlot * blockIdx.x + lane, value_word(0.0, ep, lane & 1));
+        bool ok = true;
+        for (int g = lane; ok && g < gs.nwg; g += 64) {
+          unsigned long long wd[2];
+          ok = poll_words<2>(reg + (size_t)kGmresSlot * g, ep, gs, wd);
+        }
+        ok = __all(ok);
+        if (lane == 0) sc[1] = ok ? 1.0 : 0.0;
+      }
+      __syncthreads();
+      if (sc[1] == 0.0) return;
+      product(a.x, 1.0);
+      rv = freed ? (KT)(bd - (double)w[isd ? t : 0]) : KT(0);
+      __syncthreads();
+    }
+    if (isd) w[t] = rv;
+    __syncthreads();
+    if (!norm_publish(n2, [] {})) return;
+    beta = sqrt(n2);
+    if (beta0 < 0) beta0 = beta;
+    if (!(beta > a.rtol * beta0) || total >= a.maxiter || beta0 == 0) break;
+    double inv = 1.0 / beta;
+    if (isd) V[t] = (KT)((double)w[t] * inv);
+    double g = beta;
+    int k = 0;
+    for (int j = 0; j < m; ++j) {
+      product(a.t, inv);
+      if (!dots(j + 1, h1)) return;
+      subtract(j + 1, h1);
+      if (!dots(j + 1, h2)) return;
+      subtract(j + 1, h2);
+      // the earlier rotations applied to the new column, while the norm is summed
+      auto rotate = [&] {
+        if (t != T - 64) return;
+        double* col = Rm + j * (j + 1) / 2;
+        double e = h1[0] + h2[0];
+        for (int q = 0; q < j; ++q) {
+          const double f = h1[q + 1] + h2[q + 1];
+          col[q] = cs[q] * e + sn[q] * f;
+          e = -sn[q] * e + cs[q] * f;
+        }
+        sc[2] = e;
+      };
+      if (!norm_publish(n2, rotate)) return;
+      const double hn = sqrt(n2), e = sc[2], r = hypot(e, hn);
+      const double c = r > 0 ? e / r : 1.0, s = r > 0 ? hn / r : 0.0;
+      if (t == 0) {
+        Rm[j * (j + 1) / 2 + j] = r;
+        cs[j] = c;
+        sn[j] = s;
+        gv[j] = c * g;
+      }
+      g = -s * g;
+      ++total;
+      k = j + 1;
+      if (fabs(g) <= a.rtol * beta0 || total >= a.maxiter || !(hn > 0)) break;
+      inv = 1.0 / hn;
+      if (isd) V[(j + 1) * S + t] = (KT)((double)w[t] * inv);
+    }
+    __syncthreads();
+    if (t < 64) {  // R y = g, a lane per unknown
+      double y = lane < k ? gv[lane] : 0.0;
+      for (int q = k - 1; q >= 0; --q) {
+        const double* col = Rm + q * (q + 1) / 2;
+        const double d = col[q];
+        const double yq = d != 0 ? read_lane(y, q) / d : 0.0;
+        if (lane < q) y -= col[lane] * yq;
+        if (lane == q) yv[q] = yq;
+      }
+    }
+    __syncthreads();
+    if (isd) {
+      double s = 0;
+      for (int q = 0; q < k; ++q) s += yv[q] * (double)V[q * S + t];
+      w[t] = (KT)s;
+    }
+    __syncthreads();
+    if (live) xs += d0 * w[n0] + d1 * w[n0 + 1] + d2 * w[n0 + 2];
+    __syncthreads();
+  }
+  if (live) a.x[dof] = xs;
+  if (blockIdx.x == 0 && t == 0) {
+    a.st->rr_last = beta * beta;
+    a.st->bb = beta0 * beta0;
+    a.st->iters = total;
+    a.st->k = (int32_t)(ep - a.base);  // epochs used
+    a.st->converged = (beta0 == 0 || beta <= a.rtol * beta0) ? 1 : 0;
+    a.st->done = 1;
+  }
+}
+
 // L lanes a row: 4 for rows of up to 16 blocks (structured meshes: 15), 8 up to 32
 inline int lanes_per_row(const Ctx* c) { return c->ell_width <= 16 ? 4 : 8; }
 constexpr int kResidentBlocks = 4;  // blocks a lane keeps in registers
@@ -240,6 +533,38 @@ int resident_t(Ctx* c) {
   return ONSAS_OK;
 }
 
+template <typename KT, int L>
+int gmres_t(Ctx* c, const double* b_dev, int m, int maxiter, double rtol) {
+  GmresArgs<KT> a{};
+  a.sell_ptr = c->d_sell_ptr;
+  a.slice_rounds = c->d_slice_rounds;
+  a.rstride = c->ell_rounds ? 64 * c->nslices : 64;
+  a.scol = c->d_sell_col;
+  a.sval = (const KT*)c->d_Ksell;
+  a.Dinv = (const KT*)c->d_Dinv;
+  a.b = b_dev;
+  a.mask = c->d_fixmask;
+  a.x = (KT*)c->d_px;
+  a.t = (KT*)c->d_pz;
+  a.st = &c->d_sc->pcg;
+  a.slots = c->d_gmslots;
+  a.base = c->gslot_epoch;
+  a.limit = c->gslot_ticks;
+  a.nn = c->nn;
+  a.m = m;
+  a.maxiter = maxiter;
+  a.rtol = rtol;
+  auto kern = k_gmres_resident<KT, L, kResidentBlocks>;
+  const size_t lds = gmres_lds(m, kGmresThreads / L, sizeof(KT));
+  ONSAS_HIP_TRY(c, hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  const int R = kGmresThreads / L;
+  hipLaunchKernelGGL(kern, dim3((unsigned)((c->nn + R - 1) / R)), dim3(kGmresThreads), lds,
+                     c->stream, a);
+  ONSAS_HIP_TRY(c, hipGetLastError());
+  return ONSAS_OK;
+}
+
 }  // namespace
 
 // Whether a block-Jacobi PCG of this model runs as one launch: rows short enough
@@ -250,24 +575,68 @@ bool pcg_resident_fits(const Ctx* c) {
          resident_shape(c).grid <= kMaxGridWg;
 }
 
-int pcg_resident_alloc(Ctx* c) {
+void pcg_resident_setup(Ctx* c) {
   const char* e = std::getenv("ONSAS_PCG_RESIDENT");
   c->pcg_resident = pcg_resident_fits(c) && !(e && e[0] == '0');
   if (const char* t = std::getenv("ONSAS_RESIDENT_TICKS")) c->gslot_ticks = std::atoll(t);
-  if (!c->pcg_resident) return ONSAS_OK;
-  const size_t words = 6 * (size_t)kMaxGridWg * sizeof(unsigned long long);
-  ONSAS_HIP_TRY(c, hipMalloc((void**)&c->d_gslots, words));
-  ONSAS_HIP_TRY(c, hipMemsetAsync(c->d_gslots, 0, words, c->stream));
+}
+
+// before the epochs wrap: clear the slots' marks and begin again
+static int renew_epochs(Ctx* c) {
+  if (c->gslot_epoch <= 0xf0000000u) return ONSAS_OK;
+  ONSAS_HIP_TRY(c, hipMemsetAsync(c->d_gslots, 0,
+                                  kGridSlotWords * sizeof(unsigned long long), c->stream));
+  if (c->d_gmslots)
+    ONSAS_HIP_TRY(c, hipMemsetAsync(c->d_gmslots, 0, 2 * (size_t)kMaxGridWg * kGmresSlot *
+                                                         sizeof(unsigned long long), c->stream));
+  c->gslot_epoch = 1;
   return ONSAS_OK;
 }
 
 int launch_pcg_resident(Ctx* c) {
-  if (c->gslot_epoch > 0xf0000000u) {  // the epochs wrap: clear the slots' marks
-    ONSAS_HIP_TRY(c, hipMemsetAsync(c->d_gslots, 0,
-                                    6 * (size_t)kMaxGridWg * sizeof(unsigned long long), c->stream));
-    c->gslot_epoch = 1;
-  }
+  ONSAS_TRY(renew_epochs(c));
   return c->precision == ONSAS_PRECISION_FP64 ? resident_t<double>(c) : resident_t<float>(c);
+}
+
+// GMRES of the current tangent in one launch, where the model and the restart
+// length fit (a basis of up to kGmresMax vectors in 150 KiB of LDS a workgroup);
+// *ran = false leaves the solve to the general path.
+int launch_gmres_resident(Ctx* c, const double* b_dev, int m, int maxiter, double rtol, bool* ran,
+                          int* iters, double* relres, int* converged) {
+  *ran = false;
+  const int L = lanes_per_row(c), R = kGmresThreads / L;
+  if (!c->pcg_resident || m > kGmresMax || maxiter > kMaxResidentIters ||
+      (c->nn + R - 1) / R > kMaxGridWg || gmres_lds(m, R, c->kt) > 150 * 1024)
+    return ONSAS_OK;
+  hipStream_t s = c->stream;
+  const size_t bytes = 2 * (size_t)kMaxGridWg * kGmresSlot * sizeof(unsigned long long);
+  if (!c->d_gmslots) {
+    ONSAS_HIP_TRY(c, hipMalloc((void**)&c->d_gmslots, bytes));
+    ONSAS_HIP_TRY(c, hipMemsetAsync(c->d_gmslots, 0, bytes, s));
+  }
+  ONSAS_TRY(renew_epochs(c));
+  ONSAS_HIP_TRY(c, hipMemsetAsync(&c->d_sc->pcg, 0, sizeof(PcgState), s));
+  if (c->precision == ONSAS_PRECISION_FP64)
+    ONSAS_TRY(L == 4 ? (gmres_t<double, 4>(c, b_dev, m, maxiter, rtol))
+                     : (gmres_t<double, 8>(c, b_dev, m, maxiter, rtol)));
+  else
+    ONSAS_TRY(L == 4 ? (gmres_t<float, 4>(c, b_dev, m, maxiter, rtol))
+                     : (gmres_t<float, 8>(c, b_dev, m, maxiter, rtol)));
+  ONSAS_HIP_TRY(c, hipMemcpyAsync(&c->h_sc->pcg, &c->d_sc->pcg, sizeof(PcgState),
+                                  hipMemcpyDeviceToHost, s));
+  ONSAS_HIP_TRY(c, hipStreamSynchronize(s));
+  const PcgState& ps = c->h_sc->pcg;
+  // an iteration takes 3 epochs, a restart 2
+  c->gslot_epoch += (ps.aborted ? 5u * ((uint32_t)maxiter + 2) : (uint32_t)ps.k) + 2;
+  if (ps.aborted) {
+    c->pcg_resident = false;
+    return ONSAS_OK;
+  }
+  *ran = true;
+  *iters = ps.iters;
+  *relres = ps.bb > 0 ? std::sqrt(ps.rr_last / ps.bb) : 0.0;
+  *converged = ps.converged;
+  return ONSAS_OK;
 }
 
 }  // namespace onsas

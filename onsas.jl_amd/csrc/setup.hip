@@ -411,7 +411,8 @@ int finalize_model(Ctx* c) {
   ONSAS_TRY(dev_alloc(c, (void**)&c->d_nodal, sizeof(double) * n));
   for (void** v : {&c->d_px, &c->d_pr, &c->d_pz, &c->d_pp0, &c->d_pp1, &c->d_pq})
     ONSAS_TRY(dev_alloc(c, v, c->kt * n));
-  ONSAS_TRY(dev_alloc(c, (void**)&c->d_part, sizeof(double) * kPartArrays * kMaxPartials));
+  ONSAS_TRY(dev_alloc(c, (void**)&c->d_part, sizeof(double) * (kPartArrays * kMaxPartials + kGridSlotWords)));
+  c->d_gslots = (unsigned long long*)(c->d_part + kPartArrays * kMaxPartials);  // zero: no epoch
   ONSAS_TRY(dev_alloc(c, (void**)&c->d_sc, sizeof(Scalars)));
   ONSAS_HIP_TRY(c, hipHostMalloc((void**)&c->h_sc, sizeof(Scalars), hipHostMallocDefault));
   ONSAS_HIP_TRY(c, hipHostMalloc((void**)&c->h_stage, sizeof(double) * n, hipHostMallocDefault));
@@ -483,7 +484,7 @@ int finalize_model(Ctx* c) {
     ONSAS_TRY(dev_upload(c, &c->d_sell_col, scol.data(), scol.size()));
     ONSAS_TRY(dev_alloc(c, &c->d_Ksell, c->kt * 9 * (size_t)c->nsell));
   }
-  ONSAS_TRY(pcg_resident_alloc(c));
+  pcg_resident_setup(c);
   if (c->gather) ONSAS_TRY(build_gather(c, slots_h, rstride));
 
   if (c->gather) ONSAS_TRY(launch_gather_init(c));

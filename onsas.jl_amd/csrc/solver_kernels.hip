@@ -1002,9 +1002,6 @@ int build_pcg_graph(Ctx* c, int slot, int iters) {
   return ONSAS_OK;
 }
 
-// most iterations of a solve that runs as one launch (a bound on its time)
-constexpr int kMaxResidentIters = 100000;
-
 void pcg_result(const PcgState& ps, int* iters, double* relres, int* converged, int* breakdown) {
   *iters = ps.breakdown ? ps.breakdown_k : ps.iters;
   *converged = ps.converged;
@@ -1387,6 +1384,11 @@ int gmres_solve_t(Ctx* c, const double* b_dev, int* iters, double* relres, int* 
   hipStream_t s = c->stream;
   const int m = std::max(2, c->lin.gmres_restart > 0 ? c->lin.gmres_restart : 40);
   const int64_t n = 3 * c->nn;
+  const double rtol = linear_rtol(c);
+  const int maxiter = c->lin.maxiter > 0 ? c->lin.maxiter : (int)std::min<int64_t>(c->nfree, 1 << 30);
+  bool ran = false;
+  ONSAS_TRY(launch_gmres_resident(c, b_dev, m, maxiter, rtol, &ran, iters, relres, converged));
+  if (ran) return ONSAS_OK;
   if (c->gm_m < m) {
     for (void* p : {c->d_gm_V, c->d_gm_w, (void*)c->d_gm_h})
       if (p) (void)hipFree(p);
@@ -1407,8 +1409,6 @@ int gmres_solve_t(Ctx* c, const double* b_dev, int* iters, double* relres, int* 
   double* dpart = c->d_gm_h;
   double* dres = dpart + (size_t)(m + 2) * kMaxPartials;
   double* dcoef = dres + (m + 2);
-  const double rtol = linear_rtol(c);
-  const int maxiter = c->lin.maxiter > 0 ? c->lin.maxiter : (int)std::min<int64_t>(c->nfree, 1 << 30);
   const int64_t rstride = c->ell_rounds ? 64 * c->nslices : 64;
   const unsigned gn = grid_for(n, 256), gnn = grid_for(c->nn, 256), gs = grid_for(c->nslices, 4);
 
