@@ -15,6 +15,7 @@ namespace onsas {
 // quad_perm [1,0,3,2] and [2,3,0,1], row_half_mirror, row_mirror: each pairs a
 // lane with one outside the group (of 1, 2, 4, 8 lanes) summed so far
 constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppMirror = 0x140;
+constexpr int kDppRor8 = 0x128;  // row_ror:8, lane ^ 8 of a row of 16
 
 template <int CTRL>
 __device__ inline float dpp_move(float x) {
@@ -44,6 +45,9 @@ __device__ inline T group_sum(T x) {
   return x;
 }
 
+__device__ inline float read_lane(float x, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l));
+}
 __device__ inline double read_lane(double x, int l) {
   return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), l),
                           __builtin_amdgcn_readlane(__double2loint(x), l));
