@@ -248,6 +248,8 @@ struct Ctx {
   bool ell_rounds = false;
   int32_t ell_width = 0;              // rounds of the widest slice
   std::vector<int32_t> slice_rounds;  // rounds per slice
+  // few slices: the products give a slice four waves (sell_split.hpp)
+  bool sell_split = false;
   int32_t* d_slice_rounds = nullptr;
   int32_t* d_sell_ptr = nullptr;
   int32_t* d_sell_col = nullptr;
@@ -383,6 +385,9 @@ enum PartArray {  // rows of d_part
   kPartRZ0 = 0, kPartRZ1, kPartRR, kPartPQ, kPartBB, kPartR2, kPartF2, kPartDU2, kPartU2,
   kPartArrays
 };
+
+// workgroups of the fine-level products (one partial each): a slice, or four
+inline int64_t fine_groups(const Ctx* c) { return c->sell_split ? c->nslices : (c->nslices + 3) / 4; }
 
 inline double* part(Ctx* c, int a) { return c->d_part + (size_t)a * kMaxPartials; }
 

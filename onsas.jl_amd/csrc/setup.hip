@@ -90,6 +90,14 @@ int color_group(Ctx* c, ElemGroup& g) {
   return ONSAS_OK;
 }
 
+// Most slices whose products take four waves a slice: up to about a workgroup per
+// CU and its neighbours the extra waves hide the chain of rounds, past that they
+// only add LDS sums.  Multigrid Newton solves with one / four waves a slice:
+// 14.2 / 11.6 ms at 145 slices, 20.1 / 18.2 ms at 792, 28.2 / 27.3 ms at 1,424,
+// 34.3 / 36.7 ms at 2,327 in FP32; 26.5 / 23.1 ms at 466 and 57.6 / 59.1 ms at
+// 1,424 in FP64.
+constexpr int64_t kSplitMaxSlices = 1024;
+
 std::vector<int32_t> gather_order(const ElemGroup& g) {
   return host::gather_order({g.conn.data(), g.nnode, g.ne});
 }
@@ -442,7 +450,8 @@ int finalize_model(Ctx* c) {
   // sliced-ELL layout of the tangent (kSellRows block rows per slice, padded
   // with zero blocks whose column is the row itself)
   c->nslices = (nn + kSellRows - 1) / kSellRows;
-  ONSAS_TRY(dev_alloc(c, (void**)&c->d_ppq, sizeof(double) * (size_t)((c->nslices + 3) / 4)));
+  c->sell_split = kSellLanes == 1 && c->nslices <= kSplitMaxSlices;
+  ONSAS_TRY(dev_alloc(c, (void**)&c->d_ppq, sizeof(double) * (size_t)fine_groups(c)));
   c->sell_ptr.assign(c->nslices + 1, 0);
   c->slice_rounds.assign(c->nslices, 0);
   c->ell_width = 0;
