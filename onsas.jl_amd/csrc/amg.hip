@@ -59,7 +59,6 @@ constexpr int kPowerWarm = 3;        // ... re-estimates from the last iterate
 constexpr double kProlongWeight = 1.15;
 constexpr int64_t kSell6MinRows = 2048;  // smaller levels: one wave per block row
 constexpr int kSell6Window = 256;     // rows sorted by length within windows of this size
-constexpr int kRestrictWide = 96;     // P blocks per aggregate above which 2 waves restrict
 // LDS of a sliced-ELL coarse product's workgroup for the x values of its column
 // window (2,048 nodes in FP32, 1,024 in FP64)
 constexpr size_t kX6Lds = 48 * 1024;
@@ -73,7 +72,9 @@ inline unsigned nblocks8(int64_t n, int t) { return (nblocks(n, t) + 7u) / 8u * 
 // a contiguous run, so that neighbouring rows' vector gathers share one L2.
 __device__ inline int64_t xcd_block(int64_t b, int64_t nb) { return (b & 7) * (nb >> 3) + (b >> 3); }
 
-__device__ inline bool pcg_stopped(const PcgState* st) { return st && (st->done | st->breakdown); }
+// nonzero once the PCG has stopped (outside a PCG the launches pass Amg::d_idle,
+// so that no kernel waits on a test of the pointer before it reads the flag)
+__device__ inline int32_t pcg_stopped(const PcgState* st) { return st->done | st->breakdown; }
 
 // The PCG's stop check at the start of the cycle's first kernel (256 threads),
 // run by every workgroup alike: ||r||^2 from the update's np partials, summed in
@@ -111,15 +112,18 @@ __device__ inline bool pcg_stop_check(const double* __restrict__ prr, int np, Pc
   return stop;
 }
 
+// a[u] of six values in registers.  By value: a reference to the array lets the
+// compiler turn the selects into an indexed access, which puts the array into LDS
+// or scratch, and the LDS form reads the workgroup's size from the dispatch
+// packet in host memory (6 to 14 us a launch, growing with the waves).
 template <typename T>
-__device__ inline T pick6(const T (&a)[6], int u) {
-  T r = a[0];
-  r = u == 1 ? a[1] : r;
-  r = u == 2 ? a[2] : r;
-  r = u == 3 ? a[3] : r;
-  r = u == 4 ? a[4] : r;
-  r = u == 5 ? a[5] : r;
-  return r;
+__device__ inline T pick6(T a0, T a1, T a2, T a3, T a4, T a5, int u) {
+  T r = a0;
+  r = u == 1 ? a1 : r;
+  r = u == 2 ? a2 : r;
+  r = u == 3 ? a3 : r;
+  r = u == 4 ? a4 : r;
+  return u == 5 ? a5 : r;
 }
 
 template <typename KT, typename VT>
@@ -540,9 +544,10 @@ __global__ __launch_bounds__(256) void k_sell_cheb(
       for (int q = 0; q < 3; ++q) xb[q] = x_base[3 * ic + q];
   }
   const int32_t su = __builtin_amdgcn_readfirstlane((int32_t)s);  // wave-uniform: scalar loads
-  const int32_t b0 = sell_ptr[su];
-  const int32_t rounds = live ? slice_rounds[su] : 0;
-  if (pcg_stopped(st)) return;  // the same for every wave of the launch
+  int32_t off = pcg_stopped(st), b0 = sell_ptr[su], rounds = slice_rounds[su];
+  arrive_s(b0, rounds, off);
+  if (off) return;  // the same for every wave of the launch
+  if (!live) rounds = 0;
   const uint32_t rs = (uint32_t)rstride;
   const int32_t* cp = scol + b0 + lane;
   const VT* vp = sval + 9u * (uint32_t)b0 + lane;
@@ -617,9 +622,10 @@ __global__ __launch_bounds__(256) void k_sell_cheb_split(
   __shared__ KT sha[9 * 64];
   const int64_t s = blockIdx.x;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int32_t b0 = sell_ptr[s], rounds = slice_rounds[s];
+  int32_t off = pcg_stopped(st), b0 = sell_ptr[s], rounds = slice_rounds[s];
   PartSum trr;
   if (chk_rr) trr.load(chk_rr, chk_np);
+  arrive_s(b0, rounds, off);
   const int64_t i = kSellRows * s + lane;
   const int64_t ic = i < nn ? i : nn - 1;
   KT bv[3] = {0, 0, 0}, vv[3] = {0, 0, 0}, xb[3] = {0, 0, 0}, dm[9];
@@ -644,7 +650,6 @@ __global__ __launch_bounds__(256) void k_sell_cheb_split(
   if (rounds > 0) pass.load(cp, vp, rs, w, rounds);
   // no wave leaves before the barrier: the first workgroup may set the flag
   // while the others start, and then only some of a workgroup's waves see it
-  const bool off = pcg_stopped(st);
   KT a[3] = {0, 0, 0};
   if (!off && rounds > 0) {
     pass.add(v, w, rounds, a);
@@ -718,14 +723,15 @@ __global__ __launch_bounds__(256) void k_bsr6_cheb(
   const int32_t I = __builtin_amdgcn_readfirstlane((int32_t)Iw);
   const int l = threadIdx.x & 63;
   const int u = l & 7, uc = u < 6 ? u : 5, slot = l >> 3;
-  const int32_t k0 = row_ptr[I], k1 = row_ptr[I + 1];
+  int32_t off = pcg_stopped(st), k0 = row_ptr[I], k1 = row_ptr[I + 1];
+  arrive_s(k0, k1, off);
+  if (off) return;  // the same for every wave of the launch
   const KT* bp = b ? b : v;
   const KT* xbp = x_base ? x_base : v;
   const KT bv = bp[6 * (int64_t)I + uc], vu = v[6 * (int64_t)I + uc], xb = xbp[6 * (int64_t)I + uc];
   KT dm[6];
 #pragma unroll
   for (int m = 0; m < 6; ++m) dm[m] = Dinv[36 * (int64_t)I + 6 * uc + m];
-  if (pcg_stopped(st)) return;  // the same for every wave of the launch
   KT acc = 0;
   for (int32_t kb = k0; kb < k1; kb += 8 * kBsrRounds) {
     int32_t cj[kBsrRounds];
@@ -751,9 +757,7 @@ __global__ __launch_bounds__(256) void k_bsr6_cheb(
       for (int c = 0; c < 6; ++c) acc += av[q][c] * (ok ? xv[q][c] : KT(0));
     }
   }
-  acc += dpp_move<kDppRor8>(acc);  // slots s and s ^ 1
-  acc += __shfl_xor(acc, 16, 64);
-  acc += __shfl_xor(acc, 32, 64);
+  acc = stride_sum<8>(acc);
   const KT ru = (b ? bv : KT(0)) - acc;
   if (l >= 8) return;  // lanes 0 .. 7: one slot's components
   KT r[6];
@@ -867,9 +871,11 @@ __global__ __launch_bounds__(64 * WV) void k_sell6_cheb(
   const bool live = s0 < nslices;
   const int64_t s = live ? s0 : nslices - 1;
   const int32_t su = __builtin_amdgcn_readfirstlane((int32_t)s);  // wave-uniform: scalar loads
-  const int32_t q0 = s6_ptr[su], q1 = live ? s6_ptr[su + 1] : q0;
+  int32_t off = pcg_stopped(st), q0 = s6_ptr[su], q1 = s6_ptr[su + 1];
   const int32_t lo = kWin ? s6_win[2 * blockIdx.x] : 0, span = kWin ? s6_win[2 * blockIdx.x + 1] : 0;
-  if (pcg_stopped(st)) return;  // the same for every wave of the launch
+  arrive_s(q0, q1, off);
+  if (off) return;  // the same for every wave of the launch
+  if (!live) q1 = q0;
   // rounds are clamped to qlast (a slice has at least one round; an empty one
   // reads a neighbouring round and adds exact zeros)
   const int32_t qlast = max(max(q1, q0 + 1) - 1, 0);
@@ -942,14 +948,12 @@ __global__ __launch_bounds__(64 * WV) void k_sell6_cheb(
     for (int m = 0; m < 6; ++m) bv[m] = KT(0);
   const KT xb = x_base ? xb0 : KT(0);
 #pragma unroll
-  for (int o = RPW; o < 64; o <<= 1)
-#pragma unroll
-    for (int w = 0; w < 6; ++w) acc[w] += __shfl_xor(acc[w], o, 64);
+  for (int w = 0; w < 6; ++w) acc[w] = stride_sum<RPW>(acc[w]);
   if (!live || u >= 6 || I < 0) return;
   KT r[6];
 #pragma unroll
   for (int m = 0; m < 6; ++m) r[m] = bv[m] - acc[m];
-  const KT ru = pick6(r, u);
+  const KT ru = pick6(r[0], r[1], r[2], r[3], r[4], r[5], u);
   if (r_out) r_out[6 * I + u] = ru;
   if (!d_out && !x_out) return;
   KT dr = 0;
@@ -995,74 +999,43 @@ __global__ void k_jacobi(const KT* __restrict__ Dinv, const KT* __restrict__ v, 
 
 // b_c[I] = sum over the P blocks of column I (entries rt_ptr[I].., row order; PT
 // holds them contiguously) of P_e^T r_row(e), LPA lanes per aggregate over its
-// entries: 32 (two aggregates per wave, half the waves: the fine level, about
-// a hundred entries each), 64, 128 (two waves an aggregate, two aggregates a
-// workgroup: the levels with a few hundred entries an aggregate; on the 64^3
-// cube's level 1 14.3 us against 17.4 us with 256) or 256 (four waves); the
-// waves of an aggregate add their sums in wave order through LDS.  With d0
-// non-null also d0[I] = s D_c^-1
-// b_c[I] (the first Chebyshev step of the coarse level).  An FP32 lane takes
-// two of its entries per pass (LPA apart) with clamped, unconditional index
-// loads, so both row gathers are in flight together (FP64: one, for the
-// registers); a slot past the end adds an exact zero, so the lane's sum keeps
-// the order l, l + LPA, ... of a one-entry loop.
-template <typename KT, int BS, int LPA>
-__global__ __launch_bounds__(256) void k_sa_restrict(
-    const int32_t* __restrict__ rt_ptr, const int32_t* __restrict__ rt_row,
-    const PT_t<KT>* __restrict__ PT, const KT* __restrict__ rf, KT* __restrict__ bc,
-    const KT* __restrict__ Dinv_c, KT s, KT* __restrict__ d0, int64_t nc, const PcgState* st) {
-  static_assert(LPA == 32 || LPA == 64 || LPA == 128 || LPA == 256,
-                "32, 64, 128 or 256 lanes per aggregate");
+// entries (restrict_lanes: 32, two aggregates per wave, to 256, a workgroup an
+// aggregate); the waves of an aggregate add their sums in wave order through LDS.
+// With D0 also d0[I] = s D_c^-1 b_c[I] (the first Chebyshev step of the coarse
+// level).  An FP32 lane takes two of its entries per pass (LPA apart) with
+// clamped, unconditional index loads, so both row gathers are in flight together
+// (FP64: one, for the registers); a slot past the end adds an exact zero, so the
+// lane's sum keeps the order l, l + LPA, ... of a one-entry loop.  Bound by the
+// chain of three reads on small models, by the reads of P on large ones: 20.3 ->
+// 11.2 us at 64^3 (41 MB of P), 8.6 -> 2.7 us at 15,625 nodes once the six sums
+// stayed in registers (pick6).
+template <typename KT, int BS, int LPA, int U>
+struct RestrictPass {  // entries e, e + LPA, ... (clamped to the aggregate's last one)
   using PV = PT_t<KT>;
-  constexpr int kU = sizeof(KT) == 4 ? 2 : 1;
-  __shared__ KT sh[4][6];
-  // LPA < 256: an XCD-aware run of aggregates (the grid is a multiple of 8)
-  const int64_t bl = LPA < 256 ? xcd_block(blockIdx.x, gridDim.x) : (int64_t)blockIdx.x;
-  const int64_t Iw = (bl * 256 + threadIdx.x) / LPA;
-  const int l = threadIdx.x % LPA;
-  if (LPA < 128 && Iw >= nc) return;  // no barrier below for these
-  // LPA 128: both aggregates of the workgroup reach the barrier (one past the
-  // end reads the last aggregate and writes nothing); LPA 256: Iw < nc
-  const bool live = Iw < nc;
-  const int64_t I = live ? Iw : nc - 1;
-  // the coarse row's D^-1 first (its latency hides under the gathers); an
-  // aggregate index uniform over the wave makes its bounds scalar loads
-  KT dm[6];
-  if (d0)
+  int32_t row[U];
+  PV pv[U][BS * 6];
+  __device__ inline void load(const int32_t* __restrict__ rt_row, const PV* __restrict__ PT, int32_t e,
+                              int32_t last) {
 #pragma unroll
-    for (int m = 0; m < 6; ++m) dm[m] = Dinv_c[36 * I + 6 * (l < 6 ? l : 0) + m];
-  int32_t e0, e1;
-  if (LPA >= 64) {
-    const int32_t Iu = __builtin_amdgcn_readfirstlane((int32_t)I);
-    e0 = rt_ptr[Iu];
-    e1 = rt_ptr[Iu + 1];
-  } else {
-    e0 = rt_ptr[I];
-    e1 = rt_ptr[I + 1];
-  }
-  if (pcg_stopped(st)) return;
-  KT acc[6] = {0, 0, 0, 0, 0, 0};
-  for (int32_t e = e0 + l; e < e1; e += kU * LPA) {
-    int32_t ek[kU];
-    int64_t ik[kU];
+    for (int k = 0; k < U; ++k) row[k] = rt_row[min(e + k * LPA, last)];
 #pragma unroll
-    for (int k = 0; k < kU; ++k) {
-      ek[k] = min(e + k * LPA, e1 - 1);
-      ik[k] = rt_row[ek[k]];
-    }
-    PV pv[kU][BS * 6];
-    KT rv[kU][BS];
-#pragma unroll
-    for (int k = 0; k < kU; ++k) {  // unconditional loads (clamped addresses)
-      const PV* pp = (const PV*)__builtin_assume_aligned(PT + (int64_t)BS * 6 * ek[k], 2 * sizeof(PV));
+    for (int k = 0; k < U; ++k) {
+      const PV* pp = (const PV*)__builtin_assume_aligned(
+          PT + (int64_t)BS * 6 * min(e + k * LPA, last), 2 * sizeof(PV));
 #pragma unroll
       for (int q = 0; q < BS * 6; ++q) pv[k][q] = pp[q];
-#pragma unroll
-      for (int a = 0; a < BS; ++a) rv[k][a] = rf[BS * ik[k] + a];
     }
+    arrive_all(row);
+  }
+  __device__ inline void add(const KT* __restrict__ rf, int32_t e, int32_t last, KT (&acc)[6]) const {
+    KT rv[U][BS];
 #pragma unroll
-    for (int k = 0; k < kU; ++k) {
-      const bool ok = e + k * LPA < e1;
+    for (int k = 0; k < U; ++k)
+#pragma unroll
+      for (int a = 0; a < BS; ++a) rv[k][a] = rf[BS * (int64_t)row[k] + a];
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      const bool ok = e + k * LPA <= last;
 #pragma unroll
       for (int a = 0; a < BS; ++a) {
         const KT ra = ok ? rv[k][a] : KT(0);
@@ -1071,32 +1044,69 @@ __global__ __launch_bounds__(256) void k_sa_restrict(
       }
     }
   }
+};
+
+template <typename KT, int BS, int LPA, bool D0>
+__global__ __launch_bounds__(256) void k_sa_restrict(
+    const int32_t* __restrict__ rt_ptr, const int32_t* __restrict__ rt_row,
+    const PT_t<KT>* __restrict__ PT, const KT* __restrict__ rf, KT* __restrict__ bc,
+    const KT* __restrict__ Dinv_c, KT s, KT* __restrict__ d0, int64_t nc, const PcgState* st) {
+  static_assert(LPA == 32 || LPA == 64 || LPA == 128 || LPA == 256,
+                "32, 64, 128 or 256 lanes per aggregate");
+  constexpr int kU = sizeof(KT) == 4 ? 2 : 1;
+  // an XCD-aware run of aggregates (the grid is a multiple of 8)
+  const int64_t Iw = (xcd_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x) / LPA;
+  const int l = threadIdx.x % LPA;
+  if (LPA < 128 && Iw >= nc) return;  // no barrier below for these
+  // LPA >= 128: every aggregate of the workgroup reaches the barrier (one past
+  // the end reads the last aggregate and writes nothing)
+  const bool live = Iw < nc;
+  const int32_t I = (int32_t)(live ? Iw : nc - 1);
+  // three dependent reads: the entries' bounds (with the stop flag), their rows
+  // (with P and the coarse row's D^-1), the residual there
+  int32_t off = st->done | st->breakdown;
+  int32_t e0 = rt_ptr[I], e1 = rt_ptr[I + 1];  // an aggregate has entries
+  arrive_v(e0, e1, off);
+  if (off) return;  // the same for every wave of the launch
+  const int32_t last = e1 - 1;
+  KT dm[6];
+  if constexpr (D0) {
+#pragma unroll
+    for (int m = 0; m < 6; ++m) dm[m] = Dinv_c[36 * (int64_t)I + 6 * (l < 6 ? l : 0) + m];
+  }
+  RestrictPass<KT, BS, LPA, kU> pass;
+  pass.load(rt_row, PT, e0 + l, last);
+  KT acc[6] = {0, 0, 0, 0, 0, 0};
+  pass.add(rf, e0 + l, last, acc);
+  for (int32_t e = e0 + l + kU * LPA; e <= last; e += kU * LPA) {
+    pass.load(rt_row, PT, e, last);
+    pass.add(rf, e, last, acc);
+  }
   // fixed tree over the aggregate's lanes (within its half of the wave for 32)
 #pragma unroll
-  for (int o = (LPA < 64 ? LPA : 64) / 2; o > 0; o >>= 1)
+  for (int q = 0; q < 6; ++q) acc[q] = half_or_wave_sum<(LPA < 64 ? LPA : 64)>(acc[q]);
+  if constexpr (LPA >= 128) {  // the aggregate's waves add their sums in wave order
+    __shared__ KT sh[4][6];
+    const int w = threadIdx.x >> 6, w0 = w & ~(LPA / 64 - 1);  // the aggregate's first wave
+    if ((threadIdx.x & 63) == 0)
 #pragma unroll
-    for (int q = 0; q < 6; ++q) acc[q] += __shfl_xor(acc[q], o, 64);
-  if (LPA >= 128) {  // the aggregate's waves add their sums in wave order
-    if ((threadIdx.x & 63) < 6) sh[threadIdx.x >> 6][threadIdx.x & 63] = pick6(acc, threadIdx.x & 63);
+      for (int u = 0; u < 6; ++u) sh[w][u] = acc[u];
     __syncthreads();
-    if (l < 6) {
-      const int w0 = (int)(threadIdx.x >> 6) & ~(LPA / 64 - 1);  // the aggregate's first wave
 #pragma unroll
-      for (int u = 0; u < 6; ++u) {
-        KT a = sh[w0][u];
+    for (int u = 0; u < 6; ++u) {
+      KT a = sh[w0][u];
 #pragma unroll
-        for (int w = 1; w < LPA / 64; ++w) a += sh[w0 + w][u];
-        acc[u] = a;
-      }
+      for (int v = 1; v < LPA / 64; ++v) a += sh[w0 + v][u];
+      acc[u] = a;
     }
   }
   if (l >= 6 || !live) return;
-  bc[6 * I + l] = pick6(acc, l);
-  if (d0) {
+  bc[6 * (int64_t)I + l] = pick6(acc[0], acc[1], acc[2], acc[3], acc[4], acc[5], l);
+  if constexpr (D0) {
     KT dr = 0;
 #pragma unroll
     for (int m = 0; m < 6; ++m) dr += dm[m] * acc[m];
-    d0[6 * I + l] = s * dr;
+    d0[6 * (int64_t)I + l] = s * dr;
   }
 }
 
@@ -1116,9 +1126,10 @@ __global__ void k_sa_prolong(const int32_t* __restrict__ p_ptr, const int32_t* _
   if (t >= BS * nf) return;
   const int64_t i = t / BS;
   const int a = (int)(t % BS);
-  const KT x0 = xf[t];  // loaded with the row's bounds, ahead of the gathers
-  const int32_t p0 = p_ptr[i], p1 = p_ptr[i + 1];
-  if (pcg_stopped(st)) return;
+  int32_t off = pcg_stopped(st), p0 = p_ptr[i], p1 = p_ptr[i + 1];
+  arrive_v(p0, p1, off);
+  if (off) return;
+  const KT x0 = xf[t];
   KT acc = 0;
   for (int32_t p = p0; p < p1; p += kPass) {
     int32_t cj[kPass];
@@ -1168,11 +1179,12 @@ __global__ __launch_bounds__(256) void k_sa_prolong_pair(
   const int h = (int)(t & 1);
   // both threads of a pair are in one wave and take the same exits
   if (i >= nf) return;
+  int32_t off = pcg_stopped(st), p0 = p_ptr[i], p1 = p_ptr[i + 1];
+  arrive_v(p0, p1, off);
+  if (off) return;
   KT x0[BS];
 #pragma unroll
   for (int a = 0; a < BS; ++a) x0[a] = xf[BS * i + a];
-  const int32_t p0 = p_ptr[i], p1 = p_ptr[i + 1];
-  if (pcg_stopped(st)) return;
   KT acc[BS];
 #pragma unroll
   for (int a = 0; a < BS; ++a) acc[a] = KT(0);
@@ -1218,10 +1230,9 @@ template <typename KT>
 __global__ __launch_bounds__(256) void k_dense_apply(const KT* __restrict__ Ainv,
                                                      const KT* __restrict__ b, KT* __restrict__ x,
                                                      int64_t nc, int64_t ldc, const PcgState* st) {
-  if (pcg_stopped(st)) return;
   const int64_t r = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 6;
   const int l = threadIdx.x & 63;
-  if (r >= nc) return;
+  if (r >= nc || pcg_stopped(st)) return;
   // rows padded to ldc (a multiple of 4): 4 consecutive values per lane and load
   const KT* a = Ainv + r * ldc;
   KT s = 0;
@@ -1230,8 +1241,7 @@ __global__ __launch_bounds__(256) void k_dense_apply(const KT* __restrict__ Ainv
 #pragma unroll
     for (int j = 0; j < 4; ++j) s += ap[j] * b[c + j < nc ? c + j : nc - 1];  // padding: ap[j] = 0
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  s = half_or_wave_sum<64>(s);
   if (l == 0) x[r] = s;
 }
 
@@ -1337,6 +1347,18 @@ int sell6_waves_per_group(bool f64) {
 }  // namespace
 
 // Build the hierarchy's symbolic part (host) and allocate its device arrays.
+// Lanes per aggregate of the restriction: enough that 1.5 times the mean number
+// of entries is one pass (two entries a lane in FP32, one in FP64), so that few
+// aggregates need a second chain of reads.  Measured with 32 / 64 / 128 / 256
+// lanes: fine level of 64^3 (80 entries, 14,182 aggregates) 11.3 / 11.2 / 13.5 /
+// 19.9 us, its level 1 (300 entries, 262 aggregates) 15.7 / 9.6 / 6.4 / 6.0 us;
+// 61,152 nodes (84 entries) 4.7 / 4.3 / 4.7 / 6.3 us; FP64, 8,640 nodes (69
+// entries) 5.6 / 4.2 / 3.4 / 3.7 us.
+int restrict_lanes(int64_t nnz_p, int64_t na, bool f64) {
+  const double want = 1.5 * (double)nnz_p / (double)std::max<int64_t>(na, 1) / (f64 ? 1 : 2);
+  return want <= 32 ? 32 : want <= 64 ? 64 : want <= 128 ? 128 : 256;
+}
+
 int amg_build(Ctx* c) {
   Amg& A = c->amg;
   const int64_t gen = A.gen;  // monotonic across rebuilds (graph cache key)
@@ -1424,7 +1446,7 @@ int amg_build(Ctx* c) {
     AmgLevel& F = A.lev.back();
     F.nnz_p = S.nnz_p;
     F.nnz_w = S.nnz_w;
-    F.restrict_wide = S.nnz_p > (int64_t)kRestrictWide * na;
+    F.restrict_lanes = restrict_lanes(S.nnz_p, na, f64);
     ONSAS_TRY(upload(c, &F.d_agg, S.agg));
     ONSAS_TRY(f64 ? upload_kt<double>(c, &F.d_T, S.T) : upload_kt<float>(c, &F.d_T, S.T));
     ONSAS_TRY(upload(c, &F.d_p_ptr, S.p_ptr));
@@ -1484,7 +1506,8 @@ int amg_build(Ctx* c) {
   A.ldc = (A.nc + 3) & ~3;
   ONSAS_TRY(alloc(c, &A.d_Ainv, c->kt * (size_t)A.nc * A.ldc));
   ONSAS_TRY(alloc(c, (void**)&A.d_part, sizeof(double) * 1024));
-  ONSAS_TRY(alloc(c, (void**)&A.d_rzs, sizeof(double) * 2 * (size_t)c->nslices));
+  ONSAS_TRY(alloc(c, (void**)&A.d_rzs, sizeof(double) * 2 * (size_t)c->nslices + sizeof(PcgState)));
+  A.d_idle = (const PcgState*)(A.d_rzs + 2 * c->nslices);  // zero
   A.built = true;
   A.stale = true;
   return ONSAS_OK;
@@ -1550,6 +1573,7 @@ void op_cheb(Ctx* c, int l, const KT* v, const KT* b, KT* r_out, double c1, doub
              const KT* x_base, KT* x_out, const PcgState* st, hipEvent_t ea = nullptr,
              hipEvent_t eb = nullptr, double* prz = nullptr, const double* chk_rr = nullptr) {
   hipStream_t s = c->stream;
+  if (!st) st = c->amg.d_idle;
   if (l == 0) {
     // chk_rr: the PCG's stop check runs in this kernel's prologue
     PcgState* wst = chk_rr ? const_cast<PcgState*>(st) : nullptr;
@@ -1690,23 +1714,37 @@ int amg_numeric_t(Ctx* c) {
   return ONSAS_OK;
 }
 
+template <typename KT, int BS, int LPA>
+void launch_restrict_lanes(Ctx* c, const AmgLevel& L, const AmgLevel& C, const KT* r, KT sc,
+                           KT* d0c, const PcgState* st) {
+  if (d0c)
+    hipLaunchKernelGGL((k_sa_restrict<KT, BS, LPA, true>), dim3(nblocks8(C.n, 256 / LPA)), dim3(256),
+                       0, c->stream, L.d_rt_ptr, L.d_rt_row, (const PT_t<KT>*)L.d_PT, r, (KT*)C.d_b,
+                       (const KT*)C.d_Dinv, sc, d0c, C.n, st);
+  else
+    hipLaunchKernelGGL((k_sa_restrict<KT, BS, LPA, false>), dim3(nblocks8(C.n, 256 / LPA)), dim3(256),
+                       0, c->stream, L.d_rt_ptr, L.d_rt_row, (const PT_t<KT>*)L.d_PT, r, (KT*)C.d_b,
+                       (const KT*)nullptr, sc, d0c, C.n, st);
+}
+
 template <typename KT, int BS>
 void launch_restrict(Ctx* c, const AmgLevel& L, const AmgLevel& C, const KT* r, KT sc, KT* d0c,
                      const PcgState* st) {
-  if (L.restrict_wide)
-    hipLaunchKernelGGL((k_sa_restrict<KT, BS, 128>), dim3(nblocks8(C.n, 2)), dim3(256), 0, c->stream,
-                       L.d_rt_ptr, L.d_rt_row, (const PT_t<KT>*)L.d_PT, r, (KT*)C.d_b,
-                       (const KT*)C.d_Dinv, sc, d0c, C.n, st);
+  if (L.restrict_lanes == 256)
+    launch_restrict_lanes<KT, BS, 256>(c, L, C, r, sc, d0c, st);
+  else if (L.restrict_lanes == 128)
+    launch_restrict_lanes<KT, BS, 128>(c, L, C, r, sc, d0c, st);
+  else if (L.restrict_lanes == 64)
+    launch_restrict_lanes<KT, BS, 64>(c, L, C, r, sc, d0c, st);
   else
-    hipLaunchKernelGGL((k_sa_restrict<KT, BS, 32>), dim3(nblocks8(C.n, 8)), dim3(256), 0, c->stream,
-                       L.d_rt_ptr, L.d_rt_row, (const PT_t<KT>*)L.d_PT, r, (KT*)C.d_b,
-                       (const KT*)C.d_Dinv, sc, d0c, C.n, st);
+    launch_restrict_lanes<KT, BS, 32>(c, L, C, r, sc, d0c, st);
 }
 
 template <typename KT>
 int vcycle_t(Ctx* c, const KT* b0, KT* z0, const PcgState* st, bool d0_ready, hipEvent_t* ev,
              double* prz, const double* chk_rr) {
   auto evs = [&](int l, int j) { return l == 0 && ev ? ev[j] : nullptr; };
+  if (!st) st = c->amg.d_idle;
   Amg& A = c->amg;
   hipStream_t s = c->stream;
   const int nl = (int)A.lev.size();

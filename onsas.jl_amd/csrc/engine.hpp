@@ -149,7 +149,7 @@ struct AmgLevel {
   int32_t* d_agg = nullptr;           // node -> aggregate
   void* d_T = nullptr;                // tentative prolongator, bs x 6 per node (KT)
   int64_t nnz_p = 0;                  // blocks of P
-  bool restrict_wide = false;         // restriction with 2 waves per aggregate
+  int restrict_lanes = 32;            // lanes per aggregate of the restriction
   int32_t *d_p_ptr = nullptr, *d_p_col = nullptr, *d_p_row = nullptr;
   void* d_P = nullptr;                // nnz_p x bs x 6 (KT), row-major blocks
   int64_t* d_pk_ptr = nullptr;        // per P block: the operator blocks of its row
@@ -181,6 +181,7 @@ struct Amg {
   int ldc = 0;                        // row length of d_Ainv (nc rounded up to 4)
   void* d_Ainv = nullptr;             // nc x ldc KT, zero padded
   double* d_part = nullptr;           // power-iteration partial sums
+  const struct PcgState* d_idle = nullptr;  // a state that never stops (the tail of d_rzs)
   double* d_rzs = nullptr;            // 2 x nslices r.z partials of the PCG (degree-1 fine level)
 };
 

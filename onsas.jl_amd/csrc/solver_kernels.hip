@@ -504,10 +504,11 @@ __global__ __launch_bounds__(256) void k_pcg_A_split(
   __shared__ KT sha[9 * 64];
   const int64_t s = blockIdx.x;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int32_t b0 = sell_ptr[s], rounds = slice_rounds[s];
+  int32_t off = st->done | st->breakdown, b0 = sell_ptr[s], rounds = slice_rounds[s];
   PartSum trz, trr;
   trz.load(prz, nrz);
   trr.load(prr, np);
+  arrive_s(b0, rounds, off);
   const int64_t i = kSellRows * s + lane;
   const int64_t ic = i < nn ? i : nn - 1;
   KT zi[3], pi[3], qi[3];
@@ -525,7 +526,6 @@ __global__ __launch_bounds__(256) void k_pcg_A_split(
   if (rounds > 0) pass.load(cp, vp, rs, w, rounds);
   // no wave leaves before the barrier: the first workgroup may set the flag
   // while the others start, and then only some of a workgroup's waves see it
-  const bool off = st->done | st->breakdown;
   const int k = st->k;
   const double rzp = k > 0 ? st->rzs[par ^ 1] : 0.0;
   KT a[3] = {0, 0, 0};
