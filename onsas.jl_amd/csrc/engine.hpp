@@ -301,6 +301,10 @@ struct Ctx {
   Scalars* d_sc = nullptr;
   Scalars* h_sc = nullptr;   // pinned
   double* h_stage = nullptr;  // pinned, 3 nn values: staging of state vector copies
+  // pinned ring of the large downloads (made by the first one), an event per slot
+  static constexpr int kCopySlots = 8;
+  char* h_ring = nullptr;
+  hipEvent_t ev_ring[kCopySlots] = {};
   double* h_snap[2] = {};     // pinned, 3 nn values each: U snapshots (onsas_snapshot_U)
   hipEvent_t ev_snap[2] = {};  // ... their copies' completion
   // A snapshot copies U on the stream into d_snap (device to device, a few
