@@ -8,13 +8,13 @@
 // half of the double, so a word carries its own "ready" mark and the sum is
 // exact; the partials are added by a fixed tree, the same in every workgroup,
 // so all of them take the same branches and a solve is bit-identical from run
-// to run.  Measured on one MI355X: 1.2 us for 1 to 8 workgroups, 2.0 us for 32,
+// to run.  A sum alone, measured on one MI355X: 1.2 us for 1 to 8 workgroups, 2.0 us for 32,
 // 3.3 us for 128, against 4 to 8 us for a kernel boundary with its drain,
 // launch and first loads.
 //
-// Everything shared goes through relaxed device-scope atomics (they bypass the
+// Everything shared goes through device-scope loads and stores (they bypass the
 // per-XCD L2s), and a workgroup's vector stores are complete (vmcnt 0, then the
-// barrier, DRAIN below) before its partial is published, so no L2
+// barrier, in grid_sum4) before its partial is published, so no L2
 // write-back or invalidation is needed and the read-only data stays cached.
 // Waits are bounded: a workgroup that polls past `limit` clock ticks (or sees
 // another's abort) raises the abort word and the launch drains; the host then
@@ -29,8 +29,9 @@
 
 namespace onsas {
 
-constexpr int kMaxGridWg = 128;  // workgroups of a resident launch (two polled slots per lane)
-constexpr size_t kGridSlotWords = 6 * kMaxGridWg;  // the PCG's slots: a one- and a two-value sum
+constexpr int kMaxGridWg = 128;  // workgroups of a resident launch
+constexpr int kPollSlots = 64;   // slots that grid_sum4 polls at a time
+constexpr size_t kGridSlotWords = 16 * kMaxGridWg;  // the PCG's slots: sums of four values, twice
 
 template <typename T>
 __device__ inline T agent_load(const T* p) {
@@ -39,6 +40,35 @@ __device__ inline T agent_load(const T* p) {
 template <typename T>
 __device__ inline void agent_store(T* p, T v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// The loads of values that other workgroups write: past the caches like
+// agent_load, and 12 or 16 bytes an instruction.  Every value among them is at
+// most 8 bytes and aligned, and carries its own mark.
+using SharedBuf = __amdgpu_buffer_rsrc_t;
+__device__ inline SharedBuf shared_buf(const void* p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
+}
+constexpr int kSharedLoad = (int)(0x80000000u | 16u);  // volatile (each poll loads anew), sc1
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+__device__ inline void shared_load3(SharedBuf b, uint32_t off, uint32_t (&w)[3]) {
+  const u32x3 v = __builtin_amdgcn_raw_buffer_load_b96(b, off, 0, kSharedLoad);
+  w[0] = v[0];
+  w[1] = v[1];
+  w[2] = v[2];
+}
+__device__ inline void shared_load2(SharedBuf b, uint32_t off, unsigned long long (&w)[2]) {
+  const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(b, off, 0, kSharedLoad);
+  w[0] = ((unsigned long long)v[1] << 32) | v[0];
+  w[1] = ((unsigned long long)v[3] << 32) | v[2];
+}
+__device__ inline void shared_load3(SharedBuf b, uint32_t off, unsigned long long (&w)[3]) {
+  const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(b, off, 0, kSharedLoad);
+  const u32x2 u = __builtin_amdgcn_raw_buffer_load_b64(b, off + 16, 0, kSharedLoad);
+  w[0] = ((unsigned long long)v[1] << 32) | v[0];
+  w[1] = ((unsigned long long)v[3] << 32) | v[2];
+  w[2] = ((unsigned long long)u[1] << 32) | u[0];
 }
 // this wave's stores have reached the device-coherent level
 __device__ inline void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
@@ -50,48 +80,37 @@ struct GridSlots {
   long long limit;            // ticks of the 100 MHz clock a wait may take
 };
 
-// Sum over the workgroup: over each wave, then over the wave partials in index
-// order (T threads; sh: NV * T / 64 doubles).  With DRAIN the workgroup's
-// earlier stores are complete when the barrier inside opens.  A caller that
-// reuses sh has a barrier between two uses.
-template <int NV, int T, bool DRAIN>
-__device__ inline void wg_partials(double (&v)[NV], double* sh) {
-#pragma unroll
-  for (int q = 0; q < NV; ++q) v[q] = wave_sum(v[q]);
-  if ((threadIdx.x & 63) == 0)
-#pragma unroll
-    for (int q = 0; q < NV; ++q) sh[q * (T / 64) + (threadIdx.x >> 6)] = v[q];
-  if (DRAIN) stores_done();
-  __syncthreads();
+// Four sums over the workgroup at once, lane l of a wave holding a part of sum
+// l & 3 from the first step on, so that a tree step is one addition and not four.
+// First: the wave's part of sum l & 3, in every lane (v: the thread's parts, all
+// 64 lanes active).
+__device__ inline double wave_sum4(const double (&v)[4]) {
+  const int q = threadIdx.x & 3;
+  const double a = group_sum<4>(v[0]), b = group_sum<4>(v[1]), c = group_sum<4>(v[2]),
+               d = group_sum<4>(v[3]);
+  return stride_sum<4>((q & 2) ? ((q & 1) ? d : c) : ((q & 1) ? b : a));
 }
-template <int NV, int T>
-__device__ inline void wg_total(double (&v)[NV], const double* sh) {
-#pragma unroll
-  for (int q = 0; q < NV; ++q) {
-    double s = sh[q * (T / 64)];
-#pragma unroll
-    for (int w = 1; w < T / 64; ++w) s += sh[q * (T / 64) + w];
-    v[q] = s;
-  }
-}
-template <int NV, int T>
-__device__ inline void wg_sum(double (&v)[NV], double* sh) {
-  wg_partials<NV, T, false>(v, sh);
-  wg_total<NV, T>(v, sh);
+// Then, past a barrier, the workgroup's sum l & 3 from the waves' parts in sh (T threads).
+template <int T>
+__device__ inline double wg_sum4(const double* sh) {
+  static_assert(4 * (T / 64) <= 64, "a part per lane");
+  const int lane = threadIdx.x & 63;
+  return stride_sum<4>(lane < 4 * (T / 64) ? sh[lane] : 0.0);
 }
 
-// One value of a slot: its two words once both carry the epoch; false once the
-// launch is aborted.
-template <int NW>
-__device__ inline bool poll_words(const unsigned long long* s, uint32_t epoch, const GridSlots& gs,
-                                  unsigned long long (&w)[NW]) {
+// N values at the byte offsets off, two words each, once all of them carry the
+// epoch; false once the launch is aborted.
+template <int N>
+__device__ inline bool poll_values(SharedBuf buf, const uint32_t (&off)[N], uint32_t epoch,
+                                   const GridSlots& gs, unsigned long long (&w)[N][2]) {
   long long t0 = 0;
   for (uint32_t spin = 0;; ++spin) {
     bool ready = true;
 #pragma unroll
-    for (int q = 0; q < NW; ++q) w[q] = agent_load(s + q);
+    for (int q = 0; q < N; ++q) shared_load2(buf, off[q], w[q]);
 #pragma unroll
-    for (int q = 0; q < NW; ++q) ready = ready && (uint32_t)(w[q] >> 32) == epoch;
+    for (int q = 0; q < N; ++q)
+      ready = ready && (uint32_t)(w[q][0] >> 32) == epoch && (uint32_t)(w[q][1] >> 32) == epoch;
     if (ready) return true;
     if ((spin & 63u) == 0) {
       const long long now = wall_clock64();
@@ -111,47 +130,57 @@ __device__ inline unsigned long long value_word(double p, uint32_t epoch, bool l
   return ((unsigned long long)epoch << 32) | (low ? (b & 0xffffffffull) : (b >> 32));
 }
 
-// Sum over all workgroups of the launch; false once the launch is aborted (the
-// same answer for every thread of the workgroup).  sh: NV * (T / 64 + 1) + 1
-// doubles.  With DRAIN the caller's stores are visible to every workgroup that
-// returns; the barriers inside order the workgroup's LDS.
-template <int NV, int T, bool DRAIN>
-__device__ inline bool grid_sum(double (&v)[NV], const GridSlots& gs, uint32_t epoch, double* sh) {
-  wg_partials<NV, T, DRAIN>(v, sh);
-  double* res = sh + NV * (T / 64);
+// The four sums over all workgroups of the launch; false once the launch is
+// aborted (the same answer for every thread of the workgroup).  sh: 4 T / 64 + 5
+// doubles, free again at the caller's next barrier.  The stores that the caller
+// made before it are complete at the device-coherent level before its part is
+// published.  late: an LDS word that a thread has set whose own wait expired
+// before the sum; nothing is published then.  A load takes 16 slots (a lane its
+// sum's 16 bytes of one).
+template <int T>
+__device__ inline bool grid_sum4(double (&v)[4], const GridSlots& gs, uint32_t epoch, double* sh,
+                                 const int* late) {
+  double* res = sh + 4 * (T / 64);
+  const int lane = threadIdx.x & 63;
+  {
+    const double p = wave_sum4(v);
+    if (lane < 4) sh[4 * (threadIdx.x >> 6) + lane] = p;
+  }
+  stores_done();
+  __syncthreads();
   if (threadIdx.x < 64) {
-    wg_total<NV, T>(v, sh);
-    const int lane = threadIdx.x;
-    unsigned long long* mine = gs.words + (size_t)(2 * NV) * blockIdx.x;
-    if (lane < 2 * NV) {
-      double p = v[0];
-#pragma unroll
-      for (int q = 1; q < NV; ++q) p = (lane >> 1) == q ? v[q] : p;
-      agent_store(mine + lane, value_word(p, epoch, lane & 1));
+    const double p = wg_sum4<T>(sh);
+    bool ok = *late == 0;
+    if (ok && lane < 4) {
+      unsigned long long* mine = gs.words + 8 * (size_t)blockIdx.x + 2 * lane;
+      agent_store(mine, value_word(p, epoch, false));
+      agent_store(mine + 1, value_word(p, epoch, true));
     }
-    bool ok = true;
-    double acc[NV];
+    const SharedBuf buf = shared_buf(gs.words, 64u * kMaxGridWg);
+    double acc = 0;
+    for (int g0 = 0; ok && g0 < gs.nwg; g0 += kPollSlots) {
+      unsigned long long w[4][2];
+      uint32_t off[4];
+      bool has[4];
 #pragma unroll
-    for (int q = 0; q < NV; ++q) acc[q] = 0;
-    for (int g = lane; ok && g < gs.nwg; g += 64) {
-      unsigned long long w[2 * NV];
-      ok = poll_words<2 * NV>(gs.words + (size_t)(2 * NV) * g, epoch, gs, w);
+      for (int j = 0; j < 4; ++j) {
+        const int g = g0 + 16 * j + (lane >> 2);
+        has[j] = g < gs.nwg;
+        off[j] = 64u * (has[j] ? g : blockIdx.x) + 16u * (lane & 3);
+      }
+      ok = poll_values<4>(buf, off, epoch, gs, w);
 #pragma unroll
-      for (int q = 0; q < NV; ++q) acc[q] += words_value(w[2 * q], w[2 * q + 1]);
+      for (int j = 0; j < 4; ++j) acc += has[j] ? words_value(w[j][0], w[j][1]) : 0.0;
     }
     ok = __all(ok);
-#pragma unroll
-    for (int q = 0; q < NV; ++q) acc[q] = wave_sum(acc[q]);
-    if (lane == 0) {
-#pragma unroll
-      for (int q = 0; q < NV; ++q) res[q] = acc[q];
-      res[NV] = ok ? 1.0 : 0.0;
-    }
+    acc = stride_sum<4>(acc);
+    if (lane < 4) res[lane] = acc;
+    if (lane == 0) res[4] = ok ? 1.0 : 0.0;
   }
   __syncthreads();
 #pragma unroll
-  for (int q = 0; q < NV; ++q) v[q] = res[q];
-  return res[NV] != 0.0;
+  for (int q = 0; q < 4; ++q) v[q] = res[q];
+  return res[4] != 0.0;
 }
 
 }  // namespace onsas

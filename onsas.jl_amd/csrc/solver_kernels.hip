@@ -1226,6 +1226,9 @@ int pcg_solve_t(Ctx* c, const double* b_dev, bool forcing, const void* x0, int e
     ps.k = ps.done = ps.iters = ps.breakdown = ps.converged = ps.aborted = 0;
     ps.breakdown_k = -1;
     ps.rr_last = ps.bb;
+    for (void* v : {c->d_pp0, c->d_pp1})  // the launch may have left its marks there
+      hipLaunchKernelGGL(k_fill_kt<KT>, dim3(grid_for(3 * c->nn, 256)), dim3(256), 0, s, (KT*)v,
+                         3 * c->nn, KT(0));
     ONSAS_HIP_TRY(c, hipMemcpyAsync(&c->d_sc->pcg, &ps, sizeof(PcgState), hipMemcpyHostToDevice, s));
     init_vectors();
   }

@@ -35,11 +35,13 @@ def _clique(prec, n):
 
 
 MODELS = {  # nodes: 8, 60, 128 / 140 (FP64 single workgroup ends at 128), 252 / 264 (FP32 at 256),
-    # 1331 (several workgroups, the last one partial), 9240 (workgroups of twice the threads)
+    # 1331 (several workgroups, the last one partial), 4352 (workgroups of twice the threads),
+    # 9240 (more workgroups than one poll covers)
     "1x1x1": lambda p: _box(p, 1, 1, 1), "4x3x2": lambda p: _box(p, 4, 3, 2),
     "7x3x3": lambda p: _box(p, 7, 3, 3), "6x4x3": lambda p: _box(p, 6, 4, 3),
     "8x6x3": lambda p: _box(p, 8, 6, 3), "10x5x3": lambda p: _box(p, 10, 5, 3),
     "10x10x10": lambda p: _box(p, 10, 10, 10),
+    "16x15x15": lambda p: _box(p, 16, 15, 15),
     "21x20x19": lambda p: _box(p, 21, 20, 19),
     "clique 17": lambda p: _clique(p, 17), "clique 32": lambda p: _clique(p, 32),
     "clique 33": lambda p: _clique(p, 33),  # rows too long: the general path
