@@ -254,14 +254,17 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs<KT> a) {
 // Restarted GMRES(m) with right block-Jacobi preconditioning (K D^-1 y = b,
 // x = D^-1 y), classical Gram-Schmidt twice, as gmres_solve_t in
 // solver_kernels.hip, whose iteration is some ten launches and three host round
-// trips: 157 us at 720 nodes in FP64, and 14.5 us here (289 -> 27 ms for the two
+// trips: 157 us at 720 nodes in FP64, and 8.6 us here (289 -> 16.9 ms for the two
 // load steps of a 9 x 8 x 7 box).  A workgroup holds R = T / L rows: the
 // tangent in registers, the basis V of its 3 R dofs and the working vector w in
-// LDS, the Hessenberg column and its rotations in LDS (every workgroup computes
-// the same ones).  An iteration is three grid exchanges: the dot products of
-// each Gram-Schmidt pass (a value per basis vector, four threads a value), and
-// |w| together with t = D^-1 w of the next product, which is published before w
-// is scaled: K D^-1 v = K t / |w|.
+// LDS, the Hessenberg column in LDS and its rotations in the lanes of every wave.
+// An iteration waits for the other workgroups three times: for the neighbours'
+// t = D^-1 w (handed over as z of the PCG) and for the dot products of the two
+// Gram-Schmidt passes (a value per basis vector, four threads a value).  |w| after
+// the second pass comes with it: |w|^2 before it less the squares of its
+// coefficients, all summed in FP64; where these take most of |w|^2 away it is
+// summed again.  The rotations run while t is under way.  With |w| as an exchange
+// of its own and slots polled one after the other an iteration was 14.5 us.
 constexpr int kGmresThreads = 256;
 constexpr int kGmresMax = 60;    // most basis vectors of the resident kernel (four threads each)
 constexpr int kGmresSlot = 128;  // words of a workgroup's slot: 64 values
@@ -277,7 +280,7 @@ struct GmresArgs {
   const double* b;
   const uint8_t* mask;
   KT* x;
-  KT* t;  // D^-1 w, read by the neighbouring workgroups
+  KT* tb[2];  // D^-1 w of the even and odd columns, read by the neighbouring workgroups
   PcgState* st;
   unsigned long long* slots;  // two regions of kMaxGridWg slots, used in turn
   uint32_t base;
@@ -287,23 +290,27 @@ struct GmresArgs {
   double rtol;
 };
 
-// LDS of one workgroup: packed triangle of R, two coefficient columns, rotations,
-// right-hand side, solution, four scalars; then w and the m + 1 basis vectors,
-// each padded by 4 values so that four threads of 16 vectors hit distinct banks
+// LDS of one workgroup: packed triangle of R, two coefficient columns (the second
+// with |w|^2), right-hand side, solution, two scalars; then w and the m + 1 basis
+// vectors, each padded by 4 values so that four threads of 16 vectors hit distinct
+// banks
 inline size_t gmres_lds(int m, int rows, size_t kt) {
-  return sizeof(double) * ((size_t)m * (m + 1) / 2 + 6 * 64 + 4) +
+  return sizeof(double) * ((size_t)m * (m + 1) / 2 + 4 * 64 + 2) +
          kt * (size_t)(m + 2) * (3 * rows + 4);
 }
 
 template <typename KT, int L, int NB>
 __global__ __launch_bounds__(kGmresThreads) void k_gmres_resident(GmresArgs<KT> a) {
   constexpr int T = kGmresThreads, R = T / L, DN = 3 * R, S = DN + 4;
+  using W = Unwritten<KT>;
+  using Bits = typename W::Bits;
   extern __shared__ double lds[];
+  __shared__ int late;  // a wait for t or x has expired
   const int m = a.m;
   double* Rm = lds;  // column j at j (j + 1) / 2
   double* h1 = Rm + m * (m + 1) / 2;
-  double *h2 = h1 + 64, *cs = h2 + 64, *sn = cs + 64, *gv = sn + 64, *yv = gv + 64, *sc = yv + 64;
-  KT* w = (KT*)(sc + 4);
+  double *h2 = h1 + 64, *gv = h2 + 64, *yv = gv + 64, *sc = yv + 64;
+  KT* w = (KT*)(sc + 2);
   KT* V = w + S;
   const int t = threadIdx.x;
   const int lane = t & 63;
@@ -340,17 +347,17 @@ __global__ __launch_bounds__(kGmresThreads) void k_gmres_resident(GmresArgs<KT> 
       for (int e = 0; e < 9; ++e) v[q][e] = has ? a.sval[9 * b + 64 * e + l] : KT(0);
     }
   }
+  if (t == 0) late = 0;
+  __syncthreads();
   GridSlots gs{a.slots, (int)gridDim.x, &a.st->aborted, a.limit};
+  const uint32_t bytes = 3u * (uint32_t)sizeof(KT) * (uint32_t)a.nn;
   uint32_t ep = a.base;
   auto region = [&](uint32_t e) { return a.slots + (size_t)(e & 1u) * kMaxGridWg * kGmresSlot; };
 
   // w = scale K y, y shared through device memory
   auto product = [&](const KT* y, double scale) {
     KT yj[NB][3];
-#pragma unroll
-    for (int q = 0; q < NB; ++q)
-#pragma unroll
-      for (int c = 0; c < 3; ++c) yj[q][c] = agent_load((const KT*)((const char*)y + cj[q]) + c);
+    if (!gather_published<KT, NB>(shared_buf(y, bytes), cj, gs, yj)) late = 1;
     KT a0 = 0, a1 = 0, a2 = 0;
 #pragma unroll
     for (int q = 0; q < NB; ++q) {
@@ -368,153 +375,138 @@ __global__ __launch_bounds__(kGmresThreads) void k_gmres_resident(GmresArgs<KT> 
     }
     __syncthreads();
   };
-  // |w|^2 over the launch, with t = D^-1 w published before it; `between` runs on
-  // the last wave while the first one waits for the other workgroups
-  auto norm_publish = [&](double& n2, auto between) -> bool {
-    ++ep;
-    if (live) agent_store(a.t + dof, d0 * w[n0] + d1 * w[n0 + 1] + d2 * w[n0 + 2]);
-    double p = 0;
-    if (t < 64) {
-      for (int d = lane; d < DN; d += 64) p += (double)w[d] * (double)w[d];
-      p = wave_sum(p);
-    }
-    stores_done();
-    __syncthreads();
-    if (t < 64) {
-      unsigned long long* reg = region(ep);
-      if (lane < 2) agent_store(reg + (size_t)kGmresSlot * blockIdx.x + lane, value_word(p, ep, lane & 1));
-      const SharedBuf rb = shared_buf(reg, 8u * kGmresSlot * kMaxGridWg);
-      bool ok = true;
-      double acc = 0;
-      for (int g = lane; ok && g < gs.nwg; g += 64) {
-        unsigned long long wd[1][2];
-        const uint32_t off[1] = {8u * kGmresSlot * g};
-        ok = poll_values<1>(rb, off, ep, gs, wd);
-        acc += words_value(wd[0][0], wd[0][1]);
-      }
-      ok = __all(ok);
-      acc = wave_sum(acc);
-      if (lane == 0) {
-        sc[0] = acc;
-        sc[1] = ok ? 1.0 : 0.0;
-      }
-    } else if (t >= T - 64) {
-      between();
-    }
-    __syncthreads();
-    n2 = sc[0];
-    return sc[1] != 0.0;
-  };
-  // h[0 .. nv) = V' w over the launch
-  auto dots = [&](int nv, double* h) -> bool {
+  // sum over the launch of `nval` values, four threads a value (acc: the thread's
+  // part), to h; the workgroup's earlier stores are complete when a later sum ends
+  auto share = [&](int nval, double acc, double* h) -> bool {
     ++ep;
     const int q = t >> 2, seg = t & 3;
-    double acc = 0;
-    if (q < nv) {
-      const KT* vq = V + q * S;
-      for (int d = seg; d < DN; d += 4) acc += (double)vq[d] * (double)w[d];
-    }
     acc = group_sum<4>(acc);
     unsigned long long* reg = region(ep);
-    const SharedBuf rb = shared_buf(reg, 8u * kGmresSlot * kMaxGridWg);
-    bool ok = true;
+    bool ok = late == 0;
     double sum = 0;
-    if (q < nv) {
+    if (ok && q < nval) {
       if (seg < 2)
         agent_store(reg + (size_t)kGmresSlot * blockIdx.x + 2 * q + seg, value_word(acc, ep, seg));
-      for (int g = seg; ok && g < gs.nwg; g += 4) {
-        unsigned long long wd[1][2];
-        const uint32_t off[1] = {8u * (kGmresSlot * g + 2 * q)};
-        ok = poll_values<1>(rb, off, ep, gs, wd);
-        sum += words_value(wd[0][0], wd[0][1]);
+      const SharedBuf rb = shared_buf(reg, 8u * kGmresSlot * kMaxGridWg);
+      for (int g0 = seg; ok && g0 < gs.nwg; g0 += 16) {
+        unsigned long long wd[4][2];
+        uint32_t off[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          off[e] = 8u * (kGmresSlot * (g0 + 4 * e < gs.nwg ? g0 + 4 * e : blockIdx.x) + 2 * q);
+        ok = poll_values<4>(rb, off, ep, gs, wd);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          sum += g0 + 4 * e < gs.nwg ? words_value(wd[e][0], wd[e][1]) : 0.0;
       }
     }
     sum = group_sum<4>(sum);
-    if (q < nv && seg == 0) h[q] = sum;
+    if (q < nval && seg == 0) h[q] = sum;
+    stores_done();
     return __syncthreads_and(ok);
+  };
+  // h[0 .. nv) = V' w, and h[nv] = w' w with NORM
+  auto dots = [&](int nv, double* h, bool norm) -> bool {
+    const int q = t >> 2, seg = t & 3;
+    const int nval = nv + (norm ? 1 : 0);
+    double acc = 0, ac2 = 0;
+    if (q < nval) {
+      const KT* vq = q < nv ? V + q * S : w;
+#pragma unroll 6
+      for (int d = seg; d < DN; d += 8) {
+        acc += (double)vq[d] * (double)w[d];
+        ac2 += (double)vq[d + 4] * (double)w[d + 4];
+      }
+    }
+    return share(nval, acc + ac2, h);
   };
   auto subtract = [&](int nv, const double* h) {
     if (isd) {
       double s = 0;
+#pragma unroll 4
       for (int q = 0; q < nv; ++q) s += h[q] * (double)V[q * S + t];
       w[t] = (KT)((double)w[t] - s);
     }
     __syncthreads();
   };
+  // column j of the basis, w / |w|, and t = D^-1 w of the next product (K D^-1 v is
+  // K t / |w|)
+  auto next_column = [&](int j, double inv) {
+    if (live)
+      agent_store((Bits*)a.tb[j & 1] + dof,
+                  __builtin_bit_cast(Bits, d0 * w[n0] + d1 * w[n0 + 1] + d2 * w[n0 + 2]));
+    if (isd) V[j * S + t] = (KT)((double)w[t] * inv);
+  };
+  auto mark = [&](KT* y) {
+    if (live) agent_store((Bits*)y + dof, W::mark);
+  };
 
-  double beta0 = -1, beta = 0, n2 = 0;
+  double beta0 = -1, beta = 0;
   int total = 0;
   for (bool first = true;; first = false) {
     // r = b - K x on the free dofs
     KT rv = freed ? (KT)bd : KT(0);
+    mark(a.tb[0]);
+    mark(a.tb[1]);
     if (!first) {
       if (live) agent_store(a.x + dof, xs);
       stores_done();
       __syncthreads();
-      // the exchange that makes x visible (its value is not used)
-      ++ep;
-      if (t < 64) {
-        unsigned long long* reg = region(ep);
-        const SharedBuf rb = shared_buf(reg, 8u * kGmresSlot * kMaxGridWg);
-        if (lane < 2) agent_store(reg + (size_t)kGmresSlot * blockIdx.x + lane, value_word(0.0, ep, lane & 1));
-        bool ok = true;
-        for (int g = lane; ok && g < gs.nwg; g += 64) {
-          unsigned long long wd[1][2];
-          const uint32_t off[1] = {8u * kGmresSlot * g};
-        ok = poll_values<1>(rb, off, ep, gs, wd);
-        }
-        ok = __all(ok);
-        if (lane == 0) sc[1] = ok ? 1.0 : 0.0;
-      }
-      __syncthreads();
-      if (sc[1] == 0.0) return;
+      if (!share(1, 0.0, h1)) return;  // x is visible (the sum is not used)
       product(a.x, 1.0);
       rv = freed ? (KT)(bd - (double)w[isd ? t : 0]) : KT(0);
       __syncthreads();
     }
     if (isd) w[t] = rv;
+    stores_done();
     __syncthreads();
-    if (!norm_publish(n2, [] {})) return;
-    beta = sqrt(n2);
+    if (!dots(0, h1, true)) return;
+    beta = sqrt(h1[0]);
     if (beta0 < 0) beta0 = beta;
     if (!(beta > a.rtol * beta0) || total >= a.maxiter || beta0 == 0) break;
     double inv = 1.0 / beta;
-    if (isd) V[t] = (KT)((double)w[t] * inv);
-    double g = beta;
+    next_column(0, inv);
+    double g = beta, cs = 0, sn = 0;  // lane q of every wave: rotation q
     int k = 0;
     for (int j = 0; j < m; ++j) {
-      product(a.t, inv);
-      if (!dots(j + 1, h1)) return;
+      product(a.tb[j & 1], inv);
+      if (!dots(j + 1, h1, false)) return;
+      mark(a.tb[j & 1]);  // every workgroup has read it
       subtract(j + 1, h1);
-      if (!dots(j + 1, h2)) return;
+      if (!dots(j + 1, h2, true)) return;
       subtract(j + 1, h2);
-      // the earlier rotations applied to the new column, while the norm is summed
-      auto rotate = [&] {
-        if (t != T - 64) return;
-        double* col = Rm + j * (j + 1) / 2;
-        double e = h1[0] + h2[0];
-        for (int q = 0; q < j; ++q) {
-          const double f = h1[q + 1] + h2[q + 1];
-          col[q] = cs[q] * e + sn[q] * f;
-          e = -sn[q] * e + cs[q] * f;
-        }
-        sc[2] = e;
-      };
-      if (!norm_publish(n2, rotate)) return;
-      const double hn = sqrt(n2), e = sc[2], r = hypot(e, hn);
-      const double c = r > 0 ? e / r : 1.0, s = r > 0 ? hn / r : 0.0;
-      if (t == 0) {
-        Rm[j * (j + 1) / 2 + j] = r;
-        cs[j] = c;
-        sn[j] = s;
-        gv[j] = c * g;
+      const double n1 = h2[j + 1], c2 = lane <= j ? h2[lane] : 0.0;
+      double n2 = n1 - wave_sum(c2 * c2);
+      if (n2 < 0.25 * n1) {  // the same answer in every workgroup
+        if (!dots(0, h1 + 63, true)) return;
+        n2 = h1[63];
       }
+      const double hn = sqrt(n2);
+      if (hn > 0) {
+        inv = 1.0 / hn;
+        next_column(j + 1, inv);
+      }
+      // the earlier rotations applied to the new column
+      const double col = lane <= j ? h1[lane] + h2[lane] : 0.0;
+      double e = read_lane(col, 0), mine = 0;
+      for (int q = 0; q < j; ++q) {
+        const double f = read_lane(col, q + 1), cq = read_lane(cs, q), sq = read_lane(sn, q);
+        if (lane == q) mine = cq * e + sq * f;
+        e = cq * f - sq * e;
+      }
+      const double r = hypot(e, hn);
+      const double c = r > 0 ? e / r : 1.0, s = r > 0 ? hn / r : 0.0;
+      if (lane == j) {
+        cs = c;
+        sn = s;
+        mine = r;
+      }
+      if (t <= j) Rm[j * (j + 1) / 2 + t] = mine;
+      if (t == j) gv[j] = c * g;
       g = -s * g;
       ++total;
       k = j + 1;
       if (fabs(g) <= a.rtol * beta0 || total >= a.maxiter || !(hn > 0)) break;
-      inv = 1.0 / hn;
-      if (isd) V[(j + 1) * S + t] = (KT)((double)w[t] * inv);
     }
     __syncthreads();
     if (t < 64) {  // R y = g, a lane per unknown
@@ -537,7 +529,11 @@ __global__ __launch_bounds__(kGmresThreads) void k_gmres_resident(GmresArgs<KT> 
     if (live) xs += d0 * w[n0] + d1 * w[n0 + 1] + d2 * w[n0 + 2];
     __syncthreads();
   }
-  if (live) a.x[dof] = xs;
+  if (live) {
+    a.x[dof] = xs;
+    agent_store(a.tb[0] + dof, KT(0));  // no marks are left behind
+    agent_store(a.tb[1] + dof, KT(0));
+  }
   if (blockIdx.x == 0 && t == 0) {
     a.st->rr_last = beta * beta;
     a.st->bb = beta0 * beta0;
@@ -632,7 +628,8 @@ int gmres_t(Ctx* c, const double* b_dev, int m, int maxiter, double rtol) {
   a.b = b_dev;
   a.mask = c->d_fixmask;
   a.x = (KT*)c->d_px;
-  a.t = (KT*)c->d_pz;
+  a.tb[0] = (KT*)c->d_pp0;
+  a.tb[1] = (KT*)c->d_pp1;
   a.st = &c->d_sc->pcg;
   a.slots = c->d_gmslots;
   a.base = c->gslot_epoch;
@@ -713,10 +710,12 @@ int launch_gmres_resident(Ctx* c, const double* b_dev, int m, int maxiter, doubl
                                   hipMemcpyDeviceToHost, s));
   ONSAS_HIP_TRY(c, hipStreamSynchronize(s));
   const PcgState& ps = c->h_sc->pcg;
-  // an iteration takes 3 epochs, a restart 2
+  // an iteration takes at most 3 epochs, a restart 2
   c->gslot_epoch += (ps.aborted ? 5u * ((uint32_t)maxiter + 2) : (uint32_t)ps.k) + 2;
   if (ps.aborted) {
     c->pcg_resident = false;
+    for (void* v : {c->d_pp0, c->d_pp1})  // the launch may have left its marks there
+      ONSAS_HIP_TRY(c, hipMemsetAsync(v, 0, c->kt * 3 * (size_t)c->nn, s));
     return ONSAS_OK;
   }
   *ran = true;
