@@ -110,7 +110,7 @@ typedef struct {
     double scatter_ms;       /* element + block kernels (gather: state + gather pass; */
                              /* scatter: the colour launches)                        */
     double solve_ms;         /* residual + linear solve + update                     */
-    double pcg_ms;           /* PCG iterations only                                  */
+    double pcg_ms;           /* linear solves (whole steps that are one launch)      */
     int64_t n_assemble;
     int64_t n_steps;
     int64_t pcg_iters;

@@ -204,28 +204,11 @@ float elapsed(hipEvent_t a, hipEvent_t b) {
   return ms;
 }
 
-// Solve K x = b_dev with the configured linear solver; x left in the PCG x buffer (KT).
-int linear_solve(Ctx* c, const double* b_dev, bool forcing, int* iters, double* relres,
-                 int* converged, int* solver, const void* x0 = nullptr, int expect = -1) {
-  int it = 0, conv = 0, brk = 0;
+// The GMRES part of a linear solve; *solver, *iters: what PCG did before it.
+int gmres_solve(Ctx* c, const double* b_dev, int* iters, double* relres, int* converged,
+                int* solver) {
+  int conv = 0;
   double rr = 1.0;
-  *solver = 0;
-  *iters = 0;
-  const int kind = c->lin.kind;
-  if (kind == ONSAS_LINSOLVE_PCG || kind == ONSAS_LINSOLVE_AUTO) {
-    ONSAS_TRY(onsas::launch_pcg_solve(c, b_dev, forcing, &it, &rr, &conv, &brk, x0, expect));
-    *solver = 1;
-    *iters = it;
-    c->tm.pcg_iters += it;
-    if (brk && kind == ONSAS_LINSOLVE_PCG)
-      return set_err(c, ONSAS_ERR_LINEAR_SOLVE,
-                     "PCG breakdown (p'Kp <= 0): the tangent is not positive definite");
-    if (!brk) {
-      *relres = rr;
-      *converged = conv;
-      return ONSAS_OK;
-    }
-  }
   int git = 0;
   ONSAS_TRY(onsas::launch_gmres_solve(c, b_dev, &git, &rr, &conv));
   *solver = (*solver == 1) ? 3 : 2;
@@ -234,6 +217,40 @@ int linear_solve(Ctx* c, const double* b_dev, bool forcing, int* iters, double* 
   *relres = rr;
   *converged = conv;
   return ONSAS_OK;
+}
+
+// What a PCG solve of `it` iterations means for the linear solve it is the first
+// part of: *more = true asks for gmres_solve.
+int pcg_outcome(Ctx* c, int it, double rr, int conv, int brk, bool* more, int* iters,
+                double* relres, int* converged, int* solver) {
+  *solver = 1;
+  *iters = it;
+  c->tm.pcg_iters += it;
+  *more = brk != 0;
+  if (brk && c->lin.kind == ONSAS_LINSOLVE_PCG)
+    return set_err(c, ONSAS_ERR_LINEAR_SOLVE,
+                   "PCG breakdown (p'Kp <= 0): the tangent is not positive definite");
+  if (!brk) {
+    *relres = rr;
+    *converged = conv;
+  }
+  return ONSAS_OK;
+}
+
+// Solve K x = b_dev with the configured linear solver; x left in the PCG x buffer (KT).
+int linear_solve(Ctx* c, const double* b_dev, bool forcing, int* iters, double* relres,
+                 int* converged, int* solver, const void* x0 = nullptr, int expect = -1) {
+  *solver = 0;
+  *iters = 0;
+  if (c->lin.kind != ONSAS_LINSOLVE_GMRES) {
+    int it = 0, conv = 0, brk = 0;
+    double rr = 1.0;
+    bool more = false;
+    ONSAS_TRY(onsas::launch_pcg_solve(c, b_dev, forcing, &it, &rr, &conv, &brk, x0, expect));
+    ONSAS_TRY(pcg_outcome(c, it, rr, conv, brk, &more, iters, relres, converged, solver));
+    if (!more) return ONSAS_OK;
+  }
+  return gmres_solve(c, b_dev, iters, relres, converged, solver);
 }
 
 // Sums of the R2 / F2 partial rows written by launch_refine_residual (host,
@@ -605,32 +622,50 @@ int onsas_newton_step(onsas_ctx* ctx, onsas_step_stats* out) {
   std::memset(out, 0, sizeof *out);
   hipStream_t s = c->stream;
   ONSAS_HIP_TRY(c, hipEventRecord(c->ev[4], s));
-  ONSAS_TRY(onsas::launch_residual(c));
   int iters = 0, conv = 0, solver = 0;
   double relres = 0;
-  ONSAS_HIP_TRY(c, hipEventRecord(c->ev[5], s));
   // warm start from the previous load step's update of this Newton iteration
   const int j = c->newton_it++;
   const int prev = c->warm_cur ^ 1;
   const bool slot = c->warm_start && j < Ctx::kWarmSlots;
   const void* x0 = slot && c->warm_ok[prev][j] ? c->d_warm[prev][j] : nullptr;
   const bool pslot = c->pcg_predict && j < Ctx::kPredSlots;
-  ONSAS_TRY(linear_solve(c, c->d_res, true, &iters, &relres, &conv, &solver, x0,
-                         pslot ? c->pcg_pred[prev][j] : -1));
+  // small and mid-size models: the step is one launch (with its results), unless
+  // PCG breaks down in it
+  bool ran = false, more = false;
+  {
+    int it = 0, cv = 0, brk = 0;
+    double rr = 1.0;
+    ONSAS_TRY(onsas::launch_newton_resident(c, x0, slot ? c->d_warm[c->warm_cur][j] : nullptr, &ran,
+                                            &it, &rr, &cv, &brk));
+    if (ran) ONSAS_TRY(pcg_outcome(c, it, rr, cv, brk, &more, &iters, &relres, &conv, &solver));
+  }
+  const bool whole = ran && !more;
+  if (!whole) {
+    ONSAS_TRY(onsas::launch_residual(c));
+    ONSAS_HIP_TRY(c, hipEventRecord(c->ev[5], s));
+    if (more)
+      ONSAS_TRY(gmres_solve(c, c->d_res, &iters, &relres, &conv, &solver));
+    else
+      ONSAS_TRY(linear_solve(c, c->d_res, true, &iters, &relres, &conv, &solver, x0,
+                             pslot ? c->pcg_pred[prev][j] : -1));
+  }
   if (pslot) c->pcg_pred[c->warm_cur][j] = solver == 1 ? iters : -1;
   if (slot) {  // this step's update, for the next step (PCG solutions only)
     c->warm_ok[c->warm_cur][j] = solver == 1;
-    if (solver == 1)
+    if (solver == 1 && !whole)
       ONSAS_HIP_TRY(c, hipMemcpyAsync(c->d_warm[c->warm_cur][j], c->d_px, c->kt * 3 * c->nn,
                                       hipMemcpyDeviceToDevice, s));
   }
-  ONSAS_HIP_TRY(c, hipEventRecord(c->ev[6], s));
-  ONSAS_TRY(onsas::launch_update(c));
-  ONSAS_TRY(onsas::launch_finalize_newton(c));
-  ONSAS_HIP_TRY(c, hipEventRecord(c->ev[7], s));
-  ONSAS_HIP_TRY(c, hipMemcpyAsync(&c->h_sc->nwt, &c->d_sc->nwt, sizeof(onsas::NewtonStats),
-                                  hipMemcpyDeviceToHost, s));
-  ONSAS_HIP_TRY(c, hipStreamSynchronize(s));
+  if (!whole) {
+    ONSAS_HIP_TRY(c, hipEventRecord(c->ev[6], s));
+    ONSAS_TRY(onsas::launch_update(c));
+    ONSAS_TRY(onsas::launch_finalize_newton(c));
+    ONSAS_HIP_TRY(c, hipEventRecord(c->ev[7], s));
+    ONSAS_HIP_TRY(c, hipMemcpyAsync(&c->h_sc->nwt, &c->d_sc->nwt, sizeof(onsas::NewtonStats),
+                                    hipMemcpyDeviceToHost, s));
+    ONSAS_HIP_TRY(c, hipStreamSynchronize(s));
+  }
   account_assembly(c);
   const onsas::NewtonStats& nw = c->h_sc->nwt;
   out->r_norm = std::sqrt(nw.r2);
@@ -647,7 +682,7 @@ int onsas_newton_step(onsas_ctx* ctx, onsas_step_stats* out) {
   out->assemble_ms = c->last_assemble_ms;
   out->solve_ms = elapsed(c->ev[4], c->ev[7]);
   c->tm.solve_ms += out->solve_ms;
-  c->tm.pcg_ms += elapsed(c->ev[5], c->ev[6]);
+  c->tm.pcg_ms += whole ? out->solve_ms : elapsed(c->ev[5], c->ev[6]);
   c->tm.n_steps++;
   c->assembled = false;  // the tangent belongs to the previous U
   if (!std::isfinite(out->r_norm) || !std::isfinite(out->dU_norm))

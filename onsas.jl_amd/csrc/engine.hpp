@@ -20,6 +20,7 @@
 #include "../../include/onsas_hip.h"
 #include "grid_exchange.hpp"
 #include "host_setup.hpp"
+#include "inner_tol.hpp"
 
 namespace onsas {
 
@@ -446,7 +447,15 @@ int launch_pcg_solve(Ctx* c, const double* b_dev, bool forcing, int* iters, doub
 // ---- resident_solve.hip ----
 bool pcg_resident_fits(const Ctx* c);
 void pcg_resident_setup(Ctx* c);                                // at finalize
-int launch_pcg_resident(Ctx* c);                                // after the init kernels
+int launch_pcg_resident(Ctx* c, const double* b_dev, bool* ran, int* iters, double* relres,
+                        int* converged, int* breakdown);
+// A whole Newton step (residual, solve, update, norms) as one launch; *ran = false:
+// nothing has changed and the step is to be taken launch by launch.
+int launch_newton_resident(Ctx* c, const void* x0, void* warm, bool* ran, int* iters,
+                           double* relres, int* converged, int* breakdown);
+void pcg_result(const PcgState& ps, int* iters, double* relres, int* converged, int* breakdown);
+int pcg_maxiter(const Ctx* c);
+InnerTol inner_tol(const Ctx* c, bool forcing);
 int launch_gmres_resident(Ctx* c, const double* b_dev, int m, int maxiter, double rtol, bool* ran,
                           int* iters, double* relres, int* converged);
 // most iterations of a solve that runs as one launch (a bound on its time)

@@ -53,16 +53,30 @@ struct ResidentArgs {
   const int32_t* scol;
   const KT* sval;
   const KT* Dinv;
-  const KT* r;
-  const KT* z;
+  const uint8_t* mask;
+  const double* b;     // right-hand side; of a Newton step f_ext
   KT* x;
-  KT* zb[2];  // z of the odd and even iterations, handed from workgroup to workgroup
-  PcgState* st;
+  KT* zb[2];           // z of the even and odd iterations, handed from workgroup to workgroup
+  Scalars* sc;         // device: the abort word, a Newton step's norms
+  Scalars* host;       // pinned host: the results
   unsigned long long* slots;  // two regions of 8 words per workgroup, used in turn
   uint32_t base;              // epochs base + 1, base + 2, ... are new to the slots
   long long limit;
   int64_t nn;
+  int maxiter;
+  InnerTol tol;
+  // a Newton step (fint not null)
+  const double* fint;
+  const KT* x0;        // warm start or null
+  KT* warm;            // takes a copy of x, or null
+  double *res, *U;
 };
+
+// a result for the host, in pinned host memory
+template <typename T>
+__device__ inline void host_store(T* p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 // z of the columns at the byte offsets cj, each value once its owner has written
 // it; false once the wait has expired.
@@ -100,6 +114,14 @@ __device__ inline bool gather_published(SharedBuf z, const uint32_t (&cj)[NB], c
 // NB), T threads a workgroup.  Lanes 0, 1, 2 of a row hold the row's three
 // components of every vector.  ONE: a single workgroup, z and the sums in LDS.
 //
+// The launch starts from the right-hand side and ends with the results in pinned
+// host memory; of a Newton step it is all that follows the assembly: residual,
+// warm start, stopping tolerance, solve, update of U and norms (k_residual,
+// k_spmv_sell, k_warm_dots, k_warm_init, k_pcg_init_finalize, k_update and
+// k_finalize_newton of the general path, with two copies to the host and one on
+// the device: some 60 us of a step of 195 us at 125 nodes, now 5 us; the step
+// 195 -> 152 us).
+//
 // Hand-over of z: z_k (k >= 1) is published in zb[k & 1] after sum k - 1, and
 // marked unwritten again after sum k, by when every workgroup has read it; the
 // marks are complete before their workgroup's part of sum k + 1 is published,
@@ -117,11 +139,26 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs<KT> a) {
   const int64_t i = ((int64_t)blockIdx.x * T + t) / L;
   const bool row = i < a.nn;
   const bool own = row && ph < 3;
-  PcgState* st = a.st;
-  const double tol2 = st->tol2;
-  const int maxiter = st->maxiter;
-  GridSlots gs{a.slots, (int)gridDim.x, &st->aborted, a.limit};  // sums of the even iterations
-  GridSlots go{a.slots + 8 * kMaxGridWg, (int)gridDim.x, &st->aborted, a.limit};
+  uint32_t ep = a.base;
+  // the four sums over the launch; false (and *host says so) once it is aborted
+  auto sums = [&](double(&s)[4]) -> bool {
+    ++ep;
+    if (ONE) {
+      const double p = wave_sum4(s);
+      if ((t & 63) < 4) sh[4 * (t >> 6) + (t & 63)] = p;
+      __syncthreads();
+      const double q4 = wg_sum4<T>(sh);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) s[q] = read_lane(q4, q);
+      return true;
+    }
+    const GridSlots gs{a.slots + (ep & 1u) * (8 * kMaxGridWg), (int)gridDim.x, &a.sc->pcg.aborted,
+                       a.limit};
+    if (grid_sum4<T>(s, gs, ep, sh, &late)) return true;
+    if (t == 0) host_store(&a.host->pcg.aborted, 1);
+    return false;
+  };
+  const GridSlots gw{nullptr, (int)gridDim.x, &a.sc->pcg.aborted, a.limit};
 
   KT v[NB][9];
   uint32_t cj[NB];  // the column's z: its byte offset, or its index in shz
@@ -139,39 +176,8 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs<KT> a) {
       for (int e = 0; e < 9; ++e) v[q][e] = has ? a.sval[9 * b + 64 * e + l] : KT(0);
     }
   }
-  KT xs = 0, rs = 0, zs = 0, ps = 0, qs = 0, d0 = 0, d1 = 0, d2 = 0;
-  if (own) {
-    xs = a.x[3 * i + ph];
-    rs = a.r[3 * i + ph];
-    zs = a.z[3 * i + ph];
-    d0 = a.Dinv[9 * i + 3 * ph];
-    d1 = a.Dinv[9 * i + 3 * ph + 1];
-    d2 = a.Dinv[9 * i + 3 * ph + 2];
-    if (ONE) {
-      shz[4 * i + ph] = zs;
-    } else {
-      agent_store((Bits*)a.zb[0] + 3 * i + ph, W::mark);
-      agent_store((Bits*)a.zb[1] + 3 * i + ph, W::mark);
-    }
-  }
-  if (t == 0) late = 0;
-  __syncthreads();
-
-  const uint32_t zbytes = 3u * (uint32_t)sizeof(KT) * (uint32_t)a.nn;
-  const SharedBuf z0 = shared_buf(a.zb[0], zbytes), z1 = shared_buf(a.zb[1], zbytes),
-                  zi = shared_buf(a.z, zbytes);
-  double rz = 0, rr = 0, rzp = 0, pq = 0;
-  int k = 0, conv = 0, brk = 0;
-  for (;; ++k) {
-    KT zj[NB][3];
-    if (ONE) {
-#pragma unroll
-      for (int q = 0; q < NB; ++q)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) zj[q][c] = shz[cj[q] + c];
-    } else if (!gather_published<KT, NB>(k > 0 ? ((k & 1) ? z1 : z0) : zi, cj, gs, zj)) {
-      late = 1;
-    }
+  // w = K z of the row's component ph from the columns' z
+  auto product = [&](const KT(&zj)[NB][3]) -> KT {
     KT a0 = 0, a1 = 0, a2 = 0;
 #pragma unroll
     for (int q = 0; q < NB; ++q) {
@@ -182,29 +188,110 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs<KT> a) {
     a0 = group_sum<L>(a0);
     a1 = group_sum<L>(a1);
     a2 = group_sum<L>(a2);
-    const KT w = ph == 0 ? a0 : (ph == 1 ? a1 : a2);
-    double sm[4] = {0, 0, 0, 0};
+    return ph == 0 ? a0 : (ph == 1 ? a1 : a2);
+  };
+  const int64_t dof = 3 * i + ph;
+  const bool newton = a.fint != nullptr;
+  KT xs = 0, rs = 0, zs = 0, ps = 0, qs = 0, d0 = 0, d1 = 0, d2 = 0, bk = 0;
+  double u = 0, sm[4] = {0, 0, 0, 0};
+  bool freed = false;
+  if (own) {
+    freed = !((a.mask[i] >> ph) & 1u);
+    d0 = a.Dinv[9 * i + 3 * ph];
+    d1 = a.Dinv[9 * i + 3 * ph + 1];
+    d2 = a.Dinv[9 * i + 3 * ph + 2];
+    const double be = a.b[dof];
+    double r = be;
+    if (newton) {
+      u = a.U[dof];
+      r -= a.fint[dof];
+      sm[1] = be * be;
+    }
+    if (!freed) r = 0;
+    if (newton) {
+      a.res[dof] = r;
+      sm[0] = r * r;
+    }
+    bk = (KT)r;
+    if (!ONE) {
+      agent_store((Bits*)a.zb[0] + dof, W::mark);
+      agent_store((Bits*)a.zb[1] + dof, W::mark);
+    }
+  }
+  // warm start: x = al x0, r = b - al t with t = K x0 and al = t.b / t.t, the scale
+  // that minimises ||b - al t|| (as k_warm_init)
+  KT x0 = 0, tw = 0;
+  if (a.x0) {
+    KT xj[NB][3];
+#pragma unroll
+    for (int q = 0; q < NB; ++q)
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+        xj[q][c] = ONE ? a.x0[cj[q] / 4 * 3 + c] : ((const KT*)((const char*)a.x0 + cj[q]))[c];
+    tw = product(xj);
+    if (own && freed) {
+      x0 = a.x0[dof];
+      sm[2] = (double)tw * (double)bk;
+      sm[3] = (double)tw * (double)tw;
+    }
+  }
+  if (t == 0) late = 0;
+  __syncthreads();
+  if (!sums(sm)) return;  // past it no workgroup sees what zb held before
+  const double r2 = sm[0], f2 = sm[1];
+  const double al = a.x0 && sm[3] > 0 && isfinite(sm[2]) && isfinite(sm[3]) ? sm[2] / sm[3] : 0.0;
+  if (own) {
+    xs = freed ? (KT)(al * (double)x0) : KT(0);
+    rs = freed ? (a.x0 ? (KT)((double)bk - al * (double)tw) : bk) : KT(0);
+  }
+  // z = D^-1 r, published for iteration k
+  auto next_z = [&](int k) {
+    const KT r0 = quad_lane<0>(rs), r1 = quad_lane<1>(rs), rz2 = quad_lane<2>(rs);
+    if (own) {
+      zs = d0 * r0 + d1 * r1 + d2 * rz2;
+      if (ONE)
+        shz[4 * i + ph] = zs;
+      else
+        agent_store((Bits*)a.zb[k & 1] + dof, __builtin_bit_cast(Bits, zs));
+    }
+    if (ONE) __syncthreads();
+  };
+  next_z(0);
+
+  const uint32_t zbytes = 3u * (uint32_t)sizeof(KT) * (uint32_t)a.nn;
+  const SharedBuf z0 = shared_buf(a.zb[0], zbytes), z1 = shared_buf(a.zb[1], zbytes);
+  double rz = 0, rr = 0, rzp = 0, pq = 0, bb = 0, eta = 0, tol2 = 0;
+  int k = 0, conv = 0, brk = 0;
+  for (;; ++k) {
+    KT zj[NB][3];
+    if (ONE) {
+#pragma unroll
+      for (int q = 0; q < NB; ++q)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) zj[q][c] = shz[cj[q] + c];
+    } else if (!gather_published<KT, NB>((k & 1) ? z1 : z0, cj, gw, zj)) {
+      late = 1;
+    }
+    const KT w = product(zj);
+    sm[0] = sm[1] = sm[2] = sm[3] = 0;
     if (own) {
       sm[0] = (double)rs * (double)zs;
       sm[1] = (double)rs * (double)rs;
       sm[2] = (double)zs * (double)w;
-      sm[3] = (double)zs * (double)qs + (double)ps * (double)w;
+      sm[3] = k > 0 ? (double)zs * (double)qs + (double)ps * (double)w : (double)bk * (double)bk;
     }
-    if (ONE) {
-      const double p = wave_sum4(sm);
-      if ((t & 63) < 4) sh[4 * (t >> 6) + (t & 63)] = p;
-      __syncthreads();
-      const double s = wg_sum4<T>(sh);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) sm[q] = read_lane(s, q);
-    } else if (!grid_sum4<T>(sm, (k & 1) ? go : gs, a.base + 1 + (uint32_t)k, sh, &late)) {
-      return;
+    if (!sums(sm)) return;
+    if (k == 0) {
+      bb = sm[3];
+      sm[3] = 0;
+      eta = inner_eta(a.tol, bb, f2, a.tol.forcing ? a.sc->nwt.prev_b2 : 0.0);
+      tol2 = eta * eta * bb;
     }
     rzp = rz;
     rz = sm[0];
     rr = sm[1];
     conv = rr <= tol2;
-    if (conv || k >= maxiter) break;
+    if (conv || k >= a.maxiter) break;
     const KT beta = (KT)(k > 0 ? rz / rzp : 0.0);
     pq = sm[2] + (double)beta * (sm[3] + (double)beta * pq);
     if (!(pq > 0.0) || !isfinite(pq) || !isfinite(rz)) {
@@ -217,36 +304,54 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs<KT> a) {
       qs = w + beta * qs;
       xs += alpha * ps;
       rs -= alpha * qs;
+      if (!ONE) agent_store((Bits*)a.zb[k & 1] + dof, W::mark);  // every workgroup has read it
     }
-    const KT r0 = quad_lane<0>(rs), r1 = quad_lane<1>(rs), r2 = quad_lane<2>(rs);
-    if (own) {
-      zs = d0 * r0 + d1 * r1 + d2 * r2;
-      if (ONE) {
-        shz[4 * i + ph] = zs;
-      } else {
-        agent_store((Bits*)a.zb[(k + 1) & 1] + 3 * i + ph, __builtin_bit_cast(Bits, zs));
-        agent_store((Bits*)a.zb[k & 1] + 3 * i + ph, W::mark);
-      }
-    }
-    if (ONE) __syncthreads();
+    next_z(k + 1);
   }
   if (own) {
-    a.x[3 * i + ph] = xs;
+    a.x[dof] = xs;
     if (!ONE) {  // no marks are left behind
-      agent_store(a.zb[0] + 3 * i + ph, KT(0));
-      agent_store(a.zb[1] + 3 * i + ph, KT(0));
+      agent_store(a.zb[0] + dof, KT(0));
+      agent_store(a.zb[1] + dof, KT(0));
+    }
+  }
+  // Newton update: U[free] += x, with the norms of x and of U before
+  double du = 0;
+  sm[0] = sm[1] = sm[2] = sm[3] = 0;
+  if (newton && !brk) {
+    if (own) {
+      du = freed ? (double)xs : 0.0;
+      sm[0] = du * du;
+      sm[1] = u * u;
+    }
+    if (ONE) __syncthreads();  // the last sums have been read
+    if (!sums(sm)) return;
+    if (own) {
+      a.U[dof] = u + du;
+      if (a.warm) a.warm[dof] = xs;
     }
   }
   if (blockIdx.x == 0 && t == 0) {
-    st->rr_last = rr;
-    st->k = k;
-    if (brk) {
-      st->breakdown = 1;
-      st->breakdown_k = k;
-    } else {
-      st->done = 1;
-      st->iters = k;
-      st->converged = conv;
+    PcgState* st = &a.host->pcg;
+    host_store(&st->bb, bb);
+    host_store(&st->rr_last, rr);
+    host_store(&st->k, k);
+    host_store(&st->breakdown, brk);
+    host_store(&st->breakdown_k, brk ? k : -1);
+    host_store(&st->iters, k);
+    host_store(&st->converged, brk ? 0 : conv);
+    host_store(&st->done, 1);
+    if (newton) {
+      NewtonStats* nw = &a.host->nwt;
+      host_store(&nw->r2, r2);
+      host_store(&nw->fext2, f2);
+      host_store(&nw->dU2, sm[0]);
+      host_store(&nw->U2, sm[1]);
+      if (a.tol.forcing) {  // every workgroup has passed its reading of the old one
+        a.sc->nwt.prev_b2 = bb;
+        host_store(&nw->prev_b2, bb);
+        host_store(&nw->eta, eta);
+      }
     }
   }
 }
@@ -589,7 +694,7 @@ void run_resident(Ctx* c, const ResidentArgs<KT>& a, const ResidentShape& sh) {
 }
 
 template <typename KT>
-int resident_t(Ctx* c) {
+int resident_t(Ctx* c, const double* b, const double* fint, const void* x0, void* warm) {
   ResidentArgs<KT> a{};
   a.sell_ptr = c->d_sell_ptr;
   a.slice_rounds = c->d_slice_rounds;
@@ -597,13 +702,21 @@ int resident_t(Ctx* c) {
   a.scol = c->d_sell_col;
   a.sval = (const KT*)c->d_Ksell;
   a.Dinv = (const KT*)c->d_Dinv;
-  a.r = (const KT*)c->d_pr;
-  a.z = (const KT*)c->d_pz;
+  a.mask = c->d_fixmask;
+  a.b = b;
   a.x = (KT*)c->d_px;
   a.zb[0] = (KT*)c->d_pp0;
   a.zb[1] = (KT*)c->d_pp1;
-  a.st = &c->d_sc->pcg;
+  a.sc = c->d_sc;
+  a.host = c->h_sc;
   a.slots = c->d_gslots;
+  a.maxiter = pcg_maxiter(c);
+  a.tol = inner_tol(c, fint != nullptr);
+  a.fint = fint;
+  a.x0 = (const KT*)x0;
+  a.warm = (KT*)warm;
+  a.res = c->d_res;
+  a.U = c->d_U;
   a.base = c->gslot_epoch;
   a.limit = c->gslot_ticks;
   a.nn = c->nn;
@@ -677,9 +790,58 @@ static int renew_epochs(Ctx* c) {
   return ONSAS_OK;
 }
 
-int launch_pcg_resident(Ctx* c) {
+// Launches, waits and takes the results; *ran = false once a wait has expired (the
+// GPU was too busy to hold the whole grid): the context keeps to the general
+// kernels from then on.
+static int resident_run(Ctx* c, const double* b, const double* fint, const void* x0, void* warm,
+                        bool* ran, int* iters, double* relres, int* converged, int* breakdown) {
+  hipStream_t s = c->stream;
   ONSAS_TRY(renew_epochs(c));
-  return c->precision == ONSAS_PRECISION_FP64 ? resident_t<double>(c) : resident_t<float>(c);
+  c->h_sc->pcg = PcgState{};
+  ONSAS_TRY(c->precision == ONSAS_PRECISION_FP64 ? resident_t<double>(c, b, fint, x0, warm)
+                                                 : resident_t<float>(c, b, fint, x0, warm));
+  if (fint) ONSAS_HIP_TRY(c, hipEventRecord(c->ev[7], s));
+  ONSAS_HIP_TRY(c, hipStreamSynchronize(s));
+  const PcgState& ps = c->h_sc->pcg;
+  *ran = ps.done && !ps.aborted;
+  c->gslot_epoch += (*ran ? (uint32_t)ps.k : (uint32_t)pcg_maxiter(c)) + 4;
+  if (!*ran) {
+    c->pcg_resident = false;
+    for (void* v : {c->d_pp0, c->d_pp1})  // the launch may have left its marks there
+      ONSAS_HIP_TRY(c, hipMemsetAsync(v, 0, c->kt * 3 * (size_t)c->nn, s));
+    return ONSAS_OK;
+  }
+  pcg_result(ps, iters, relres, converged, breakdown);
+  return ONSAS_OK;
+}
+
+inline bool pcg_resident_now(const Ctx* c) {
+  return c->pcg_resident && c->lin.precond != ONSAS_PRECOND_AMG &&
+         pcg_maxiter(c) <= kMaxResidentIters;
+}
+
+int launch_pcg_resident(Ctx* c, const double* b_dev, bool* ran, int* iters, double* relres,
+                        int* converged, int* breakdown) {
+  *ran = false;
+  if (!pcg_resident_now(c)) return ONSAS_OK;
+  return resident_run(c, b_dev, nullptr, nullptr, nullptr, ran, iters, relres, converged, breakdown);
+}
+
+int launch_newton_resident(Ctx* c, const void* x0, void* warm, bool* ran, int* iters,
+                           double* relres, int* converged, int* breakdown) {
+  *ran = false;
+  if (!pcg_resident_now(c) || c->lin.kind == ONSAS_LINSOLVE_GMRES) return ONSAS_OK;
+  const double prev_b2 = c->h_sc->nwt.prev_b2;
+  ONSAS_TRY(resident_run(c, c->d_fext, c->d_fint, x0, warm, ran, iters, relres, converged,
+                         breakdown));
+  if (!*ran) {  // U and the forcing's memory as they were (some workgroups may have got that far)
+    ONSAS_HIP_TRY(c, hipMemcpyAsync(c->d_U, c->d_Uasm, 3 * c->nn * sizeof(double),
+                                    hipMemcpyDeviceToDevice, c->stream));
+    c->h_sc->nwt.prev_b2 = prev_b2;
+    ONSAS_HIP_TRY(c, hipMemcpyAsync(&c->d_sc->nwt.prev_b2, &c->h_sc->nwt.prev_b2, sizeof(double),
+                                    hipMemcpyHostToDevice, c->stream));
+  }
+  return ONSAS_OK;
 }
 
 // GMRES of the current tangent in one launch, where the model and the restart

@@ -423,6 +423,7 @@ int finalize_model(Ctx* c) {
   c->d_gslots = (unsigned long long*)(c->d_part + kPartArrays * kMaxPartials);  // zero: no epoch
   ONSAS_TRY(dev_alloc(c, (void**)&c->d_sc, sizeof(Scalars)));
   ONSAS_HIP_TRY(c, hipHostMalloc((void**)&c->h_sc, sizeof(Scalars), hipHostMallocDefault));
+  *c->h_sc = Scalars{};
   ONSAS_HIP_TRY(c, hipHostMalloc((void**)&c->h_stage, sizeof(double) * n, hipHostMallocDefault));
   for (double*& h : c->h_snap)
     ONSAS_HIP_TRY(c, hipHostMalloc((void**)&h, sizeof(double) * n, hipHostMallocDefault));

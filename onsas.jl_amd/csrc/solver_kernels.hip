@@ -268,44 +268,19 @@ __global__ __launch_bounds__(NT) void k_pcg_init(const double* __restrict__ b,
   }
 }
 
-// Stopping rule of the inner solve.  Fixed: ||r|| <= rtol ||b||.  Forcing
-// (inexact Newton): eta = max(0.9 (||b_k|| / ||b_{k-1}||)^2 [Eisenstat-Walker
-// choice 2, gamma = 0.9, alpha = 2], kForcingGuard tau / ||b_k||) clamped to
-// [rtol, eta_max], where b_k is this Newton iteration's residual and
-// tau = newton_tol ||f_ext|| the outer target: no inner accuracy is bought
-// beyond what the quadratic model or the outer tolerance can use.  The first
-// iteration of a load step uses eta_first.
-//
-// kForcingGuard = 0.5 is the safeguard of C. T. Kelley, Iterative Methods for
-// Linear and Nonlinear Equations (SIAM 1995), sec. 6.3.  On the 64^3 cube
-// (80 Newton iterations at every factor tried) it took the mixed solve from
-// 425 PCG iterations / 0.149 s at 0.1 to 379 / 0.137 s (FP64 384 -> 350),
-// with 1.0 at 363 / 0.133 s: 0.5 keeps the last inner solve a factor of two
-// inside the outer tolerance.
-constexpr double kForcingGuard = 0.5;
+// Start of a solve: ||b||^2, the stopping tolerance and a fresh state.
 __global__ __launch_bounds__(NT) void k_pcg_init_finalize(const double* __restrict__ pbb,
                                                             const double* __restrict__ pf2,
                                                             PcgState* __restrict__ st,
-                                                            NewtonStats* __restrict__ nw, double rtol,
-                                                            int maxiter, int np, int forcing,
-                                                            double newton_tol, double eta_max,
-                                                            double eta_first, double guard) {
+                                                            NewtonStats* __restrict__ nw,
+                                                            InnerTol tol, int maxiter, int np) {
   __shared__ double sh[NT / 64];
   const double bb = sum_parts(pbb, np, sh);
-  double eta = rtol;
-  if (forcing) {
-    const double ff = sum_parts(pf2, np, sh);
-    const double tau = newton_tol * sqrt(ff);
-    const double prev = nw->prev_b2;
-    double e = prev > 0 ? 0.9 * (bb / prev) : eta_first;
-    if (bb > 0) e = fmax(e, guard * tau / sqrt(bb));
-    // the residual already meets the outer tolerance: this solve only refines
-    // (the reference applies it before its convergence test sees the residual)
-    const double cap = (bb > 0 && sqrt(bb) <= tau) ? fmax(eta_max, 0.5) : eta_max;
-    eta = fmin(fmax(e, rtol), cap);
-  }
+  const double ff = tol.forcing ? sum_parts(pf2, np, sh) : 0.0;
+  const double eta = inner_eta(tol, bb, ff, tol.forcing ? nw->prev_b2 : 0.0);
+  __syncthreads();  // every thread has read the previous ||b||^2
   if (threadIdx.x == 0) {
-    if (forcing) {
+    if (tol.forcing) {
       nw->prev_b2 = bb;
       nw->eta = eta;
     }
@@ -1149,23 +1124,20 @@ int build_pcg_graph(Ctx* c, int slot, int iters) {
   return ONSAS_OK;
 }
 
-void pcg_result(const PcgState& ps, int* iters, double* relres, int* converged, int* breakdown) {
-  *iters = ps.breakdown ? ps.breakdown_k : ps.iters;
-  *converged = ps.converged;
-  *breakdown = ps.breakdown;
-  *relres = ps.bb > 0 ? std::sqrt(ps.rr_last / ps.bb) : 0.0;
-}
-
 template <typename KT>
 int pcg_solve_t(Ctx* c, const double* b_dev, bool forcing, const void* x0, int expect, int* iters,
                 double* relres, int* converged, int* breakdown) {
   hipStream_t s = c->stream;
   const int np = c->np;
-  const double rtol = linear_rtol(c);
-  const int maxiter = c->lin.maxiter > 0 ? c->lin.maxiter : (int)std::min<int64_t>(c->nfree, 1 << 30);
+  const int maxiter = pcg_maxiter(c);
   int chunk_iters = c->lin.check_every > 0 ? c->lin.check_every : 16;
   chunk_iters += chunk_iters & 1;  // even: the parity ping-pong repeats per chunk
   const bool amg = c->lin.precond == ONSAS_PRECOND_AMG;
+  if (!forcing) {  // Newton steps have launch_newton_resident
+    bool ran = false;
+    ONSAS_TRY(launch_pcg_resident(c, b_dev, &ran, iters, relres, converged, breakdown));
+    if (ran) return ONSAS_OK;
+  }
   if (amg) {  // hierarchy on first use; coarse numerics per the refresh policy
     if (!c->amg.built) ONSAS_TRY(amg_build(c));
     const int pol = c->lin.amg_refresh;
@@ -1204,34 +1176,9 @@ int pcg_solve_t(Ctx* c, const double* b_dev, bool forcing, const void* x0, int e
     }
   };
   init_vectors();
-  const bool f = forcing && c->lin.forcing;
   hipLaunchKernelGGL(k_pcg_init_finalize, dim3(1), dim3(NT), 0, s, part(c, kPartBB),
-                     part(c, kPartF2), &c->d_sc->pcg, &c->d_sc->nwt, rtol, maxiter, np, f ? 1 : 0,
-                     c->lin.newton_tol, c->lin.eta_max > 0 ? c->lin.eta_max : 0.1,
-                     c->lin.eta_first > 0 ? c->lin.eta_first : 1e-3, kForcingGuard);
-  if (c->pcg_resident && !amg && maxiter <= kMaxResidentIters) {
-    ONSAS_TRY(launch_pcg_resident(c));
-    ONSAS_HIP_TRY(c, hipMemcpyAsync(&c->h_sc->pcg, &c->d_sc->pcg, sizeof(PcgState),
-                                    hipMemcpyDeviceToHost, s));
-    ONSAS_HIP_TRY(c, hipStreamSynchronize(s));
-    PcgState& ps = c->h_sc->pcg;
-    c->gslot_epoch += (ps.aborted ? (uint32_t)maxiter : (uint32_t)ps.k) + 2;
-    if (!ps.aborted) {
-      pcg_result(ps, iters, relres, converged, breakdown);
-      return ONSAS_OK;
-    }
-    // a wait expired (the GPU was too busy to hold the whole grid): this solve
-    // starts again on the kernels below, which the context keeps to from here
-    c->pcg_resident = false;
-    ps.k = ps.done = ps.iters = ps.breakdown = ps.converged = ps.aborted = 0;
-    ps.breakdown_k = -1;
-    ps.rr_last = ps.bb;
-    for (void* v : {c->d_pp0, c->d_pp1})  // the launch may have left its marks there
-      hipLaunchKernelGGL(k_fill_kt<KT>, dim3(grid_for(3 * c->nn, 256)), dim3(256), 0, s, (KT*)v,
-                         3 * c->nn, KT(0));
-    ONSAS_HIP_TRY(c, hipMemcpyAsync(&c->d_sc->pcg, &ps, sizeof(PcgState), hipMemcpyHostToDevice, s));
-    init_vectors();
-  }
+                     part(c, kPartF2), &c->d_sc->pcg, &c->d_sc->nwt, inner_tol(c, forcing), maxiter,
+                     np);
   if (amg) {
     // a (warm) start that already meets the tolerance stops in the prologue of
     // the cycle's first fine-level product, before the preconditioner
@@ -1410,12 +1357,29 @@ int launch_pcg_solve(Ctx* c, const double* b_dev, bool forcing, int* iters, doub
              : pcg_solve_t<float>(c, b_dev, forcing, x0, expect, iters, relres, converged, breakdown);
 }
 
+int pcg_maxiter(const Ctx* c) {
+  return c->lin.maxiter > 0 ? c->lin.maxiter : (int)std::min<int64_t>(c->nfree, 1 << 30);
+}
+
+InnerTol inner_tol(const Ctx* c, bool forcing) {
+  return {linear_rtol(c), c->lin.newton_tol, c->lin.eta_max > 0 ? c->lin.eta_max : 0.1,
+          c->lin.eta_first > 0 ? c->lin.eta_first : 1e-3, forcing && c->lin.forcing ? 1 : 0};
+}
+
+void pcg_result(const PcgState& ps, int* iters, double* relres, int* converged, int* breakdown) {
+  *iters = ps.breakdown ? ps.breakdown_k : ps.iters;
+  *converged = ps.converged;
+  *breakdown = ps.breakdown;
+  *relres = ps.bb > 0 ? std::sqrt(ps.rr_last / ps.bb) : 0.0;
+}
+
 double linear_rtol(const Ctx* c) {
   return c->lin.rtol > 0 ? c->lin.rtol
                          : (c->precision == ONSAS_PRECISION_FP64 ? 1.4901161193847656e-08 : 1e-6);
 }
 
 int reset_forcing(Ctx* c) {
+  c->h_sc->nwt.prev_b2 = 0;  // the host's copy (launch_newton_resident)
   ONSAS_HIP_TRY(c, hipMemsetAsync(&c->d_sc->nwt.prev_b2, 0, sizeof(double), c->stream));
   return ONSAS_OK;
 }
@@ -1532,7 +1496,7 @@ int gmres_solve_t(Ctx* c, const double* b_dev, int* iters, double* relres, int* 
   const int m = std::max(2, c->lin.gmres_restart > 0 ? c->lin.gmres_restart : 40);
   const int64_t n = 3 * c->nn;
   const double rtol = linear_rtol(c);
-  const int maxiter = c->lin.maxiter > 0 ? c->lin.maxiter : (int)std::min<int64_t>(c->nfree, 1 << 30);
+  const int maxiter = pcg_maxiter(c);
   bool ran = false;
   ONSAS_TRY(launch_gmres_resident(c, b_dev, m, maxiter, rtol, &ran, iters, relres, converged));
   if (ran) return ONSAS_OK;

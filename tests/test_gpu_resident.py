@@ -4,6 +4,7 @@ lanes a row, models just past its limits, and the path a launch takes when a
 wait for the other workgroups expires."""
 import numpy as np
 import pytest
+from scipy.sparse.linalg import eigsh
 
 from onsas_amd import _capi, meshes
 from onsas_amd._capi import Context
@@ -113,3 +114,96 @@ def test_expired_wait_solves_on_the_general_path(monkeypatch, prec, kind):
     monkeypatch.setenv("ONSAS_RESIDENT_TICKS", "-1")
     _, res, bound = _solve(MODELS["10x10x10"], prec, rtol, kind)
     assert res <= bound
+
+
+def _newton_run(make, prec, forcing=False, kind=_capi.LINSOLVE_AUTO, steps=2, its=6):
+    """`steps` load steps of `its` Newton iterations (the later steps start warm): U after
+    every iteration, the statistics and the last tangent on the free dofs."""
+    c, nn = make(prec)
+    try:
+        c.set_linear_solver(kind, rtol=1e-6 if prec == _capi.PRECISION_MIXED else 1e-10,
+                            maxiter=20000, forcing=forcing, newton_tol=1e-8 if forcing else 0.0)
+        f = np.zeros((nn, 3))
+        f[:, 0], f[:, 2] = 4e3 / nn, -2e3 / nn
+        c.set_U(np.zeros(3 * nn))
+        Us, log = [], []
+        for s in range(steps):
+            c.set_loads(nodal=(s + 1.0) * f.reshape(-1))
+            for _ in range(its):
+                c.assemble()
+                log.append(c.newton_step())
+                Us.append(c.get_U())
+        fnorm = np.linalg.norm(c.get_fext())
+        c.assemble()
+        K = c.tangent_bsr().tocsr()
+        free = np.flatnonzero(np.asarray(abs(K).sum(axis=1)).ravel() != 1)
+        K = K[free][:, free].tocsc()
+        return Us, log, K, fnorm
+    finally:
+        c.close()
+
+
+def _stat(st, name):
+    return st[name] if isinstance(st, dict) else getattr(st, name)
+
+
+def _compare_newton(make, prec, monkeypatch, forcing=False, solver=1):
+    its = 6 if not forcing else 9
+    U, log, K, fn = _newton_run(make, prec, forcing, its=its)
+    monkeypatch.setenv("ONSAS_PCG_RESIDENT", "0")
+    Ug, logg, _, _ = _newton_run(make, prec, forcing, its=its)
+    first, firstg = log[0], logg[0]
+    for name in ("r_norm", "fext_norm", "U_norm"):  # of the same data, in another order
+        assert np.isclose(_stat(first, name), _stat(firstg, name), rtol=1e-12, atol=0)
+    for s in (log, logg):
+        assert all(_stat(d, "lin_solver") == solver for d in s)
+    # both end within eps of their last residuals' preimage: |U - U'| <= (|r| + |r'|) / smin(K)
+    lam = abs(eigsh(K, k=1, sigma=0, return_eigenvectors=False)[0])
+    for k in (its - 1, 2 * its - 1):
+        r, rg = _stat(log[k], "r_norm"), _stat(logg[k], "r_norm")
+        assert r <= 1e-6 * fn and rg <= 1e-6 * fn
+        assert np.linalg.norm(U[k] - Ug[k]) <= 2 * (r + rg) / lam + 1e-12 * np.linalg.norm(Ug[k])
+    return log, logg
+
+
+@pytest.mark.parametrize("forcing", [False, True])
+@pytest.mark.parametrize("prec", [_capi.PRECISION_MIXED, _capi.PRECISION_FP64])
+@pytest.mark.parametrize("model", ["1x1x1", "4x3x2", "6x4x3", "10x5x3", "10x10x10"])
+def test_resident_newton_step(monkeypatch, model, prec, forcing):
+    """The one-launch Newton step against the step launch by launch."""
+    print(f"[gpu] resident newton {model} precision {prec} forcing {forcing}", flush=True)
+    log, logg = _compare_newton(MODELS[model], prec, monkeypatch, forcing)
+    assert abs(_stat(log[0], "lin_iters") - _stat(logg[0], "lin_iters")) <= \
+        2 + _stat(logg[0], "lin_iters") // 20
+
+
+@pytest.mark.parametrize("prec", [_capi.PRECISION_MIXED, _capi.PRECISION_FP64])
+def test_resident_newton_breakdown(monkeypatch, prec):
+    """A negative definite tangent: PCG breaks down inside the launch, GMRES takes over."""
+    print(f"[gpu] resident newton, breakdown, precision {prec}", flush=True)
+
+    def make(p):
+        sm = meshes.cube(4, ny=3, nz=2, jitter=0.05, seed=4)
+        c = Context(p)
+        c.set_nodes(sm.coords)
+        c.add_tet_group(sm.tets, _capi.MAT_NEOHOOKEAN, (-8.3e5, -3.8e5))
+        c.set_fixed_dofs((3 * sm.node_sets["x0"][:, None] + np.arange(3)).reshape(-1))
+        c.finalize()
+        return c, sm.nn
+
+    _compare_newton(make, prec, monkeypatch, solver=3)
+
+
+@pytest.mark.parametrize("prec", [_capi.PRECISION_MIXED, _capi.PRECISION_FP64])
+def test_resident_newton_expired_wait(monkeypatch, prec):
+    """A step whose launch gave up is taken again from the state before it, bit for bit."""
+    print(f"[gpu] resident newton, expired wait, precision {prec}", flush=True)
+    monkeypatch.setenv("ONSAS_RESIDENT_TICKS", "-1")
+    U, log, _, _ = _newton_run(MODELS["10x10x10"], prec, forcing=True, its=3)
+    monkeypatch.setenv("ONSAS_PCG_RESIDENT", "0")
+    Ug, logg, _, _ = _newton_run(MODELS["10x10x10"], prec, forcing=True, its=3)
+    for a, b in zip(U, Ug):
+        assert np.array_equal(a, b)
+    for a, b in zip(log, logg):
+        assert _stat(a, "r_norm") == _stat(b, "r_norm")
+        assert _stat(a, "lin_iters") == _stat(b, "lin_iters")
