@@ -830,22 +830,22 @@ __device__ inline void load_tet(const KT* __restrict__ st, const double* __restr
   c.w = valid ? KT(1) : KT(0);
   c.tet = 1;
   c.hasM = HM;
-  // tet_plane's records: node a's (v_a, g_aa) and (c1, c2) in one vector load
-  // each; node b's record and the off-diagonal g_ab only when b != a
-  KT A[4], C2[2];
+  // tet_plane's records: node a's and node b's v and (c1, c2) in one vector load
+  // each, and g_ab.  On the diagonal b's record is a's, in the cache: read again,
+  // because a branch there would wait for a's first and so undo the NC
+  // contributions in flight.
+  KT A[4], B[4], C2[2];
   ld4(st, 4u * ((uint32_t)a * ne + e), A);
+  ld4(st, 4u * ((uint32_t)b * ne + e), B);
   ld2(st, 16u * ne + 2u * e, C2);
+  const uint32_t off = (18u + (uint32_t)((kOffPairTable >> (16 * a + 4 * b)) & 15u)) * ne + e;
+  c.g = ld32(st, a != b ? off : 4u * ((uint32_t)a * ne + e) + 3u);
   c.c1 = C2[0];
   c.c2 = C2[1];
 #pragma unroll
-  for (int i = 0; i < 3; ++i) c.va[i] = c.vb[i] = A[i];
-  c.g = A[3];
-  if (a != b) {
-    KT B[4];
-    ld4(st, 4u * ((uint32_t)b * ne + e), B);
-#pragma unroll
-    for (int i = 0; i < 3; ++i) c.vb[i] = B[i];
-    c.g = ld32(st, (18u + (uint32_t)((kOffPairTable >> (16 * a + 4 * b)) & 15u)) * ne + e);
+  for (int i = 0; i < 3; ++i) {
+    c.va[i] = A[i];
+    c.vb[i] = B[i];
   }
   const int p = (int)((kPairTable >> (16 * a + 4 * b)) & 15u);
   c.h = KT(0);
@@ -864,8 +864,10 @@ __device__ inline void load_tet(const KT* __restrict__ st, const double* __restr
 // k_gather for a model of one tet group: the same contributions added in the
 // same order, the group's state at a wave-uniform base with 32-bit offsets (no
 // per-lane group lookup or 64-bit address arithmetic), read as tet_plane's
-// vector records (3 to 4 loads per contribution instead of 9 scalar ones), NC
-// contributions per step.
+// vector records (4 loads per contribution instead of 9 scalar ones), NC
+// contributions per step.  Small models are bound by the chain group -> bounds and
+// entries -> column and states -> nodal forces and the steps after it, large ones by
+// the L2's reads (44 bytes a contribution, 16 contributions an element).
 template <typename KT, bool HM, int NC>
 __global__ __launch_bounds__(256) void k_gather_tet(
     const KT* __restrict__ st, const double* __restrict__ fe, uint32_t ne,
@@ -881,36 +883,38 @@ __global__ __launch_bounds__(256) void k_gather_tet(
   if (w >= ngroups) return;
   const SellGroup sg = groups[w];
   const int64_t r = sg.row0 + lane % kSellRows;
+  const int64_t rc = r < nn ? r : nn - 1;
   const int k = kSellLanes * sg.round + lane / kSellRows;
-  if (r >= nn) return;
-  const int32_t rs = row_ptr[r];
-  if (k >= row_ptr[r + 1] - rs) return;
+  int32_t rs = row_ptr[rc], re = row_ptr[rc + 1];
+  const uint32_t* cp = contrib + sg.cbase + lane;
+  const int qw = sg.qwidth;
+  int32_t nx[NC];
+#pragma unroll
+  for (int j = 0; j < NC; ++j) nx[j] = j < qw ? (int32_t)cp[64 * j] : (int32_t)kNoContrib;
+  arrive_all(nx);  // with the row's bounds, not after them
+  if (r >= nn || k >= re - rs) return;
   const int32_t cc = col[rs + k];
   const bool dg = (cc == r);
+  uint32_t mr = mask[r], mc = mask[cc];
   KT acc[9];
 #pragma unroll
   for (int q = 0; q < 9; ++q) acc[q] = KT(0);
   double f0 = 0, f1 = 0, f2 = 0;
-  const uint32_t* cp = contrib + sg.cbase + lane;
-  const int qw = sg.qwidth;
-  uint32_t nx[NC];
-#pragma unroll
-  for (int j = 0; j < NC; ++j) nx[j] = j < qw ? cp[64 * j] : kNoContrib;
   for (int q = 0; q < qw; q += NC) {
     uint32_t ex[NC];
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
-      ex[j] = nx[j];
-      nx[j] = q + NC + j < qw ? cp[64 * (int64_t)(q + NC + j)] : kNoContrib;
+      ex[j] = (uint32_t)nx[j];
+      nx[j] = q + NC + j < qw ? (int32_t)cp[64 * (int64_t)(q + NC + j)] : (int32_t)kNoContrib;
     }
     Contrib<KT, HM> cx[NC];
 #pragma unroll
     for (int j = 0; j < NC; ++j) load_tet(st, fe, ne, ex[j], dg, cx[j]);
 #pragma unroll
     for (int j = 0; j < NC; ++j) add_contrib(cx[j], acc, f0, f1, f2);
+    asm volatile("" : "+v"(mr), "+v"(mc));  // the masks come with the first states
   }
-  gather_finish(acc, mask[r], mask[cc], dg, Ks + 9 * (int64_t)sg.base + lane, Dinv, fint, r, f0, f1,
-                f2);
+  gather_finish(acc, mr, mc, dg, Ks + 9 * (int64_t)sg.base + lane, Dinv, fint, r, f0, f1, f2);
 }
 
 // ---- staged gather ---------------------------------------------------------------
@@ -1621,12 +1625,18 @@ int assemble_gather_t(Ctx* c) {
   const bool one_tet = ga.ng == 1 && g0.type == kTet &&
                        (uint64_t)kTetStateM * g0.ne * sizeof(KT) < (uint64_t(1) << 32) &&
                        (uint64_t)12 * g0.ne * sizeof(double) < (uint64_t(1) << 32);
-  // two contributions per step (on the 64^3 cube, gather pass in FP32 / FP64:
-  // 0.217 / 0.337 ms with 2, 0.227 / 0.378 ms with 4, 0.240 ms with 6 and
-  // 0.347 ms with 1; the general kernel 0.275 / 0.388 ms)
-  constexpr int kNC = 2;
+  // contributions per step: enough to hide the loads of small models, as many as the
+  // registers leave waves for in large ones.  Gather pass with 2 / 3 / 4 / 6: FP32
+  // 11.4 / 10.6 / 10.6 / 10.2 us at 4^3, 16.8 / 16.5 / 16.1 / 16.0 us at 24^3 and
+  // 218 / 214 / 212 / 210 us at 64^3, with the M term 14.0 / 13.6 / 13.7 / 13.6 us,
+  // 22.0 / 22.0 / 21.8 / 22.1 us and 331 / 325 / 323 / 323 us; FP64 12.8 / 12.1 / 11.9 /
+  // 11.5 us, 21.2 / 20.8 / 21.0 / 23.2 us and 338 / 336 / 341 / 364 us, with it
+  // 15.0 / 15.3 / 15.1 / 15.4 us, 28.4 / 29.7 / 32.6 / 40.2 us and 514 / 518 / 544 /
+  // 763 us.  With b's record read under a branch, the row's bounds, entries and masks
+  // one after the other and 2 per step: 13.9, 20.9 and 220 us in FP32.
+  constexpr int kNC = sizeof(KT) == 4 ? 4 : 3, kNCM = sizeof(KT) == 4 ? 4 : 2;
   if (one_tet && hm)
-    hipLaunchKernelGGL((k_gather_tet<KT, true, kNC>), dim3(gb), dim3(256), 0, s,
+    hipLaunchKernelGGL((k_gather_tet<KT, true, kNCM>), dim3(gb), dim3(256), 0, s,
                        (const KT*)g0.d_state, (const double*)g0.d_fe, (uint32_t)g0.ne,
                        c->d_sell_groups, ngrp, c->d_contrib, c->d_row_ptr, c->d_col, c->d_fixmask,
                        (KT*)c->d_Ksell, (KT*)c->d_Dinv, c->d_fint, c->nn);

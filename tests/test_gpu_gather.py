@@ -153,3 +153,38 @@ def test_staged_gather_on_compression_cube(prec):
         ref = res["lists"][k]
         np.testing.assert_allclose(res["staged"][k], ref, rtol=0,
                                    atol=K_TOL[prec] * np.abs(ref).max())
+
+
+def _tangent(prec, mat, coords, tets, fixed, mode):
+    with _env(ONSAS_ASSEMBLY=mode):
+        c = _capi.Context(PREC[prec])
+        try:
+            c.set_nodes(coords)
+            c.add_tet_group(tets, *MATS[mat])
+            c.set_fixed_dofs(fixed)
+            c.finalize()
+            c.set_U(1e-2 * np.random.default_rng(3).standard_normal(3 * len(coords)))
+            f = c.assemble(want_fint=True)
+            return f, c.tangent_bsr().tocsr()
+        finally:
+            c.close()
+
+
+@pytest.mark.parametrize("prec", ["mixed", "fp64"])
+@pytest.mark.parametrize("mat", ["svk", "nh"])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (3, 2, 1), (3, 3, 3), (5, 4, 3)])
+def test_lists_match_scatter_at_the_edges(prec, mat, shape):
+    """The list-driven gather where its steps end: lists of every length of small boxes (1
+    to 24 contributions, with remainders), 8 to 120 rows, a slice that is not full, a
+    node of no element."""
+    print(f"[gpu] gather edges {prec} {mat} {shape}", flush=True)
+    sm = meshes.cube(shape[0], ny=shape[1], nz=shape[2], jitter=0.1, seed=5)
+    coords = np.concatenate([sm.coords, [[3.0, 3.0, 3.0]]])
+    lone = 3 * (len(coords) - 1) + np.arange(3)
+    fixed = np.concatenate([(3 * sm.node_sets["x0"][:, None] + np.arange(3)).reshape(-1), lone])
+    f, K = _tangent(prec, mat, coords, sm.tets, fixed, "gather")
+    fs, Ks = _tangent(prec, mat, coords, sm.tets, fixed, "scatter")
+    # sums of up to 24 terms in another order, on terms up to 8 times the largest entry
+    eps = 2.0 ** -24 if prec == "mixed" else 2.0 ** -53
+    assert abs(K - Ks).max() <= 24 * 8 * eps * abs(Ks).max()
+    assert np.abs(f - fs).max() <= 24 * 8 * 2.0 ** -53 * np.abs(fs).max()
