@@ -316,12 +316,16 @@ int refined_solve(Ctx* c, const double* b, double* x, double* y, double* r, doub
 
 // f_int and K at the current U (the body of onsas_assemble).
 int assemble_now(Ctx* c) {
-  ONSAS_HIP_TRY(c, hipEventRecord(c->ev[0], c->stream));
-  ONSAS_HIP_TRY(c, hipMemcpyAsync(c->d_Uasm, c->d_U, 3 * c->nn * sizeof(double),
-                                  hipMemcpyDeviceToDevice, c->stream));
-  ONSAS_TRY(onsas::launch_assemble(c));
-  if (!c->gather) ONSAS_TRY(onsas::launch_pack_sell(c));
-  ONSAS_HIP_TRY(c, hipEventRecord(c->ev[3], c->stream));
+  if (c->gather) {  // keeps U and stamps its events itself
+    ONSAS_TRY(onsas::launch_assemble(c));
+  } else {
+    ONSAS_HIP_TRY(c, hipEventRecord(c->ev[0], c->stream));
+    ONSAS_HIP_TRY(c, hipMemcpyAsync(c->d_Uasm, c->d_U, 3 * c->nn * sizeof(double),
+                                    hipMemcpyDeviceToDevice, c->stream));
+    ONSAS_TRY(onsas::launch_assemble(c));
+    ONSAS_TRY(onsas::launch_pack_sell(c));
+    ONSAS_HIP_TRY(c, hipEventRecord(c->ev[3], c->stream));
+  }
   c->amg.stale = true;  // its Galerkin products belong to the previous tangent
   return ONSAS_OK;
 }
@@ -330,7 +334,7 @@ int assemble_now(Ctx* c) {
 void account_assembly(Ctx* c) {
   if (!c->asm_timing_pending) return;
   c->asm_timing_pending = false;
-  c->last_assemble_ms = elapsed(c->ev[0], c->ev[3]);
+  c->last_assemble_ms = c->gather ? elapsed(c->ev[1], c->ev[2]) : elapsed(c->ev[0], c->ev[3]);
   c->tm.assemble_ms += c->last_assemble_ms;
   c->tm.scatter_ms += elapsed(c->ev[1], c->ev[2]);
   if (c->gather) c->tm.elem_ms += elapsed(c->ev[1], c->ev[8]);
@@ -621,7 +625,6 @@ int onsas_newton_step(onsas_ctx* ctx, onsas_step_stats* out) {
   if (!c->assembled) return set_err(c, ONSAS_ERR_STATE, "onsas_assemble must precede onsas_newton_step");
   std::memset(out, 0, sizeof *out);
   hipStream_t s = c->stream;
-  ONSAS_HIP_TRY(c, hipEventRecord(c->ev[4], s));
   int iters = 0, conv = 0, solver = 0;
   double relres = 0;
   // warm start from the previous load step's update of this Newton iteration
@@ -642,6 +645,7 @@ int onsas_newton_step(onsas_ctx* ctx, onsas_step_stats* out) {
   }
   const bool whole = ran && !more;
   if (!whole) {
+    if (!ran) ONSAS_HIP_TRY(c, hipEventRecord(c->ev[4], s));
     ONSAS_TRY(onsas::launch_residual(c));
     ONSAS_HIP_TRY(c, hipEventRecord(c->ev[5], s));
     if (more)

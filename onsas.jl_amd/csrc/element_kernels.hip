@@ -23,6 +23,8 @@
 //            cI = S11 A / l, cdd = (E A / l0 - S11 A / l) / l^2, cf = A S11 / l
 //   Green:   eps = (l^2 - l0^2) / (2 l0^2),  S11 = E eps,
 //            cI = S11 A / l0, cdd = E A / l0^3, cf = A S11 / l0
+#include <hip/hip_ext.h>
+
 #include "engine.hpp"
 
 namespace onsas {
@@ -466,6 +468,14 @@ __device__ inline void tet_gradients_dev(const double X[12], double n[4][3], dou
     }
 }
 
+// The state pass of an assembly's first group also keeps the U it is taken at (a
+// copy of its own is a launch: 2.5 us and its gaps).
+__device__ inline void keep_U(const double* __restrict__ U, double* __restrict__ Uasm, int64_t n) {
+  if (!Uasm) return;
+  for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < n; q += (int64_t)gridDim.x * 256)
+    Uasm[q] = U[q];
+}
+
 // Element pass of the gather assembly: the tet's gradients are recomputed
 // from the nodal reference coordinates (read with U at the same nodes, mostly
 // from L2) instead of streaming the stored 104-byte geometry record.
@@ -475,8 +485,10 @@ __global__ __launch_bounds__(256) void k_tet_state(TetArgs ta, const double* __r
                                                    const double* __restrict__ Yr,
                                                    const double* __restrict__ Zr,
                                                    KT* __restrict__ st, double* __restrict__ fe,
-                                                   int hasM) {
+                                                   int hasM, double* __restrict__ Uasm,
+                                                   int64_t ndof) {
   const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  keep_U(U, Uasm, ndof);
   if (e >= ta.ne) return;
   const int64_t ne = ta.ne;
   int32_t nd[4];
@@ -548,8 +560,10 @@ __global__ __launch_bounds__(256) void k_tet_state(TetArgs ta, const double* __r
 
 template <typename KT>
 __global__ __launch_bounds__(256) void k_truss_state(TrussArgs ta, const double* __restrict__ U,
-                                                     KT* __restrict__ st, double* __restrict__ fe) {
+                                                     KT* __restrict__ st, double* __restrict__ fe,
+                                                     double* __restrict__ Uasm, int64_t ndof) {
   const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  keep_U(U, Uasm, ndof);
   if (e >= ta.ne) return;
   const int64_t ne = ta.ne;
   const int32_t nd0 = ta.conn[e], nd1 = ta.conn[ne + e];
@@ -1565,7 +1579,7 @@ int stage_run(Ctx* c, bool set_attr) {
   const unsigned gb = (unsigned)((c->nstage_groups + 7) / 8 * 8);  // a multiple of 8 (XCD mapping)
   int rlog2 = 0;
   while ((1 << rlog2) < c->stage_rows) ++rlog2;
-  hipLaunchKernelGGL(kern, dim3(gb), dim3(kStageThreads), lds, c->stream, (const KT*)g.d_state,
+  hipExtLaunchKernelGGL(kern, dim3(gb), dim3(kStageThreads), lds, c->stream, nullptr, c->ev[2], 0, (const KT*)g.d_state,
                      g.d_fe, g.ne, c->d_stage_groups, c->nstage_groups, c->d_stage,
                      c->d_stage_steps, c->d_stage_words, c->d_stage_pairs, c->d_pair_row, rlog2,
                      c->stage_cap, c->stage_pairs_cap, c->stage_steps_cap, c->d_row_ptr,
@@ -1592,28 +1606,30 @@ int stage_dispatch(Ctx* c, bool set_attr) {
                            : stage_dispatch_ks<KT, kTetStateBase>(c, set_attr);
 }
 
+// The passes stamp the timing events themselves (an event recorded between two
+// launches is a packet of its own that the next one waits for: with the copy of U,
+// five of them were 25 us of a 4^3 box's 150 us Newton step).
 template <typename KT>
 int assemble_gather_t(Ctx* c) {
   hipStream_t s = c->stream;
-  ONSAS_HIP_TRY(c, hipEventRecord(c->ev[1], s));
   GatherArgs ga{};
   ga.ng = (int)c->groups.size();
   for (int gi = 0; gi < ga.ng; ++gi) {
     const ElemGroup& g = c->groups[gi];
+    const hipEvent_t e0 = gi == 0 ? c->ev[1] : nullptr, e1 = gi == ga.ng - 1 ? c->ev[8] : nullptr;
+    double* Uasm = gi == 0 ? c->d_Uasm : nullptr;
     if (g.type == kTet)
-      hipLaunchKernelGGL(k_tet_state<KT>, dim3(grid_for(g.ne, 256)), dim3(256), 0, s,
-                         tet_args(g, 0, g.ne), c->d_U, c->d_x, c->d_y, c->d_z, (KT*)g.d_state,
-                         g.d_fe, (int)g.hasM);
+      hipExtLaunchKernelGGL(k_tet_state<KT>, dim3(grid_for(g.ne, 256)), dim3(256), 0, s, e0, e1, 0,
+                            tet_args(g, 0, g.ne), c->d_U, c->d_x, c->d_y, c->d_z, (KT*)g.d_state,
+                            g.d_fe, (int)g.hasM, Uasm, 3 * c->nn);
     else
-      hipLaunchKernelGGL(k_truss_state<KT>, dim3(grid_for(g.ne, 256)), dim3(256), 0, s,
-                         truss_args(g, 0, g.ne), c->d_U, (KT*)g.d_state, g.d_fe);
+      hipExtLaunchKernelGGL(k_truss_state<KT>, dim3(grid_for(g.ne, 256)), dim3(256), 0, s, e0, e1, 0,
+                            truss_args(g, 0, g.ne), c->d_U, (KT*)g.d_state, g.d_fe, Uasm, 3 * c->nn);
     ga.g[gi] = GatherGroup{g.d_state, g.d_fe, g.ne, g.goff, g.type, (int)g.hasM};
   }
   ONSAS_HIP_TRY(c, hipGetLastError());
-  ONSAS_HIP_TRY(c, hipEventRecord(c->ev[8], s));
   if (c->stage_rows > 0) {
     ONSAS_TRY(stage_dispatch<KT>(c, false));
-    ONSAS_HIP_TRY(c, hipEventRecord(c->ev[2], s));
     c->bsr_stale = true;
     return ONSAS_OK;
   }
@@ -1636,25 +1652,24 @@ int assemble_gather_t(Ctx* c) {
   // one after the other and 2 per step: 13.9, 20.9 and 220 us in FP32.
   constexpr int kNC = sizeof(KT) == 4 ? 4 : 3, kNCM = sizeof(KT) == 4 ? 4 : 2;
   if (one_tet && hm)
-    hipLaunchKernelGGL((k_gather_tet<KT, true, kNCM>), dim3(gb), dim3(256), 0, s,
+    hipExtLaunchKernelGGL((k_gather_tet<KT, true, kNCM>), dim3(gb), dim3(256), 0, s, nullptr, c->ev[2], 0,
                        (const KT*)g0.d_state, (const double*)g0.d_fe, (uint32_t)g0.ne,
                        c->d_sell_groups, ngrp, c->d_contrib, c->d_row_ptr, c->d_col, c->d_fixmask,
                        (KT*)c->d_Ksell, (KT*)c->d_Dinv, c->d_fint, c->nn);
   else if (one_tet)
-    hipLaunchKernelGGL((k_gather_tet<KT, false, kNC>), dim3(gb), dim3(256), 0, s,
+    hipExtLaunchKernelGGL((k_gather_tet<KT, false, kNC>), dim3(gb), dim3(256), 0, s, nullptr, c->ev[2], 0,
                        (const KT*)g0.d_state, (const double*)g0.d_fe, (uint32_t)g0.ne,
                        c->d_sell_groups, ngrp, c->d_contrib, c->d_row_ptr, c->d_col, c->d_fixmask,
                        (KT*)c->d_Ksell, (KT*)c->d_Dinv, c->d_fint, c->nn);
   else if (hm)
-    hipLaunchKernelGGL((k_gather<KT, true>), dim3(gb), dim3(256), 0, s, ga, c->d_sell_groups,
+    hipExtLaunchKernelGGL((k_gather<KT, true>), dim3(gb), dim3(256), 0, s, nullptr, c->ev[2], 0, ga, c->d_sell_groups,
                        ngrp, c->d_contrib, c->d_row_ptr, c->d_col, c->d_fixmask, (KT*)c->d_Ksell,
                        (KT*)c->d_Dinv, c->d_fint, c->nn);
   else
-    hipLaunchKernelGGL((k_gather<KT, false>), dim3(gb), dim3(256), 0, s, ga, c->d_sell_groups,
+    hipExtLaunchKernelGGL((k_gather<KT, false>), dim3(gb), dim3(256), 0, s, nullptr, c->ev[2], 0, ga, c->d_sell_groups,
                        ngrp, c->d_contrib, c->d_row_ptr, c->d_col, c->d_fixmask, (KT*)c->d_Ksell,
                        (KT*)c->d_Dinv, c->d_fint, c->nn);
   ONSAS_HIP_TRY(c, hipGetLastError());
-  ONSAS_HIP_TRY(c, hipEventRecord(c->ev[2], s));
   c->bsr_stale = true;
   return ONSAS_OK;
 }

@@ -23,6 +23,8 @@
 #include <cmath>
 #include <cstdlib>
 
+#include <hip/hip_ext.h>
+
 #include "engine.hpp"
 #include "grid_exchange.hpp"
 
@@ -675,22 +677,22 @@ inline ResidentShape resident_shape(const Ctx* c) {
   return {t, (lanes + t - 1) / t};
 }
 
+// A Newton step's launch stamps the step's timing events.
 template <typename KT, int L>
 void run_resident(Ctx* c, const ResidentArgs<KT>& a, const ResidentShape& sh) {
   constexpr int T1 = resident_one_threads(sizeof(KT)), T = kResidentThreads;
-  const dim3 grid((unsigned)sh.grid);
+  const hipEvent_t e0 = a.fint ? c->ev[4] : nullptr, e1 = a.fint ? c->ev[7] : nullptr;
+  auto go = [&](auto kern, int threads) {
+    hipExtLaunchKernelGGL(kern, dim3((unsigned)sh.grid), dim3(threads), 0, c->stream, e0, e1, 0, a);
+  };
   if (sh.grid == 1 && sh.threads == 512)
-    hipLaunchKernelGGL((k_pcg_resident<KT, L, kResidentBlocks, 512, true>), grid, dim3(512), 0,
-                       c->stream, a);
+    go(k_pcg_resident<KT, L, kResidentBlocks, 512, true>, 512);
   else if (sh.grid == 1)
-    hipLaunchKernelGGL((k_pcg_resident<KT, L, kResidentBlocks, T1, true>), grid, dim3(T1), 0,
-                       c->stream, a);
+    go(k_pcg_resident<KT, L, kResidentBlocks, T1, true>, T1);
   else if (sh.threads == T)
-    hipLaunchKernelGGL((k_pcg_resident<KT, L, kResidentBlocks, T, false>), grid, dim3(T), 0,
-                       c->stream, a);
+    go(k_pcg_resident<KT, L, kResidentBlocks, T, false>, T);
   else
-    hipLaunchKernelGGL((k_pcg_resident<KT, L, kResidentBlocks, 2 * T, false>), grid, dim3(2 * T), 0,
-                       c->stream, a);
+    go(k_pcg_resident<KT, L, kResidentBlocks, 2 * T, false>, 2 * T);
 }
 
 template <typename KT>
@@ -800,7 +802,6 @@ static int resident_run(Ctx* c, const double* b, const double* fint, const void*
   c->h_sc->pcg = PcgState{};
   ONSAS_TRY(c->precision == ONSAS_PRECISION_FP64 ? resident_t<double>(c, b, fint, x0, warm)
                                                  : resident_t<float>(c, b, fint, x0, warm));
-  if (fint) ONSAS_HIP_TRY(c, hipEventRecord(c->ev[7], s));
   ONSAS_HIP_TRY(c, hipStreamSynchronize(s));
   const PcgState& ps = c->h_sc->pcg;
   *ran = ps.done && !ps.aborted;
