@@ -373,90 +373,115 @@ __global__ void k_dense_scatter(const int32_t* __restrict__ row_ptr, const int32
   if (drow[t] == 0) drow[t] = 1;
 }
 
-// Blocked Gauss-Jordan inverse of the dense SPD coarsest matrix M (n x n, FP64,
-// in place; SPD: the pivots are the diagonal).  Per pivot block [k0, k0 + kb):
-// A11 <- A11^-1 (k_gj_diag), C <- A21 and A12 <- A11^-1 A12 (k_gj_rows),
-// then A22 <- A22 - C A12 and A21 <- -C A11^-1 (k_gj_update).
+// Blocked Gauss-Jordan inverse of the dense SPD coarsest matrix (n x n, FP64; SPD:
+// the pivots are the diagonal), one launch per pivot block P = [k0, k0 + kb) from
+// one buffer into another, which is A22, A21 and A12 of the step before without an
+// order between workgroups:
+//   rows of P: W;  other rows i: (j in P ? 0 : M[i][j]) - sum_b M[i][P_b] W[b][j],
+//   W = A11^-1 [A12 | I].
+// A workgroup has a 64 x 64 tile and makes A11^-1 and its columns of W for itself:
+// the step is bound by the 32 pivots' chain (LDS round trip, barrier, division),
+// which every workgroup runs at once, and not by the arithmetic.  A thread keeps
+// four entries of the pivot block and only the next pivot's row and column go
+// through LDS.  At n = 576: 18 us a step; with the pivot block inverted in LDS by
+// one workgroup (40 us), the rows (33 us, a chain of 32 x 32 loads a thread) and the
+// update (13 us) as launches of their own, 87 us.
 constexpr int kGJ = 32;  // pivot block
 
-__global__ __launch_bounds__(256) void k_gj_diag(double* __restrict__ M, int64_t n, int64_t k0, int kb) {
-  __shared__ double S[kGJ][kGJ + 1];
-  __shared__ double colk[kGJ];
-  for (int t = threadIdx.x; t < kb * kb; t += blockDim.x) S[t / kb][t % kb] = M[(k0 + t / kb) * n + k0 + t % kb];
-  __syncthreads();
-  for (int k = 0; k < kb; ++k) {
-    if ((int)threadIdx.x < kb) colk[threadIdx.x] = S[threadIdx.x][k];
-    __syncthreads();
-    const double piv = 1.0 / colk[k];
-    if ((int)threadIdx.x < kb) S[k][threadIdx.x] = ((int)threadIdx.x == k) ? piv : S[k][threadIdx.x] * piv;
-    __syncthreads();
-    for (int t = threadIdx.x; t < kb * kb; t += blockDim.x) {
-      const int r = t / kb, c = t % kb;
-      if (r == k) continue;
-      S[r][c] = (c == k) ? -colk[r] * piv : S[r][c] - colk[r] * S[k][c];
-    }
-    __syncthreads();
-  }
-  for (int t = threadIdx.x; t < kb * kb; t += blockDim.x) M[(k0 + t / kb) * n + k0 + t % kb] = S[t / kb][t % kb];
-}
-
-// Threads [0, n kGJ): C[i][b] = M[i][k0 + b] for rows i outside the block; then
-// one thread per column j outside the block: M[k0 + r][j] = (A11^-1 A12)[r][j].
-__global__ __launch_bounds__(256) void k_gj_rows(double* __restrict__ M, double* __restrict__ C, int64_t n,
-                                                 int64_t k0, int kb) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t nA = n * kGJ;
-  if (t < nA) {
-    const int64_t i = t / kGJ;
-    const int b = (int)(t % kGJ);
-    if (b < kb && (i < k0 || i >= k0 + kb)) C[t] = M[i * n + k0 + b];
-    return;
-  }
-  const int64_t j = t - nA;
-  if (j >= n || (j >= k0 && j < k0 + kb)) return;
-  // every address below stays inside the block (b, r < kb; clamped otherwise)
-  double a[kGJ];
-#pragma unroll
-  for (int b = 0; b < kGJ; ++b) {
-    const int bb = b < kb ? b : 0;
-    a[b] = b < kb ? M[(k0 + bb) * n + j] : 0.0;
-  }
-#pragma unroll
-  for (int r = 0; r < kGJ; ++r) {
-    if (r >= kb) break;
-    const double* ai = M + (k0 + r) * n + k0;  // row r of A11^-1
-    double s = 0;
-#pragma unroll
-    for (int b = 0; b < kGJ; ++b) {
-      const int bb = b < kb ? b : 0;
-      s += (b < kb ? ai[bb] : 0.0) * a[b];
-    }
-    M[(k0 + r) * n + j] = s;
-  }
-}
-
-// Rows i outside the block: M[i][j] = (j in the block ? 0 : M[i][j]) -
-// sum_b C[i][b] M[k0 + b][j]; 64 x 64 output tiles, 4 x 4 per thread, C and the
-// block rows staged in LDS.
-__global__ __launch_bounds__(256) void k_gj_update(double* __restrict__ M, const double* __restrict__ C,
-                                                   int64_t n, int64_t k0, int kb) {
-  __shared__ double Cs[64][kGJ + 1];
-  __shared__ double Ms[kGJ][64 + 1];
+__global__ __launch_bounds__(256) void k_gj_step(const double* __restrict__ M,
+                                                 double* __restrict__ out, int64_t n, int64_t k0,
+                                                 int kb) {
+  __shared__ double prow[2][kGJ], pcol[2][kGJ];
+  __shared__ double Ai[kGJ][kGJ + 1];  // A11^-1
+  __shared__ double Cs[64][kGJ + 1];   // the tile's rows of A21 (zero in P)
+  __shared__ double Ws[kGJ][64 + 2];   // the tile's columns of [A12 | I], then of W
+  const int t = threadIdx.x;
   const int64_t i0 = (int64_t)blockIdx.y * 64, j0 = (int64_t)blockIdx.x * 64;
-  for (int t = threadIdx.x; t < 64 * kGJ; t += 256) {  // clamped addresses, masked values
-    const int r = t / kGJ, b = t % kGJ;
-    const int64_t i = i0 + r;
-    const bool ok = i < n && b < kb && (i < k0 || i >= k0 + kb);
-    Cs[r][b] = ok ? C[(ok ? i : 0) * kGJ + b] : 0.0;
+  const int pr = t >> 3, pc = 4 * (t & 7);
+  double e[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const bool ok = pr < kb && pc + q < kb;  // past kb: the identity
+    const double m = M[(k0 + (ok ? pr : 0)) * n + k0 + (ok ? pc + q : 0)];
+    e[q] = ok ? m : (pr == pc + q ? 1.0 : 0.0);
   }
-  for (int t = threadIdx.x; t < kGJ * 64; t += 256) {
-    const int b = t / 64, cc = t % 64;
+  // the rest of the tile's operands arrive while the pivots run
+  const int ty = t >> 4, tx = t & 15;
+  double m[4][4], cv[8], wv[8];
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const int64_t i = i0 + 4 * ty + q, j = j0 + tx + 16 * p;
+      const bool ok = i < n && j < n;
+      m[q][p] = M[ok ? i * n + j : 0];
+      if (j >= k0 && j < k0 + kb) m[q][p] = 0.0;
+    }
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const int r = (t >> 5) + 8 * q, bb = t & 31;  // A21: 64 x 32
+    const int64_t i = i0 + r;
+    const bool ok = i < n && bb < kb && (i < k0 || i >= k0 + kb);
+    const double x = M[ok ? i * n + k0 + bb : 0];
+    cv[q] = ok ? x : 0.0;
+    const int b = (t >> 6) + 4 * q, cc = t & 63;  // [A12 | I]: 32 x 64
     const int64_t j = j0 + cc;
-    const bool ok = b < kb && j < n;
-    Ms[b][cc] = ok ? M[(k0 + (ok ? b : 0)) * n + (ok ? j : 0)] : 0.0;
+    const bool inb = j >= k0 && j < k0 + kb, okw = b < kb && j < n;
+    const double y = M[okw ? (k0 + b) * n + j : 0];
+    wv[q] = inb ? (j - k0 == b ? 1.0 : 0.0) : (okw ? y : 0.0);
+  }
+  auto publish = [&](int k) {
+    if (pr == k)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) prow[k & 1][pc + q] = e[q];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (pc + q == k) pcol[k & 1][pr] = e[q];
+  };
+  publish(0);
+  for (int k = 0; k < kGJ; ++k) {
+    __syncthreads();
+    const double piv = 1.0 / prow[k & 1][k], c = pcol[k & 1][pr];
+    double row[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) row[q] = prow[k & 1][pc + q];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const bool diag = pc + q == k;
+      const double s = diag ? piv : row[q] * piv;
+      e[q] = pr == k ? s : (diag ? -c * piv : e[q] - c * s);
+    }
+    if (k + 1 < kGJ) publish(k + 1);
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) Ai[pr][pc + q] = e[q];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    Cs[(t >> 5) + 8 * q][t & 31] = cv[q];
+    Ws[(t >> 6) + 4 * q][t & 63] = wv[q];
   }
   __syncthreads();
-  const int ty = threadIdx.x / 16, tx = threadIdx.x % 16;
+  {  // W: four rows and two columns a thread
+    const int r0 = 4 * (t >> 5), c0 = 2 * (t & 31);
+    double w[4][2] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
+#pragma unroll 8
+    for (int b = 0; b < kGJ; ++b) {
+      const double x0 = Ws[b][c0], x1 = Ws[b][c0 + 1];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const double av = Ai[r0 + q][b];
+        w[q][0] += av * x0;
+        w[q][1] += av * x1;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      Ws[r0 + q][c0] = w[q][0];
+      Ws[r0 + q][c0 + 1] = w[q][1];
+    }
+    __syncthreads();
+  }
   double acc[4][4];
 #pragma unroll
   for (int q = 0; q < 4; ++q)
@@ -464,27 +489,27 @@ __global__ __launch_bounds__(256) void k_gj_update(double* __restrict__ M, const
     for (int p = 0; p < 4; ++p) acc[q][p] = 0;
 #pragma unroll 8
   for (int b = 0; b < kGJ; ++b) {
-    double cv[4], mv[4];
+    double c4[4], w4[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      cv[q] = Cs[4 * ty + q][b];
-      mv[q] = Ms[b][4 * tx + q];
+      c4[q] = Cs[4 * ty + q][b];
+      w4[q] = Ws[b][tx + 16 * q];
     }
 #pragma unroll
     for (int q = 0; q < 4; ++q)
 #pragma unroll
-      for (int p = 0; p < 4; ++p) acc[q][p] += cv[q] * mv[p];
+      for (int p = 0; p < 4; ++p) acc[q][p] += c4[q] * w4[p];
   }
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     const int64_t i = i0 + 4 * ty + q;
-    if (i >= n || (i >= k0 && i < k0 + kb)) continue;
+    if (i >= n) continue;
+    const bool inp = i >= k0 && i < k0 + kb;
+    const int b = inp ? (int)(i - k0) : 0;
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
-      const int64_t j = j0 + 4 * tx + p;
-      if (j >= n) continue;
-      const bool inb = j >= k0 && j < k0 + kb;
-      M[i * n + j] = (inb ? 0.0 : M[i * n + j]) - acc[q][p];
+      const int64_t j = j0 + tx + 16 * p;
+      if (j < n) out[i * n + j] = inp ? Ws[b][tx + 16 * p] : m[q][p] - acc[q][p];
     }
   }
 }
@@ -1502,7 +1527,7 @@ int amg_build(Ctx* c) {
     ONSAS_TRY(alloc(c, v, c->kt * 3 * (size_t)nn));
   A.nc = 6 * (int)A.lev.back().n;
   ONSAS_TRY(alloc(c, (void**)&A.d_dense, sizeof(double) * (size_t)A.nc * A.nc));
-  ONSAS_TRY(alloc(c, (void**)&A.d_gjc, sizeof(double) * (size_t)A.nc * kGJ));
+  ONSAS_TRY(alloc(c, (void**)&A.d_dense2, sizeof(double) * (size_t)A.nc * A.nc));
   A.ldc = (A.nc + 3) & ~3;
   ONSAS_TRY(alloc(c, &A.d_Ainv, c->kt * (size_t)A.nc * A.ldc));
   ONSAS_TRY(alloc(c, (void**)&A.d_part, sizeof(double) * 1024));
@@ -1697,16 +1722,14 @@ int amg_numeric_t(Ctx* c) {
   hipLaunchKernelGGL(k_zero_f64, dim3(256), dim3(256), 0, s, A.d_dense, nc * nc);
   hipLaunchKernelGGL(k_dense_scatter<KT>, dim3(nblocks(nc, 128)), dim3(128), 0, s, Lc.d_row_ptr,
                      Lc.d_col, (const KT*)Lc.d_A, A.d_dense, Lc.n);
+  double *from = A.d_dense, *to = A.d_dense2;
   for (int64_t k0 = 0; k0 < nc; k0 += kGJ) {
-    const int kb = (int)std::min<int64_t>(kGJ, nc - k0);
-    hipLaunchKernelGGL(k_gj_diag, dim3(1), dim3(256), 0, s, A.d_dense, nc, k0, kb);
-    hipLaunchKernelGGL(k_gj_rows, dim3(nblocks(nc * kGJ + nc, 256)), dim3(256), 0, s, A.d_dense,
-                       A.d_gjc, nc, k0, kb);
-    hipLaunchKernelGGL(k_gj_update, dim3(nblocks(nc, 64), nblocks(nc, 64)), dim3(256), 0, s,
-                       A.d_dense, (const double*)A.d_gjc, nc, k0, kb);
+    hipLaunchKernelGGL(k_gj_step, dim3(nblocks(nc, 64), nblocks(nc, 64)), dim3(256), 0, s,
+                       (const double*)from, to, nc, k0, (int)std::min<int64_t>(kGJ, nc - k0));
+    std::swap(from, to);
   }
   hipLaunchKernelGGL(k_to_kt<KT>, dim3(nblocks((int64_t)A.nc * A.ldc, 256)), dim3(256), 0, s,
-                     A.d_dense, (KT*)A.d_Ainv, (int64_t)A.nc, (int64_t)A.ldc);
+                     (const double*)from, (KT*)A.d_Ainv, (int64_t)A.nc, (int64_t)A.ldc);
   ONSAS_HIP_TRY(c, hipGetLastError());
   A.lam_set = true;
   A.stale = false;
@@ -2005,7 +2028,7 @@ void amg_free(Ctx* c) {
                     (void*)L.d_s6_ptr, (void*)L.d_s6_col, (void*)L.d_s6_src,
                     (void*)L.d_s6_row, (void*)L.d_s6_win, L.d_A6s})
       if (p) (void)hipFree(p);
-  for (void* p : {(void*)A.d_dense, (void*)A.d_gjc, A.d_Ainv, (void*)A.d_part,
+  for (void* p : {(void*)A.d_dense, (void*)A.d_dense2, A.d_Ainv, (void*)A.d_part,
                   (void*)A.d_rzs})
     if (p) (void)hipFree(p);
   A = Amg{};

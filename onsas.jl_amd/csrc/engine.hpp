@@ -177,8 +177,8 @@ struct Amg {
   int coarse_degree = 2;   // and of the coarser levels'
   std::vector<AmgLevel> lev;
   int nc = 0;                         // dofs of the coarsest level (dense inverse)
-  double* d_dense = nullptr;          // nc x nc FP64 work (the inverse in place)
-  double* d_gjc = nullptr;            // nc x 32 FP64: a pivot block's column
+  double* d_dense = nullptr;          // nc x nc FP64 work of the inverse, taken in turn
+  double* d_dense2 = nullptr;
   int ldc = 0;                        // row length of d_Ainv (nc rounded up to 4)
   void* d_Ainv = nullptr;             // nc x ldc KT, zero padded
   double* d_part = nullptr;           // power-iteration partial sums
