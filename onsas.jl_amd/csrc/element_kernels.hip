@@ -1266,6 +1266,160 @@ __global__ __launch_bounds__(kScatterThreads) void k_truss_apply(TrussArgs ta,
   for (int i = 0; i < 3; ++i) yp[i] += ((ma >> i) & 1u) ? 0.0 : sa * (tv.cI * w[i] + tv.cdd * tv.d[i] * dw);
 }
 
+// The same product of a model with gather lists, in two passes like its assembly:
+// an element's 12 (truss: 3) product values to its planes of nodal forces, which
+// are free between assemblies, then each row's incidences added in the order of
+// the assembly (the list of its diagonal block).  With w_b the masked nodal values,
+// sum_b K_ab w_b = V [c1 (sum_b v_b.w_b) v_a + c2 G v_a + c2 M H' .. + (S N)' n_a],
+// G = sum_b v_b w_b', N = sum_b n_b w_b' (H' = G' v_a, or N' n_a without v): 9 + 9
+// sums an element instead of 16 blocks.  Bound by latency at these sizes: 83 k
+// elements (24^3) take 9 + 30 + 5 us in three launches, against 33 coloured launches
+// of 11.8 us, four lanes an element each with the whole evaluation.
+__global__ __launch_bounds__(256) void k_tet_product(TetArgs ta, const double* __restrict__ U,
+                                                     const double* __restrict__ v,
+                                                     double* __restrict__ fe,
+                                                     const uint8_t* __restrict__ mask) {
+  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= ta.ne) return;
+  int32_t nd[4];
+  double n[4][3], u[4][3], w[4][3], V, p1;
+  tet_load(ta, e, U, nd, n, V, u, p1);
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    const uint32_t mb = mask[nd[b]];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const double x = v[3 * (int64_t)nd[b] + j];
+      w[b][j] = ((mb >> j) & 1u) ? 0.0 : x;
+    }
+  }
+  TetEval ev;
+  tet_eval(ta.mat, ta.p0, p1, n, u, ev);
+  double G[9], N[9], tr = 0;
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      double g = 0, h = 0;
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        g += ev.v[b][i] * w[b][j];
+        h += n[b][i] * w[b][j];
+      }
+      G[i * 3 + j] = g;
+      N[i * 3 + j] = h;
+      if (i == j) tr += g;
+    }
+  double SN[9];  // S N, or zero
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+      SN[i * 3 + j] =
+          ev.geo ? ev.S[i * 3] * N[j] + ev.S[i * 3 + 1] * N[3 + j] + ev.S[i * 3 + 2] * N[6 + j] : 0.0;
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    double h[3], o[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+      h[j] = ev.sv ? G[j] * ev.v[a][0] + G[3 + j] * ev.v[a][1] + G[6 + j] * ev.v[a][2]
+                   : N[j] * n[a][0] + N[3 + j] * n[a][1] + N[6 + j] * n[a][2];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const double gv = G[i * 3] * ev.v[a][0] + G[i * 3 + 1] * ev.v[a][1] + G[i * 3 + 2] * ev.v[a][2];
+      const double mh = ev.M[i * 3] * h[0] + ev.M[i * 3 + 1] * h[1] + ev.M[i * 3 + 2] * h[2];
+      const double sn = SN[i] * n[a][0] + SN[3 + i] * n[a][1] + SN[6 + i] * n[a][2];
+      o[i] = V * (ev.c1 * tr * ev.v[a][i] + ev.c2 * gv + ev.c2 * mh + sn);
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) fe[(3 * a + i) * ta.ne + e] = o[i];
+  }
+}
+
+__global__ __launch_bounds__(256) void k_truss_product(TrussArgs ta, const double* __restrict__ U,
+                                                       const double* __restrict__ v,
+                                                       double* __restrict__ fe,
+                                                       const uint8_t* __restrict__ mask) {
+  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= ta.ne) return;
+  const int64_t ne = ta.ne;
+  const int32_t nd0 = ta.conn[e], nd1 = ta.conn[ne + e];
+  double d0[3] = {ta.geo[e], ta.geo[ne + e], ta.geo[2 * ne + e]};
+  const double l0 = ta.geo[3 * ne + e], A = ta.geo[4 * ne + e];
+  const uint32_t m0 = mask[nd0], m1 = mask[nd1];
+  double du[3], w[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    du[d] = U[3 * (int64_t)nd1 + d] - U[3 * (int64_t)nd0 + d];
+    w[d] = (((m1 >> d) & 1u) ? 0.0 : v[3 * (int64_t)nd1 + d]) -
+           (((m0 >> d) & 1u) ? 0.0 : v[3 * (int64_t)nd0 + d]);
+  }
+  TrussEval tv;
+  truss_eval(ta.strain, ta.E, A, d0, l0, du, tv);
+  const double dw = tv.d[0] * w[0] + tv.d[1] * w[1] + tv.d[2] * w[2];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) fe[i * ne + e] = tv.cI * w[i] + tv.cdd * tv.d[i] * dw;
+}
+
+// y = the sums of the rows' incidences on the free dofs (one wave per sliced-ELL
+// group, the lanes of diagonal blocks, as k_gather sums f_int).
+__global__ __launch_bounds__(256) void k_product_rows(GatherArgs ga,
+                                                      const SellGroup* __restrict__ groups,
+                                                      int64_t ngroups,
+                                                      const uint32_t* __restrict__ contrib,
+                                                      const int32_t* __restrict__ row_ptr,
+                                                      const int32_t* __restrict__ diag,
+                                                      const uint8_t* __restrict__ mask,
+                                                      double* __restrict__ y, int64_t nn) {
+  const int64_t g = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (g >= ngroups) return;
+  const SellGroup sg = groups[g];
+  const int64_t r = sg.row0 + lane % kSellRows;
+  const int k = kSellLanes * sg.round + lane / kSellRows;
+  if (r >= nn || diag[r] - row_ptr[r] != k) return;
+  double f[3] = {0, 0, 0};
+  const uint32_t* cp = contrib + sg.cbase + lane;
+  constexpr int NC = 4;
+  for (int q = 0; q < sg.qwidth; q += NC) {
+    uint32_t en[NC];
+    double x[NC][3];
+#pragma unroll
+    for (int j = 0; j < NC; ++j)
+      en[j] = q + j < sg.qwidth ? cp[64 * (int64_t)(q + j)] : kNoContrib;
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      const bool valid = en[j] != kNoContrib;
+      const int64_t ge = valid ? en[j] >> 4 : 0;
+      const int a = valid ? (int)((en[j] >> 2) & 3u) : 0;
+      const double* fp = ga.g[0].fe;
+      int64_t ne = ga.g[0].ne, goff = ga.g[0].goff;
+      int type = ga.g[0].type;
+#pragma unroll
+      for (int i = 1; i < kMaxGatherGroups; ++i)
+        if (i < ga.ng && ge >= ga.g[i].goff) {
+          fp = ga.g[i].fe;
+          ne = ga.g[i].ne;
+          goff = ga.g[i].goff;
+          type = ga.g[i].type;
+        }
+      const bool tet = type == kTet;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        const double p = fp[((tet ? 3 * a : 0) + d) * ne + ge - goff];
+        x[j][d] = valid ? (tet || a ? p : -p) : 0.0;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NC; ++j)
+#pragma unroll
+      for (int d = 0; d < 3; ++d) f[d] += x[j][d];
+  }
+  const uint32_t m = mask[r];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) y[3 * r + d] = ((m >> d) & 1u) ? 0.0 : f[d];
+}
+
 // y[fixed] = v[fixed] (the identity rows of the assembled operator).
 __global__ void k_fixed_copy(const double* __restrict__ v, double* __restrict__ y,
                              const uint8_t* __restrict__ mask, int64_t nn) {
@@ -1702,22 +1856,43 @@ int launch_gather_init(Ctx* c) {
   return ONSAS_OK;
 }
 
+// The rows without an element are fixed, so k_fixed_copy completes either path.
+// The coloured launches are left for the assemblies without gather lists.
 int launch_tangent_apply_f64(Ctx* c, const double* v, double* y) {
   hipStream_t s = c->stream;
-  hipLaunchKernelGGL(k_fill<double>, dim3(512), dim3(256), 0, s, y, 3 * c->nn, 0.0);
-  for (const ElemGroup& g : c->groups) {
-    const int ncol = (int)g.color_off.size() - 1;
-    for (int k = 0; k < ncol; ++k) {
-      const int64_t e0 = g.color_off[k], e1 = g.color_off[k + 1];
-      if (e1 <= e0) continue;
+  if (c->gather && c->stage_rows == 0) {
+    GatherArgs ga{};
+    ga.ng = (int)c->groups.size();
+    for (int gi = 0; gi < ga.ng; ++gi) {
+      const ElemGroup& g = c->groups[gi];
       if (g.type == kTet)
-        hipLaunchKernelGGL(k_tet_apply, dim3(grid_for(4 * (e1 - e0), kScatterThreads)),
-                           dim3(kScatterThreads), 0, s, tet_args(g, e0, e1), c->d_U, v, y,
-                           c->d_fixmask);
+        hipLaunchKernelGGL(k_tet_product, dim3(grid_for(g.ne, 256)), dim3(256), 0, s,
+                           tet_args(g, 0, g.ne), c->d_U, v, g.d_fe, c->d_fixmask);
       else
-        hipLaunchKernelGGL(k_truss_apply, dim3(grid_for(2 * (e1 - e0), kScatterThreads)),
-                           dim3(kScatterThreads), 0, s, truss_args(g, e0, e1), c->d_U, v, y,
-                           c->d_fixmask);
+        hipLaunchKernelGGL(k_truss_product, dim3(grid_for(g.ne, 256)), dim3(256), 0, s,
+                           truss_args(g, 0, g.ne), c->d_U, v, g.d_fe, c->d_fixmask);
+      ga.g[gi] = GatherGroup{g.d_state, g.d_fe, g.ne, g.goff, g.type, (int)g.hasM};
+    }
+    const int64_t ngrp = (int64_t)c->sell_groups.size();
+    hipLaunchKernelGGL(k_product_rows, dim3(grid_for(ngrp, 4)), dim3(256), 0, s, ga,
+                       c->d_sell_groups, ngrp, c->d_contrib, c->d_row_ptr, c->d_diag, c->d_fixmask,
+                       y, c->nn);
+  } else {
+    hipLaunchKernelGGL(k_fill<double>, dim3(512), dim3(256), 0, s, y, 3 * c->nn, 0.0);
+    for (const ElemGroup& g : c->groups) {
+      const int ncol = (int)g.color_off.size() - 1;
+      for (int k = 0; k < ncol; ++k) {
+        const int64_t e0 = g.color_off[k], e1 = g.color_off[k + 1];
+        if (e1 <= e0) continue;
+        if (g.type == kTet)
+          hipLaunchKernelGGL(k_tet_apply, dim3(grid_for(4 * (e1 - e0), kScatterThreads)),
+                             dim3(kScatterThreads), 0, s, tet_args(g, e0, e1), c->d_U, v, y,
+                             c->d_fixmask);
+        else
+          hipLaunchKernelGGL(k_truss_apply, dim3(grid_for(2 * (e1 - e0), kScatterThreads)),
+                             dim3(kScatterThreads), 0, s, truss_args(g, e0, e1), c->d_U, v, y,
+                             c->d_fixmask);
+      }
     }
   }
   hipLaunchKernelGGL(k_fixed_copy, dim3(grid_for(c->nn, 256)), dim3(256), 0, s, v, y, c->d_fixmask,

@@ -141,3 +141,44 @@ def test_adjoint_vs_finite_differences(prec):
         print(f"  element {e}: rel {abs(fd - g[e]) / abs(g[e]):.2e}", flush=True)
         assert abs(fd - g[e]) <= 1e-5 * abs(g[e]), (e, fd, g[e])
     sol.analysis.state.close()
+
+
+@pytest.mark.parametrize("prec", [_capi.PRECISION_MIXED, _capi.PRECISION_FP64])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (4, 3, 3), (9, 7, 5)])
+@pytest.mark.parametrize("mat", [_capi.MAT_NEOHOOKEAN, _capi.MAT_SVK])
+def test_tangent_product_by_rows_matches_colours(monkeypatch, mat, shape, prec):
+    """The refined solve's tangent product by element and row passes (gather assembly)
+    against its coloured launches (scatter assembly): two tet groups of different
+    materials, bars, partly fixed nodes and a node of no element; row counts under,
+    at the edge of and past a slice.  Both solves end at 1e-11 of the right-hand side,
+    as in the oracle test above."""
+    print(f"[gpu] tangent product {mat} {shape} precision {prec}", flush=True)
+    sm = meshes.cube(shape[0], ny=shape[1], nz=shape[2], jitter=0.05, seed=2)
+    coords = np.concatenate([sm.coords, [[4.0, 4.0, 4.0]]])
+    nn, half = len(coords), (len(sm.tets) + 1) // 2
+    bars = sm.tets[:: max(1, len(sm.tets) // 20), :2]
+    fixed = np.concatenate([(3 * sm.node_sets["x0"][:, None] + np.arange(3)).reshape(-1),
+                            [3 * sm.node_sets["x1"][0] + 1], 3 * (nn - 1) + np.arange(3)])
+    r = np.random.default_rng(6)
+    U = 1e-2 * r.normal(size=3 * nn)
+    U[fixed] = 0
+    g = r.normal(size=3 * nn)
+    out = []
+    for mode in ("gather", "scatter"):
+        monkeypatch.setenv("ONSAS_ASSEMBLY", mode)
+        c = _capi.Context(prec)
+        try:
+            c.set_nodes(coords)
+            c.add_tet_group(sm.tets[:half], mat, (8.3e5, 3.8e5))
+            c.add_tet_group(sm.tets[half:], _capi.MAT_LINEAR, (1.0e6, 0.3))
+            c.add_truss_group(bars, _capi.STRAIN_GREEN, 2e5, 1e-2)
+            c.set_fixed_dofs(np.unique(fixed))
+            c.finalize()
+            c.set_linear_solver(_capi.LINSOLVE_AUTO, maxiter=20000)
+            c.set_U(U)
+            res = c.adjoint_shear(0, g)
+            out.append(np.asarray(res[0] if isinstance(res, tuple) else res))
+        finally:
+            c.close()
+    assert np.abs(out[0]).max() > 0
+    assert np.abs(out[0] - out[1]).max() <= 1e-9 * np.abs(out[1]).max()
