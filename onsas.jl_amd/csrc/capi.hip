@@ -403,7 +403,7 @@ void onsas_destroy(onsas_ctx* ctx) {
   for (auto& g : c->groups)
     for (void* p : {(void*)g.d_conn, (void*)g.d_geo, (void*)g.d_slot, (void*)g.d_G, (void*)g.d_perm,
                     g.d_state, (void*)g.d_fe, (void*)g.d_cidx, (void*)g.locate.d_ptr,
-                    (void*)g.locate.d_elem})
+                    (void*)g.locate.d_elem, (void*)g.locate.d_rec})
       if (p) (void)hipFree(p);
   void* ptrs[] = {c->d_x, c->d_y, c->d_z, c->d_fixmask, c->d_row_ptr, c->d_col, c->d_diag, c->d_K,
                   c->d_Dinv, c->d_U, c->d_Uasm, c->d_fint, c->d_fext, c->d_res, c->d_nodal, c->d_px, c->d_pr,
@@ -1059,6 +1059,11 @@ int build_locate_grid(Ctx* c, ElemGroup& g) {
       for (int y = b0[1]; y <= b1[1]; ++y)
         for (int x = b0[0]; x <= b1[0]; ++x) list[fill[((int64_t)z * lg.nb[1] + y) * lg.nb[0] + x]++] = pos[u];
   }
+  for (void** p : {(void**)&lg.d_rec, (void**)&lg.d_ptr, (void**)&lg.d_elem}) {
+    (void)hipFree(*p);  // of an attempt that ran out of memory
+    *p = nullptr;
+  }
+  ONSAS_TRY(onsas::launch_locate_records(c, g, &lg.d_rec));
   ONSAS_HIP_TRY(c, hipMalloc((void**)&lg.d_ptr, ptr.size() * sizeof(int64_t)));
   ONSAS_HIP_TRY(c, hipMemcpy(lg.d_ptr, ptr.data(), ptr.size() * sizeof(int64_t), hipMemcpyHostToDevice));
   ONSAS_HIP_TRY(c, hipMalloc((void**)&lg.d_elem, list.size() * sizeof(int32_t)));

@@ -53,6 +53,7 @@ struct LocateGrid {
   int nb[3] = {0, 0, 0};
   int64_t* d_ptr = nullptr;
   int32_t* d_elem = nullptr;  // array positions
+  double* d_rec = nullptr;    // the candidates' records (k_locate)
 };
 
 struct ElemGroup {
@@ -411,6 +412,7 @@ size_t stage_gather_lds(const Ctx* c);  // its LDS bytes per workgroup
 int launch_gather_init(Ctx* c);                                 // zero padding, identity Dinv
 int ensure_bsr(Ctx* c);                                         // d_K from d_Ksell if stale
 int launch_tangent_apply_f64(Ctx* c, const double* v_dev, double* y_dev);  // y = K(U) v, FP64
+int launch_locate_records(Ctx* c, const ElemGroup& g, double** rec);
 int launch_locate(Ctx* c, int g, const double* px, const double* py, const double* pz, int64_t np,
                   double tol, int64_t* elem, double* w);
 

@@ -250,3 +250,37 @@ def test_stored_stress_is_at_the_last_assembly(oracle, monkeypatch, prec):
           flush=True)
     assert seen_gap > 1e-7  # the test can tell U_k from U_k + dU
     sol.analysis.state.close()
+
+
+@pytest.mark.parametrize("npts", [1, 3, 4, 5, 15, 16, 17, 257])
+def test_point_location_counts(npts):
+    """Point counts around the lanes' groups (16 a point, 4 points a wave, 16 a
+    workgroup), on a box so flat that its bins hold long candidate lists, and on one
+    tetrahedron; not-a-number coordinates are in no element."""
+    from onsas_amd import _capi, meshes
+    print(f"[gpu] point location, {npts} points", flush=True)
+    rng = np.random.default_rng(npts)
+    for sm, tets in ((meshes.cube(5, ny=4, nz=1, jitter=0.1, seed=2), None),
+                     (meshes.cube(1, seed=2), slice(0, 1))):
+        t = sm.tets if tets is None else sm.tets[tets]
+        used = np.unique(t)
+        renum = np.full(sm.nn, -1)
+        renum[used] = np.arange(len(used))
+        X, t = sm.coords[used], renum[t].astype(np.int32)
+        c = _capi.Context(_capi.PRECISION_FP64)
+        try:
+            c.set_nodes(X)
+            c.add_tet_group(t, _capi.MAT_NEOHOOKEAN, (8.3e5, 3.8e5))
+            c.set_fixed_dofs(np.arange(9))
+            c.finalize()
+            P = rng.uniform(X.min(0) - 0.1, X.max(0) + 0.1, size=(npts, 3))
+            P[::2] = X[t[rng.integers(len(t), size=len(P[::2]))]].mean(axis=1)
+            eb, wb = _brute_locate(X, t, P)
+            if npts > 4:
+                P[3, 1] = np.nan
+                eb[3], wb[3] = -1, 0
+            e, w = c.locate_points(0, P)
+            np.testing.assert_array_equal(e, eb)
+            np.testing.assert_allclose(w, wb, rtol=0, atol=1e-12)
+        finally:
+            c.close()
