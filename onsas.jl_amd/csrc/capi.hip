@@ -413,7 +413,7 @@ void onsas_destroy(onsas_ctx* ctx) {
                   c->d_contrib, c->d_sell_groups, (void*)c->d_stage_groups,
                   (void*)c->d_stage_steps, c->d_stage, c->d_stage_words, c->d_stage_pairs,
                   c->d_pair_row, c->d_colmask, c->d_snap[0], c->d_snap[1], c->d_ppq,
-                  (void*)c->d_gmslots};
+                  (void*)c->d_gmslots, (void*)c->d_share};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (c->h_sc) (void)hipHostFree(c->h_sc);

@@ -365,8 +365,10 @@ struct Ctx {
   // one-launch PCG and GMRES of small models (resident_solve.hip): the exchange's
   // slots; epochs in use so far; the longest wait in ticks of the 100 MHz clock (ONSAS_RESIDENT_TICKS)
   bool pcg_resident = false;  // ONSAS_PCG_RESIDENT=0 turns it off (read at finalize)
+  bool one_xcd = true;        // resident launches may meet in one XCD (ONSAS_RESIDENT_XCD=0: not)
   unsigned long long* d_gslots = nullptr;    // the tail of d_part's allocation
   unsigned long long* d_gmslots = nullptr;  // the same for GMRES (on its first use)
+  unsigned long long* d_share = nullptr;    // a vector handed from workgroup to workgroup
   uint32_t gslot_epoch = 1;
   long long gslot_ticks = 20000000;  // 0.2 s
 
@@ -448,7 +450,7 @@ int launch_pcg_solve(Ctx* c, const double* b_dev, bool forcing, int* iters, doub
                      int* converged, int* breakdown, const void* x0 = nullptr, int expect = -1);
 // ---- resident_solve.hip ----
 bool pcg_resident_fits(const Ctx* c);
-void pcg_resident_setup(Ctx* c);                                // at finalize
+int pcg_resident_setup(Ctx* c);                                 // at finalize
 int launch_pcg_resident(Ctx* c, const double* b_dev, bool* ran, int* iters, double* relres,
                         int* converged, int* breakdown);
 // A whole Newton step (residual, solve, update, norms) as one launch; *ran = false:

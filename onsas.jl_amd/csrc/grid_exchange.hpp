@@ -8,14 +8,12 @@
 // half of the double, so a word carries its own "ready" mark and the sum is
 // exact; the partials are added by a fixed tree, the same in every workgroup,
 // so all of them take the same branches and a solve is bit-identical from run
-// to run.  A sum alone, measured on one MI355X: 1.2 us for 1 to 8 workgroups, 2.0 us for 32,
-// 3.3 us for 128, against 4 to 8 us for a kernel boundary with its drain,
-// launch and first loads.
+// to run.  A sum alone, measured on one MI355X: 1.2 us for 2 workgroups, 1.9 us for
+// 32, 2.4 us for 64 and 3.3 us for 128 across the device, against 4 to 8 us for a
+// kernel boundary with its drain, launch and first loads.  Vectors are handed over in
+// the same way, every component in words of its own, so nothing else orders the
+// workgroups' memory and the read-only data stays cached.
 //
-// Everything shared goes through device-scope loads and stores (they bypass the
-// per-XCD L2s), and a workgroup's vector stores are complete (vmcnt 0, then the
-// barrier, in grid_sum4) before its partial is published, so no L2
-// write-back or invalidation is needed and the read-only data stays cached.
 // Waits are bounded: a workgroup that polls past `limit` clock ticks (or sees
 // another's abort) raises the abort word and the launch drains; the host then
 // solves with the one-kernel-per-step path.
@@ -31,7 +29,7 @@ namespace onsas {
 
 constexpr int kMaxGridWg = 128;  // workgroups of a resident launch
 constexpr int kPollSlots = 64;   // slots that grid_sum4 polls at a time
-constexpr size_t kGridSlotWords = 16 * kMaxGridWg;  // the PCG's slots: sums of four values, twice
+constexpr size_t kGridSlotWords = 32 * kMaxGridWg;  // the PCG's slots: sums of four values, four times
 
 template <typename T>
 __device__ inline T agent_load(const T* p) {
@@ -41,41 +39,42 @@ template <typename T>
 __device__ inline void agent_store(T* p, T v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// The loads of values that other workgroups write: past the caches like
-// agent_load, and 12 or 16 bytes an instruction.  Every value among them is at
-// most 8 bytes and aligned, and carries its own mark.
+// Where the workgroups meet.  Device: the loads and stores of everything shared pass
+// the caches (sc1).  One XCD: they meet in its L2 (stores are written through to it,
+// loads take sc0 nt and so do not stay in the CU's cache); an exchange of 27 / 64
+// workgroups is 1.1 / 1.1 us against 1.9 / 2.4.  A load that did come from the CU's
+// cache would show an old mark and be repeated.
+enum class Meet { kDevice, kXcd };
+
+// 16 bytes that other workgroups write; the caller keeps the load in its loop (poll).
 using SharedBuf = __amdgpu_buffer_rsrc_t;
 __device__ inline SharedBuf shared_buf(const void* p, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
 }
-constexpr int kSharedLoad = (int)(0x80000000u | 16u);  // volatile (each poll loads anew), sc1
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
+template <Meet M>
+constexpr int kSharedLoad = M == Meet::kXcd ? 3 : 16;  // sc0 nt, sc1
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-__device__ inline void shared_load3(SharedBuf b, uint32_t off, uint32_t (&w)[3]) {
-  const u32x3 v = __builtin_amdgcn_raw_buffer_load_b96(b, off, 0, kSharedLoad);
-  w[0] = v[0];
-  w[1] = v[1];
-  w[2] = v[2];
+template <Meet M>
+__device__ inline u32x4 shared_load(SharedBuf b, uint32_t off) {
+  return __builtin_amdgcn_raw_buffer_load_b128(b, off, 0, kSharedLoad<M>);
 }
-__device__ inline void shared_load2(SharedBuf b, uint32_t off, unsigned long long (&w)[2]) {
-  const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(b, off, 0, kSharedLoad);
-  w[0] = ((unsigned long long)v[1] << 32) | v[0];
-  w[1] = ((unsigned long long)v[3] << 32) | v[2];
+template <Meet M>
+__device__ inline void shared_store(unsigned long long* p, unsigned long long w) {
+  if (M == Meet::kXcd)
+    __hip_atomic_store(p, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  else
+    agent_store(p, w);
 }
-__device__ inline void shared_load3(SharedBuf b, uint32_t off, unsigned long long (&w)[3]) {
-  const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(b, off, 0, kSharedLoad);
-  const u32x2 u = __builtin_amdgcn_raw_buffer_load_b64(b, off + 16, 0, kSharedLoad);
-  w[0] = ((unsigned long long)v[1] << 32) | v[0];
-  w[1] = ((unsigned long long)v[3] << 32) | v[2];
-  w[2] = ((unsigned long long)u[1] << 32) | u[0];
+// the XCD this wave runs on
+__device__ inline int xcd_id() {
+  int x;
+  asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(x));
+  return x;
 }
-// this wave's stores have reached the device-coherent level
-__device__ inline void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 struct GridSlots {
-  unsigned long long* words;  // kMaxGridWg slots of the sum's 2 NV words each
-  int nwg;
+  unsigned long long* words;  // kMaxGridWg slots
+  int nwg, id;
   int* abort;                 // device word: nonzero once a wait has expired
   long long limit;            // ticks of the 100 MHz clock a wait may take
 };
@@ -98,20 +97,13 @@ __device__ inline double wg_sum4(const double* sh) {
   return stride_sum<4>(lane < 4 * (T / 64) ? sh[lane] : 0.0);
 }
 
-// N values at the byte offsets off, two words each, once all of them carry the
-// epoch; false once the launch is aborted.
-template <int N>
-__device__ inline bool poll_values(SharedBuf buf, const uint32_t (&off)[N], uint32_t epoch,
-                                   const GridSlots& gs, unsigned long long (&w)[N][2]) {
+// load() until it says that everything has arrived; false once the launch is aborted
+template <typename Load>
+__device__ inline bool poll(const GridSlots& gs, Load load) {
   long long t0 = 0;
   for (uint32_t spin = 0;; ++spin) {
-    bool ready = true;
-#pragma unroll
-    for (int q = 0; q < N; ++q) shared_load2(buf, off[q], w[q]);
-#pragma unroll
-    for (int q = 0; q < N; ++q)
-      ready = ready && (uint32_t)(w[q][0] >> 32) == epoch && (uint32_t)(w[q][1] >> 32) == epoch;
-    if (ready) return true;
+    asm volatile("" ::: "memory");  // the loads stay in the loop
+    if (load()) return true;
     if ((spin & 63u) == 0) {
       const long long now = wall_clock64();
       if (spin == 0) t0 = now;
@@ -122,22 +114,96 @@ __device__ inline bool poll_values(SharedBuf buf, const uint32_t (&off)[N], uint
     }
   }
 }
-__device__ inline double words_value(unsigned long long hi, unsigned long long lo) {
-  return __longlong_as_double((long long)((hi << 32) | (lo & 0xffffffffull)));
+// N values at the byte offsets off, a high and a low word each, once all carry the epoch
+template <Meet M, int N>
+__device__ inline bool poll_values(SharedBuf buf, const uint32_t (&off)[N], uint32_t epoch,
+                                   const GridSlots& gs, double (&v)[N]) {
+  return poll(gs, [&] {
+    u32x4 w[N];
+    bool ready = true;
+#pragma unroll
+    for (int q = 0; q < N; ++q) w[q] = shared_load<M>(buf, off[q]);
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+      ready = ready && w[q][1] == epoch && w[q][3] == epoch;
+      v[q] = __hiloint2double((int)w[q][0], (int)w[q][2]);
+    }
+    return ready;
+  });
 }
 __device__ inline unsigned long long value_word(double p, uint32_t epoch, bool low) {
   const unsigned long long b = (unsigned long long)__double_as_longlong(p);
   return ((unsigned long long)epoch << 32) | (low ? (b & 0xffffffffull) : (b >> 32));
 }
 
+// A node of a vector that its neighbours read: 16 bytes, its three components and the
+// epoch (FP64: twice 16 bytes, each with 12 bytes of the components and the epoch).
+// An aligned 16-byte store or load of a lane is one request to one cache line and so
+// is seen whole (1.2e8 reads of words being written showed no mixture, in either
+// meeting place).  A sum between the readers' use and the next hand-over makes sure
+// that nothing is overwritten before all have read it.
+template <typename KT>
+constexpr uint32_t kShareBytes = 4 * sizeof(KT);  // per node
+template <typename KT>
+constexpr int kShareLanes = sizeof(KT) / 4;       // lanes that store a node
+template <Meet M>
+__device__ inline void shared_store(SharedBuf b, uint32_t off, u32x4 w) {
+  if (M == Meet::kXcd)
+    __builtin_amdgcn_raw_buffer_store_b128(w, b, off, 0, 1);   // sc0
+  else
+    __builtin_amdgcn_raw_buffer_store_b128(w, b, off, 0, 16);  // sc1
+}
+// node i's part of lane `part` (0, and in FP64 0 and 1)
+template <Meet M>
+__device__ inline void share_node(SharedBuf z, uint32_t i, int part, float a, float b, float c,
+                                  uint32_t epoch) {
+  (void)part;
+  shared_store<M>(z, kShareBytes<float> * i,
+                  u32x4{__float_as_uint(a), __float_as_uint(b), __float_as_uint(c), epoch});
+}
+template <Meet M>
+__device__ inline void share_node(SharedBuf z, uint32_t i, int part, double a, double b, double c,
+                                  uint32_t epoch) {
+  const double x = part ? c : a;
+  shared_store<M>(z, kShareBytes<double> * i + 16u * part,
+                  u32x4{(uint32_t)__double2loint(x), (uint32_t)__double2hiint(x),
+                        (uint32_t)(part ? __double2hiint(b) : __double2loint(b)), epoch});
+}
+// The three components of the nodes at the byte offsets off, once they carry the
+// epoch; false once the launch is aborted.
+template <Meet M, typename KT, int N>
+__device__ inline bool gather_shared(SharedBuf z, const uint32_t (&off)[N], uint32_t epoch,
+                                     const GridSlots& gs, KT (&zj)[N][3]) {
+  constexpr int P = kShareLanes<KT>;
+  return poll(gs, [&] {
+    u32x4 w[N][P];
+    bool ready = true;
+#pragma unroll
+    for (int q = 0; q < N; ++q)
+#pragma unroll
+      for (int p = 0; p < P; ++p) w[q][p] = shared_load<M>(z, off[q] + 16u * p);
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+      ready = ready && w[q][0][3] == epoch && w[q][P - 1][3] == epoch;
+      if constexpr (P == 1) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) zj[q][c] = __uint_as_float(w[q][0][c]);
+      } else {
+        zj[q][0] = __hiloint2double((int)w[q][0][1], (int)w[q][0][0]);
+        zj[q][1] = __hiloint2double((int)w[q][1][2], (int)w[q][0][2]);
+        zj[q][2] = __hiloint2double((int)w[q][1][1], (int)w[q][1][0]);
+      }
+    }
+    return ready;
+  });
+}
+
 // The four sums over all workgroups of the launch; false once the launch is
 // aborted (the same answer for every thread of the workgroup).  sh: 4 T / 64 + 5
-// doubles, free again at the caller's next barrier.  The stores that the caller
-// made before it are complete at the device-coherent level before its part is
-// published.  late: an LDS word that a thread has set whose own wait expired
-// before the sum; nothing is published then.  A load takes 16 slots (a lane its
-// sum's 16 bytes of one).
-template <int T>
+// doubles, free again at the caller's next barrier.  late: an LDS word that a thread
+// has set whose own wait expired before the sum; nothing is published then.  A load
+// takes 16 slots (a lane its sum's 16 bytes of one).
+template <Meet M, int T>
 __device__ inline bool grid_sum4(double (&v)[4], const GridSlots& gs, uint32_t epoch, double* sh,
                                  const int* late) {
   double* res = sh + 4 * (T / 64);
@@ -146,31 +212,30 @@ __device__ inline bool grid_sum4(double (&v)[4], const GridSlots& gs, uint32_t e
     const double p = wave_sum4(v);
     if (lane < 4) sh[4 * (threadIdx.x >> 6) + lane] = p;
   }
-  stores_done();
   __syncthreads();
   if (threadIdx.x < 64) {
     const double p = wg_sum4<T>(sh);
     bool ok = *late == 0;
     if (ok && lane < 4) {
-      unsigned long long* mine = gs.words + 8 * (size_t)blockIdx.x + 2 * lane;
-      agent_store(mine, value_word(p, epoch, false));
-      agent_store(mine + 1, value_word(p, epoch, true));
+      unsigned long long* mine = gs.words + 8 * (size_t)gs.id + 2 * lane;
+      shared_store<M>(mine, value_word(p, epoch, false));
+      shared_store<M>(mine + 1, value_word(p, epoch, true));
     }
     const SharedBuf buf = shared_buf(gs.words, 64u * kMaxGridWg);
     double acc = 0;
     for (int g0 = 0; ok && g0 < gs.nwg; g0 += kPollSlots) {
-      unsigned long long w[4][2];
+      double x[4];
       uint32_t off[4];
       bool has[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int g = g0 + 16 * j + (lane >> 2);
         has[j] = g < gs.nwg;
-        off[j] = 64u * (has[j] ? g : blockIdx.x) + 16u * (lane & 3);
+        off[j] = 64u * (has[j] ? g : gs.id) + 16u * (lane & 3);
       }
-      ok = poll_values<4>(buf, off, epoch, gs, w);
+      ok = poll_values<M, 4>(buf, off, epoch, gs, x);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) acc += has[j] ? words_value(w[j][0], w[j][1]) : 0.0;
+      for (int j = 0; j < 4; ++j) acc += has[j] ? x[j] : 0.0;
     }
     ok = __all(ok);
     acc = stride_sum<4>(acc);

@@ -14,14 +14,16 @@
 //   p <- z + beta p, q <- w + beta q;  p.q <- z.w + beta (z.q + p.w) + beta^2 p.q
 // The last line is p.q written out (no conjugacy is assumed), so the recurrences,
 // the stop and breakdown rules and the scalars are those of k_pcg_A / k_pcg_B and
-// only the rounding of p.q differs.  z needs no sum to be safe to read: a
-// component that is not there yet reads as a mark.
-// 3.4 us an iteration at 1,680 nodes (27 workgroups), 1.7 us at 125 nodes (one
-// workgroup, z and the sums in LDS).  With p.q and (r.z, r.r) as two sums, z safe to
-// read only after the second, a tree per sum and 4- and 8-byte loads it was 4.6 and
-// 2.6 us; polling by every wave of a workgroup instead of one costs 1 us.
+// only the rounding of p.q differs.  z needs no sum to be safe to read: a node that
+// is not there yet carries an old epoch.
+// An iteration takes 2.3 us at 1,680 nodes (27 workgroups, met in one XCD), 1.1 us at
+// 125 nodes (one workgroup, z and the sums in LDS).  Met in device memory it is 3.4 us;
+// with p.q and (r.z, r.r) as two sums, z safe to read only after the second, a tree per
+// sum and 4- and 8-byte loads it was 4.6 and 2.6 us.  Polling by every wave of a
+// workgroup instead of one costs 1 us.
 #include <cmath>
 #include <cstdlib>
+#include <type_traits>
 
 #include <hip/hip_ext.h>
 
@@ -31,21 +33,6 @@
 namespace onsas {
 
 namespace {
-
-// A component of z that its owner has not written yet: a signalling NaN, which
-// no arithmetic produces.
-template <typename KT>
-struct Unwritten;
-template <>
-struct Unwritten<float> {
-  using Bits = uint32_t;
-  static constexpr Bits mark = 0x7f9a5a5au;
-};
-template <>
-struct Unwritten<double> {
-  using Bits = unsigned long long;
-  static constexpr Bits mark = 0x7ff25a5a5a5a5a5aull;
-};
 
 template <typename KT>
 struct ResidentArgs {
@@ -58,11 +45,12 @@ struct ResidentArgs {
   const uint8_t* mask;
   const double* b;     // right-hand side; of a Newton step f_ext
   KT* x;
-  KT* zb[2];           // z of the even and odd iterations, handed from workgroup to workgroup
+  unsigned long long* z;  // z, handed from workgroup to workgroup (share_node)
   Scalars* sc;         // device: the abort word, a Newton step's norms
   Scalars* host;       // pinned host: the results
-  unsigned long long* slots;  // two regions of 8 words per workgroup, used in turn
-  uint32_t base;              // epochs base + 1, base + 2, ... are new to the slots
+  unsigned long long* slots;  // four regions of 8 words per workgroup
+  uint32_t base;              // epochs base + 1, base + 2, ... are new to the slots and z
+  int nwg;                    // workgroups (of kXcd launches every 8th)
   long long limit;
   int64_t nn;
   int maxiter;
@@ -74,43 +62,17 @@ struct ResidentArgs {
   double *res, *U;
 };
 
+// PcgState::aborted of a launch whose workgroups did not share one XCD
+constexpr int kNotOneXcd = 2;
+
 // a result for the host, in pinned host memory
 template <typename T>
 __device__ inline void host_store(T* p, T v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// z of the columns at the byte offsets cj, each value once its owner has written
-// it; false once the wait has expired.
-template <typename KT, int NB>
-__device__ inline bool gather_published(SharedBuf z, const uint32_t (&cj)[NB], const GridSlots& gs,
-                                        KT (&zj)[NB][3]) {
-  using W = Unwritten<KT>;
-  using Bits = typename W::Bits;
-  long long t0 = 0;
-  for (uint32_t spin = 0;; ++spin) {
-    Bits w[NB][3];
-    bool ready = true;
-#pragma unroll
-    for (int q = 0; q < NB; ++q) shared_load3(z, cj[q], w[q]);
-#pragma unroll
-    for (int q = 0; q < NB; ++q)
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        ready = ready && w[q][c] != W::mark;
-        zj[q][c] = __builtin_bit_cast(KT, w[q][c]);
-      }
-    if (ready) return true;
-    if ((spin & 63u) == 0) {
-      const long long now = wall_clock64();
-      if (spin == 0) t0 = now;
-      if (now - t0 > gs.limit || agent_load(gs.abort) != 0) {
-        agent_store(gs.abort, 1);
-        return false;
-      }
-    }
-  }
-}
+// Waves a SIMD that the registers of k_pcg_resident leave (up to 168 and 256 of them).
+constexpr int xcd_waves(size_t kt) { return kt == 4 ? 3 : 2; }
 
 // L lanes a block row (lane ph takes the row's slots ph, ph + L, ...: at most
 // NB), T threads a workgroup.  Lanes 0, 1, 2 of a row hold the row's three
@@ -124,26 +86,31 @@ __device__ inline bool gather_published(SharedBuf z, const uint32_t (&cj)[NB], c
 // the device: some 60 us of a step of 195 us at 125 nodes, now 5 us; the step
 // 195 -> 152 us).
 //
-// Hand-over of z: z_k (k >= 1) is published in zb[k & 1] after sum k - 1, and
-// marked unwritten again after sum k, by when every workgroup has read it; the
-// marks are complete before their workgroup's part of sum k + 1 is published,
-// and z_{k+2} is polled only after that sum.  The sums take two slot regions in
-// turn: a workgroup may be in sum k + 1 while another still reads sum k.
-template <typename KT, int L, int NB, int T, bool ONE>
+// The sums take two slot regions in turn: a workgroup may be in sum k + 1 while
+// another still reads sum k.  z has one buffer: the sum before its next hand-over is
+// complete only when every workgroup has made its product.
+//
+// kXcd: every 8th workgroup takes part.  Consecutive workgroups go round the 8 XCDs, so
+// these share one, which a first sum across the device confirms (if not, nothing has
+// been done and the host launches the other kernel); they then meet in its L2.
+template <typename KT, int L, int NB, int T, bool ONE, Meet M>
 __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs<KT> a) {
-  using W = Unwritten<KT>;
-  using Bits = typename W::Bits;
+  constexpr int kSpread = M == Meet::kXcd ? 8 : 1;
+  if (blockIdx.x % kSpread) return;
+  const int wg = (int)(blockIdx.x / kSpread);
   __shared__ double sh[4 * (T / 64) + 5];
   __shared__ __align__(16) KT shz[ONE ? 4 * (T / L) : 4];  // a node's z and a pad: 16-byte reads
   __shared__ int late;  // a wait for z has expired
   const int t = threadIdx.x;
   const int ph = t % L;
-  const int64_t i = ((int64_t)blockIdx.x * T + t) / L;
+  const int64_t i = ((int64_t)wg * T + t) / L;
   const bool row = i < a.nn;
   const bool own = row && ph < 3;
   uint32_t ep = a.base;
+  GridSlots gs{a.slots, a.nwg, wg, &a.sc->pcg.aborted, a.limit};
   // the four sums over the launch; false (and *host says so) once it is aborted
-  auto sums = [&](double(&s)[4]) -> bool {
+  auto sums = [&](double(&s)[4], auto m) -> bool {
+    constexpr Meet W = decltype(m)::value;
     ++ep;
     if (ONE) {
       const double p = wave_sum4(s);
@@ -154,13 +121,11 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs<KT> a) {
       for (int q = 0; q < 4; ++q) s[q] = read_lane(q4, q);
       return true;
     }
-    const GridSlots gs{a.slots + (ep & 1u) * (8 * kMaxGridWg), (int)gridDim.x, &a.sc->pcg.aborted,
-                       a.limit};
-    if (grid_sum4<T>(s, gs, ep, sh, &late)) return true;
+    gs.words = a.slots + ((ep & 1u) + (W == Meet::kXcd ? 2u : 0u)) * (8 * kMaxGridWg);
+    if (grid_sum4<W, T>(s, gs, ep, sh, &late)) return true;
     if (t == 0) host_store(&a.host->pcg.aborted, 1);
     return false;
   };
-  const GridSlots gw{nullptr, (int)gridDim.x, &a.sc->pcg.aborted, a.limit};
 
   KT v[NB][9];
   uint32_t cj[NB];  // the column's z: its byte offset, or its index in shz
@@ -173,7 +138,7 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs<KT> a) {
       const int m = ph + L * q;
       const bool has = row && m < rounds;
       const int64_t b = b0 + a.rstride * (has ? m : 0);
-      cj[q] = (ONE ? 4u : 3u * (uint32_t)sizeof(KT)) * (uint32_t)(has ? a.scol[b + l] : 0);
+      cj[q] = (ONE ? 4u : kShareBytes<KT>) * (uint32_t)(has ? a.scol[b + l] : 0);
 #pragma unroll
       for (int e = 0; e < 9; ++e) v[q][e] = has ? a.sval[9 * b + 64 * e + l] : KT(0);
     }
@@ -215,9 +180,17 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs<KT> a) {
       sm[0] = r * r;
     }
     bk = (KT)r;
-    if (!ONE) {
-      agent_store((Bits*)a.zb[0] + dof, W::mark);
-      agent_store((Bits*)a.zb[1] + dof, W::mark);
+  }
+  const std::integral_constant<Meet, M> here;
+  if (M == Meet::kXcd) {  // do they share one XCD?  n sum x^2 = (sum x)^2
+    if (t == 0) late = 0;
+    __syncthreads();
+    const double x = t == 0 ? (double)xcd_id() : 0.0;
+    double q[4] = {x, x * x, 0, 0};
+    if (!sums(q, std::integral_constant<Meet, Meet::kDevice>())) return;
+    if (a.nwg * q[1] != q[0] * q[0]) {
+      if (t == 0) host_store(&a.host->pcg.aborted, kNotOneXcd);
+      return;
     }
   }
   // warm start: x = al x0, r = b - al t with t = K x0 and al = t.b / t.t, the scale
@@ -229,7 +202,7 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs<KT> a) {
     for (int q = 0; q < NB; ++q)
 #pragma unroll
       for (int c = 0; c < 3; ++c)
-        xj[q][c] = ONE ? a.x0[cj[q] / 4 * 3 + c] : ((const KT*)((const char*)a.x0 + cj[q]))[c];
+        xj[q][c] = a.x0[cj[q] / (ONE ? 4u : kShareBytes<KT>) * 3 + c];
     tw = product(xj);
     if (own && freed) {
       x0 = a.x0[dof];
@@ -239,29 +212,28 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs<KT> a) {
   }
   if (t == 0) late = 0;
   __syncthreads();
-  if (!sums(sm)) return;  // past it no workgroup sees what zb held before
+  if (!sums(sm, here)) return;
   const double r2 = sm[0], f2 = sm[1];
   const double al = a.x0 && sm[3] > 0 && isfinite(sm[2]) && isfinite(sm[3]) ? sm[2] / sm[3] : 0.0;
   if (own) {
     xs = freed ? (KT)(al * (double)x0) : KT(0);
     rs = freed ? (a.x0 ? (KT)((double)bk - al * (double)tw) : bk) : KT(0);
   }
-  // z = D^-1 r, published for iteration k
-  auto next_z = [&](int k) {
+  const SharedBuf z = shared_buf(a.z, kShareBytes<KT> * (uint32_t)a.nn);
+  // z = D^-1 r, published
+  auto next_z = [&]() {
     const KT r0 = quad_lane<0>(rs), r1 = quad_lane<1>(rs), rz2 = quad_lane<2>(rs);
-    if (own) {
-      zs = d0 * r0 + d1 * r1 + d2 * rz2;
-      if (ONE)
-        shz[4 * i + ph] = zs;
-      else
-        agent_store((Bits*)a.zb[k & 1] + dof, __builtin_bit_cast(Bits, zs));
+    if (own) zs = d0 * r0 + d1 * r1 + d2 * rz2;
+    if (ONE) {
+      if (own) shz[4 * i + ph] = zs;
+      __syncthreads();
+    } else {
+      const KT s0 = quad_lane<0>(zs), s1 = quad_lane<1>(zs), s2 = quad_lane<2>(zs);
+      if (row && ph < kShareLanes<KT>) share_node<M>(z, (uint32_t)i, ph, s0, s1, s2, ep);
     }
-    if (ONE) __syncthreads();
   };
-  next_z(0);
+  next_z();
 
-  const uint32_t zbytes = 3u * (uint32_t)sizeof(KT) * (uint32_t)a.nn;
-  const SharedBuf z0 = shared_buf(a.zb[0], zbytes), z1 = shared_buf(a.zb[1], zbytes);
   double rz = 0, rr = 0, rzp = 0, pq = 0, bb = 0, eta = 0, tol2 = 0;
   int k = 0, conv = 0, brk = 0;
   for (;; ++k) {
@@ -271,7 +243,7 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs<KT> a) {
       for (int q = 0; q < NB; ++q)
 #pragma unroll
         for (int c = 0; c < 3; ++c) zj[q][c] = shz[cj[q] + c];
-    } else if (!gather_published<KT, NB>((k & 1) ? z1 : z0, cj, gw, zj)) {
+    } else if (!gather_shared<M, KT, NB>(z, cj, ep, gs, zj)) {
       late = 1;
     }
     const KT w = product(zj);
@@ -282,7 +254,7 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs<KT> a) {
       sm[2] = (double)zs * (double)w;
       sm[3] = k > 0 ? (double)zs * (double)qs + (double)ps * (double)w : (double)bk * (double)bk;
     }
-    if (!sums(sm)) return;
+    if (!sums(sm, here)) return;
     if (k == 0) {
       bb = sm[3];
       sm[3] = 0;
@@ -306,17 +278,10 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs<KT> a) {
       qs = w + beta * qs;
       xs += alpha * ps;
       rs -= alpha * qs;
-      if (!ONE) agent_store((Bits*)a.zb[k & 1] + dof, W::mark);  // every workgroup has read it
     }
-    next_z(k + 1);
+    next_z();
   }
-  if (own) {
-    a.x[dof] = xs;
-    if (!ONE) {  // no marks are left behind
-      agent_store(a.zb[0] + dof, KT(0));
-      agent_store(a.zb[1] + dof, KT(0));
-    }
-  }
+  if (own) a.x[dof] = xs;
   // Newton update: U[free] += x, with the norms of x and of U before
   double du = 0;
   sm[0] = sm[1] = sm[2] = sm[3] = 0;
@@ -327,13 +292,13 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs<KT> a) {
       sm[1] = u * u;
     }
     if (ONE) __syncthreads();  // the last sums have been read
-    if (!sums(sm)) return;
+    if (!sums(sm, here)) return;
     if (own) {
       a.U[dof] = u + du;
       if (a.warm) a.warm[dof] = xs;
     }
   }
-  if (blockIdx.x == 0 && t == 0) {
+  if (wg == 0 && t == 0) {
     PcgState* st = &a.host->pcg;
     host_store(&st->bb, bb);
     host_store(&st->rr_last, rr);
@@ -361,7 +326,7 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs<KT> a) {
 // Restarted GMRES(m) with right block-Jacobi preconditioning (K D^-1 y = b,
 // x = D^-1 y), classical Gram-Schmidt twice, as gmres_solve_t in
 // solver_kernels.hip, whose iteration is some ten launches and three host round
-// trips: 157 us at 720 nodes in FP64, and 8.6 us here (289 -> 16.9 ms for the two
+// trips: 157 us at 720 nodes in FP64, and 7.2 us here (289 -> 14.4 ms for the two
 // load steps of a 9 x 8 x 7 box).  A workgroup holds R = T / L rows: the
 // tangent in registers, the basis V of its 3 R dofs and the working vector w in
 // LDS, the Hessenberg column in LDS and its rotations in the lanes of every wave.
@@ -387,10 +352,11 @@ struct GmresArgs {
   const double* b;
   const uint8_t* mask;
   KT* x;
-  KT* tb[2];  // D^-1 w of the even and odd columns, read by the neighbouring workgroups
+  unsigned long long* t;  // D^-1 w, handed from workgroup to workgroup (share_node)
   PcgState* st;
-  unsigned long long* slots;  // two regions of kMaxGridWg slots, used in turn
+  unsigned long long* slots;  // four regions of kMaxGridWg slots
   uint32_t base;
+  int nwg, spread;
   long long limit;
   int64_t nn;
   int m, maxiter;
@@ -406,11 +372,12 @@ inline size_t gmres_lds(int m, int rows, size_t kt) {
          kt * (size_t)(m + 2) * (3 * rows + 4);
 }
 
-template <typename KT, int L, int NB>
+template <typename KT, int L, int NB, Meet M>
 __global__ __launch_bounds__(kGmresThreads) void k_gmres_resident(GmresArgs<KT> a) {
   constexpr int T = kGmresThreads, R = T / L, DN = 3 * R, S = DN + 4;
-  using W = Unwritten<KT>;
-  using Bits = typename W::Bits;
+  constexpr int kSpread = M == Meet::kXcd ? 8 : 1;
+  if (blockIdx.x % kSpread) return;
+  const int wg = (int)(blockIdx.x / kSpread);
   extern __shared__ double lds[];
   __shared__ int late;  // a wait for t or x has expired
   const int m = a.m;
@@ -422,15 +389,22 @@ __global__ __launch_bounds__(kGmresThreads) void k_gmres_resident(GmresArgs<KT> 
   const int t = threadIdx.x;
   const int lane = t & 63;
   const int ph = t % L, lrow = t / L;
-  const int64_t i = (int64_t)blockIdx.x * R + lrow;
+  const int64_t i = (int64_t)wg * R + lrow;
   const bool row = i < a.nn;
   // a thread's dof (t < DN)
   const bool isd = t < DN;
   const int comp = t % 3, n0 = t - comp;
-  const int64_t dof = (int64_t)blockIdx.x * DN + t;
+  const int64_t dof = (int64_t)wg * DN + t;
   const bool live = isd && dof < 3 * a.nn;
   const bool freed = live && !((a.mask[live ? dof / 3 : 0] >> comp) & 1u);
   const double bd = freed ? a.b[dof] : 0.0;
+  // the node that this thread hands over (FP64: a half of it)
+  const int gnode = t / kShareLanes<KT>, gpart = t % kShareLanes<KT>;
+  const uint32_t gi = (uint32_t)(wg * R + gnode);
+  const bool gives = gnode < R && gi < a.nn;
+  KT gd[9];
+#pragma unroll
+  for (int q = 0; q < 9; ++q) gd[q] = gives ? a.Dinv[9 * (int64_t)gi + q] : KT(0);
   KT d0 = 0, d1 = 0, d2 = 0, xs = 0;
   if (live) {
     const KT* D = a.Dinv + 9 * (dof / 3) + 3 * comp;
@@ -449,22 +423,20 @@ __global__ __launch_bounds__(kGmresThreads) void k_gmres_resident(GmresArgs<KT> 
       const int mr = ph + L * q;
       const bool has = row && mr < rounds;
       const int64_t b = b0 + a.rstride * (has ? mr : 0);
-      cj[q] = has ? 3u * (uint32_t)sizeof(KT) * (uint32_t)a.scol[b + l] : 0u;
+      cj[q] = has ? kShareBytes<KT> * (uint32_t)a.scol[b + l] : 0u;
 #pragma unroll
       for (int e = 0; e < 9; ++e) v[q][e] = has ? a.sval[9 * b + 64 * e + l] : KT(0);
     }
   }
   if (t == 0) late = 0;
   __syncthreads();
-  GridSlots gs{a.slots, (int)gridDim.x, &a.st->aborted, a.limit};
-  const uint32_t bytes = 3u * (uint32_t)sizeof(KT) * (uint32_t)a.nn;
+  const GridSlots gs{a.slots, a.nwg, wg, &a.st->aborted, a.limit};
+  const SharedBuf tbuf = shared_buf(a.t, kShareBytes<KT> * (uint32_t)a.nn);
   uint32_t ep = a.base;
-  auto region = [&](uint32_t e) { return a.slots + (size_t)(e & 1u) * kMaxGridWg * kGmresSlot; };
-
-  // w = scale K y, y shared through device memory
-  auto product = [&](const KT* y, double scale) {
+  // w = scale K y, y the vector shared at this epoch
+  auto product = [&](double scale) {
     KT yj[NB][3];
-    if (!gather_published<KT, NB>(shared_buf(y, bytes), cj, gs, yj)) late = 1;
+    if (!gather_shared<M, KT, NB>(tbuf, cj, ep, gs, yj)) late = 1;
     KT a0 = 0, a1 = 0, a2 = 0;
 #pragma unroll
     for (int q = 0; q < NB; ++q) {
@@ -483,33 +455,34 @@ __global__ __launch_bounds__(kGmresThreads) void k_gmres_resident(GmresArgs<KT> 
     __syncthreads();
   };
   // sum over the launch of `nval` values, four threads a value (acc: the thread's
-  // part), to h; the workgroup's earlier stores are complete when a later sum ends
-  auto share = [&](int nval, double acc, double* h) -> bool {
+  // part), to h
+  auto share = [&](int nval, double acc, double* h, auto m) -> bool {
+    constexpr Meet W = decltype(m)::value;
     ++ep;
     const int q = t >> 2, seg = t & 3;
     acc = group_sum<4>(acc);
-    unsigned long long* reg = region(ep);
+    unsigned long long* reg =
+        a.slots + (size_t)((ep & 1u) + (W == Meet::kXcd ? 2u : 0u)) * kMaxGridWg * kGmresSlot;
     bool ok = late == 0;
     double sum = 0;
     if (ok && q < nval) {
       if (seg < 2)
-        agent_store(reg + (size_t)kGmresSlot * blockIdx.x + 2 * q + seg, value_word(acc, ep, seg));
+        shared_store<W>(reg + (size_t)kGmresSlot * wg + 2 * q + seg, value_word(acc, ep, seg));
       const SharedBuf rb = shared_buf(reg, 8u * kGmresSlot * kMaxGridWg);
       for (int g0 = seg; ok && g0 < gs.nwg; g0 += 16) {
-        unsigned long long wd[4][2];
+        double x[4];
         uint32_t off[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          off[e] = 8u * (kGmresSlot * (g0 + 4 * e < gs.nwg ? g0 + 4 * e : blockIdx.x) + 2 * q);
-        ok = poll_values<4>(rb, off, ep, gs, wd);
+          off[e] = 8u * (kGmresSlot * (g0 + 4 * e < gs.nwg ? g0 + 4 * e : wg) + 2 * q);
+        ok = poll_values<W, 4>(rb, off, ep, gs, x);
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          sum += g0 + 4 * e < gs.nwg ? words_value(wd[e][0], wd[e][1]) : 0.0;
+          sum += g0 + 4 * e < gs.nwg ? x[e] : 0.0;
       }
     }
     sum = group_sum<4>(sum);
     if (q < nval && seg == 0) h[q] = sum;
-    stores_done();
     return __syncthreads_and(ok);
   };
   // h[0 .. nv) = V' w, and h[nv] = w' w with NORM
@@ -525,7 +498,7 @@ __global__ __launch_bounds__(kGmresThreads) void k_gmres_resident(GmresArgs<KT> 
         ac2 += (double)vq[d + 4] * (double)w[d + 4];
       }
     }
-    return share(nval, acc + ac2, h);
+    return share(nval, acc + ac2, h, std::integral_constant<Meet, M>());
   };
   auto subtract = [&](int nv, const double* h) {
     if (isd) {
@@ -539,33 +512,41 @@ __global__ __launch_bounds__(kGmresThreads) void k_gmres_resident(GmresArgs<KT> 
   // column j of the basis, w / |w|, and t = D^-1 w of the next product (K D^-1 v is
   // K t / |w|)
   auto next_column = [&](int j, double inv) {
-    if (live)
-      agent_store((Bits*)a.tb[j & 1] + dof,
-                  __builtin_bit_cast(Bits, d0 * w[n0] + d1 * w[n0 + 1] + d2 * w[n0 + 2]));
+    if (gives) {
+      const KT x = w[3 * gnode], y = w[3 * gnode + 1], z = w[3 * gnode + 2];
+      share_node<M>(tbuf, gi, gpart, gd[0] * x + gd[1] * y + gd[2] * z,
+                 gd[3] * x + gd[4] * y + gd[5] * z, gd[6] * x + gd[7] * y + gd[8] * z, ep);
+    }
     if (isd) V[j * S + t] = (KT)((double)w[t] * inv);
   };
-  auto mark = [&](KT* y) {
-    if (live) agent_store((Bits*)y + dof, W::mark);
-  };
+  if (M == Meet::kXcd) {  // one XCD, as in k_pcg_resident: n sum x^2 = (sum x)^2
+    const double x = t < 8 && (t & 3) == 0 ? (double)xcd_id() : 0.0;
+    if (!share(2, t < 4 ? x : x * x, h1, std::integral_constant<Meet, Meet::kDevice>())) return;
+    if (a.nwg * h1[1] != h1[0] * h1[0]) {
+      if (t == 0) a.st->aborted = kNotOneXcd;
+      return;
+    }
+    __syncthreads();
+  }
 
   double beta0 = -1, beta = 0;
   int total = 0;
   for (bool first = true;; first = false) {
     // r = b - K x on the free dofs
     KT rv = freed ? (KT)bd : KT(0);
-    mark(a.tb[0]);
-    mark(a.tb[1]);
     if (!first) {
-      if (live) agent_store(a.x + dof, xs);
-      stores_done();
+      // x at an epoch without a sum (two on, so that the sums' regions stay in turn);
+      // the t that the last column left there is read by no one
+      ep += 2;
+      if (isd) w[t] = xs;
       __syncthreads();
-      if (!share(1, 0.0, h1)) return;  // x is visible (the sum is not used)
-      product(a.x, 1.0);
+      if (gives)
+        share_node<M>(tbuf, gi, gpart, w[3 * gnode], w[3 * gnode + 1], w[3 * gnode + 2], ep);
+      product(1.0);
       rv = freed ? (KT)(bd - (double)w[isd ? t : 0]) : KT(0);
       __syncthreads();
     }
     if (isd) w[t] = rv;
-    stores_done();
     __syncthreads();
     if (!dots(0, h1, true)) return;
     beta = sqrt(h1[0]);
@@ -576,9 +557,8 @@ __global__ __launch_bounds__(kGmresThreads) void k_gmres_resident(GmresArgs<KT> 
     double g = beta, cs = 0, sn = 0;  // lane q of every wave: rotation q
     int k = 0;
     for (int j = 0; j < m; ++j) {
-      product(a.tb[j & 1], inv);
+      product(inv);
       if (!dots(j + 1, h1, false)) return;
-      mark(a.tb[j & 1]);  // every workgroup has read it
       subtract(j + 1, h1);
       if (!dots(j + 1, h2, true)) return;
       subtract(j + 1, h2);
@@ -636,12 +616,8 @@ __global__ __launch_bounds__(kGmresThreads) void k_gmres_resident(GmresArgs<KT> 
     if (live) xs += d0 * w[n0] + d1 * w[n0 + 1] + d2 * w[n0 + 2];
     __syncthreads();
   }
-  if (live) {
-    a.x[dof] = xs;
-    agent_store(a.tb[0] + dof, KT(0));  // no marks are left behind
-    agent_store(a.tb[1] + dof, KT(0));
-  }
-  if (blockIdx.x == 0 && t == 0) {
+  if (live) a.x[dof] = xs;
+  if (wg == 0 && t == 0) {
     a.st->rr_last = beta * beta;
     a.st->bb = beta0 * beta0;
     a.st->iters = total;
@@ -654,13 +630,13 @@ __global__ __launch_bounds__(kGmresThreads) void k_gmres_resident(GmresArgs<KT> 
 // L lanes a row: 4 for rows of up to 16 blocks (structured meshes: 15), 8 up to 32
 inline int lanes_per_row(const Ctx* c) { return c->ell_width <= 16 ? 4 : 8; }
 constexpr int kResidentBlocks = 4;  // blocks a lane keeps in registers
-// Threads a workgroup: few, because a grid exchange waits for the workgroup's own
-// barriers too, but no more workgroups than one poll of the slots covers.  Newton
-// solves of 1,680 / 4,096 / 4,913 nodes (27 / 64 / 77 workgroups of 256) took 14.9 /
-// - / 11.5 ms with 128 threads, 14.8 / 9.7 / 11.6 ms with 256 and 15.5 / 10.2 /
-// 10.9 ms with 512 (FP64, 2,080 nodes: 3.8 / 3.6 / 3.7 ms), against 49.6 ms on two
-// kernels an iteration.  The single workgroup gathers from LDS: 512 threads, and in
-// FP32 1024 where the rows need them (125 nodes: 1.8 us an iteration against 2.6).
+// Threads a workgroup: few, because an exchange waits for the workgroup's own barriers
+// too.  Newton solves of 1,680 / 4,096 nodes took 14.9 / - ms with 128 threads, 14.8 /
+// 9.7 ms with 256 and 15.5 / 10.2 ms with 512 across the device, against 49.6 ms on two
+// kernels an iteration; of 4,913 / 6,859 / 8,000 nodes 9.4 / 12.9 / 13.7 ms with 256 (the
+// first in one XCD) and 13.6 / 13.8 / 15.7 ms with 512, which are left for more than
+// kMaxGridWg workgroups of 256.  The single workgroup gathers from LDS: 512 threads, and
+// in FP32 1024 where the rows need them (125 nodes: 1.8 us an iteration against 2.6).
 constexpr int kResidentThreads = 256;
 constexpr int resident_one_threads(size_t kt) { return kt == 4 ? 1024 : 512; }
 
@@ -673,26 +649,40 @@ inline ResidentShape resident_shape(const Ctx* c) {
   if (lanes <= 512) return {512, 1};
   if (lanes <= resident_one_threads(c->kt)) return {resident_one_threads(c->kt), 1};
   int t = kResidentThreads;
-  if ((lanes + t - 1) / t > kPollSlots) t *= 2;
+  if ((lanes + t - 1) / t > kMaxGridWg) t *= 2;
   return {t, (lanes + t - 1) / t};
 }
+
+// Every 8th workgroup of a launch shares an XCD: 32 CUs, on which 64 workgroups of 256
+// threads are resident together with two waves a SIMD, and 96 with three.  That many
+// do better there, met in its L2, than spread over the device: FP32 1,680 / 4,096 /
+// 5,832 nodes 10.3 / 7.6 / 9.8 ms against 14.1 / 9.6 / 12.6 ms, FP64 2,080 / 3,375
+// nodes 2.8 / 9.4 ms against 3.8 / 11.2 ms, GMRES at 720 nodes 14.4 ms against 17.3 ms.
+inline bool on_one_xcd(const Ctx* c, int64_t grid, int waves) {
+  return c->one_xcd && grid <= 32 * waves;
+}
+inline size_t share_words(const Ctx* c) { return (size_t)c->nn * c->kt / 2; }  // kShareBytes a node
 
 // A Newton step's launch stamps the step's timing events.
 template <typename KT, int L>
 void run_resident(Ctx* c, const ResidentArgs<KT>& a, const ResidentShape& sh) {
   constexpr int T1 = resident_one_threads(sizeof(KT)), T = kResidentThreads;
+  constexpr int NB = kResidentBlocks;
+  constexpr Meet D = Meet::kDevice, X = Meet::kXcd;
   const hipEvent_t e0 = a.fint ? c->ev[4] : nullptr, e1 = a.fint ? c->ev[7] : nullptr;
-  auto go = [&](auto kern, int threads) {
-    hipExtLaunchKernelGGL(kern, dim3((unsigned)sh.grid), dim3(threads), 0, c->stream, e0, e1, 0, a);
+  auto go = [&](auto kern, int threads, int64_t grid) {
+    hipExtLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(threads), 0, c->stream, e0, e1, 0, a);
   };
   if (sh.grid == 1 && sh.threads == 512)
-    go(k_pcg_resident<KT, L, kResidentBlocks, 512, true>, 512);
+    go(k_pcg_resident<KT, L, NB, 512, true, D>, 512, 1);
   else if (sh.grid == 1)
-    go(k_pcg_resident<KT, L, kResidentBlocks, T1, true>, T1);
+    go(k_pcg_resident<KT, L, NB, T1, true, D>, T1, 1);
+  else if (sh.threads == T && on_one_xcd(c, sh.grid, xcd_waves(sizeof(KT))))
+    go(k_pcg_resident<KT, L, NB, T, false, X>, T, 8 * sh.grid);
   else if (sh.threads == T)
-    go(k_pcg_resident<KT, L, kResidentBlocks, T, false>, T);
+    go(k_pcg_resident<KT, L, NB, T, false, D>, T, sh.grid);
   else
-    go(k_pcg_resident<KT, L, kResidentBlocks, 2 * T, false>, 2 * T);
+    go(k_pcg_resident<KT, L, NB, 2 * T, false, D>, 2 * T, sh.grid);
 }
 
 template <typename KT>
@@ -707,8 +697,7 @@ int resident_t(Ctx* c, const double* b, const double* fint, const void* x0, void
   a.mask = c->d_fixmask;
   a.b = b;
   a.x = (KT*)c->d_px;
-  a.zb[0] = (KT*)c->d_pp0;
-  a.zb[1] = (KT*)c->d_pp1;
+  a.z = c->d_share;
   a.sc = c->d_sc;
   a.host = c->h_sc;
   a.slots = c->d_gslots;
@@ -723,6 +712,7 @@ int resident_t(Ctx* c, const double* b, const double* fint, const void* x0, void
   a.limit = c->gslot_ticks;
   a.nn = c->nn;
   const ResidentShape sh = resident_shape(c);
+  a.nwg = (int)sh.grid;
   if (lanes_per_row(c) == 4)
     run_resident<KT, 4>(c, a, sh);
   else
@@ -743,8 +733,7 @@ int gmres_t(Ctx* c, const double* b_dev, int m, int maxiter, double rtol) {
   a.b = b_dev;
   a.mask = c->d_fixmask;
   a.x = (KT*)c->d_px;
-  a.tb[0] = (KT*)c->d_pp0;
-  a.tb[1] = (KT*)c->d_pp1;
+  a.t = c->d_share;
   a.st = &c->d_sc->pcg;
   a.slots = c->d_gmslots;
   a.base = c->gslot_epoch;
@@ -753,13 +742,21 @@ int gmres_t(Ctx* c, const double* b_dev, int m, int maxiter, double rtol) {
   a.m = m;
   a.maxiter = maxiter;
   a.rtol = rtol;
-  auto kern = k_gmres_resident<KT, L, kResidentBlocks>;
-  const size_t lds = gmres_lds(m, kGmresThreads / L, sizeof(KT));
-  ONSAS_HIP_TRY(c, hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   const int R = kGmresThreads / L;
-  hipLaunchKernelGGL(kern, dim3((unsigned)((c->nn + R - 1) / R)), dim3(kGmresThreads), lds,
-                     c->stream, a);
+  const int64_t grid = (c->nn + R - 1) / R;
+  a.nwg = (int)grid;
+  const size_t lds = gmres_lds(m, R, sizeof(KT));
+  auto go = [&](auto kern, int64_t n) -> int {
+    ONSAS_HIP_TRY(c, hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(kern, dim3((unsigned)n), dim3(kGmresThreads), lds, c->stream, a);
+    return ONSAS_OK;
+  };
+  // two workgroups a CU where the LDS holds two
+  if (on_one_xcd(c, grid, lds <= 78 * 1024 ? 2 : 1))
+    ONSAS_TRY(go(k_gmres_resident<KT, L, kResidentBlocks, Meet::kXcd>, 8 * grid));
+  else
+    ONSAS_TRY(go(k_gmres_resident<KT, L, kResidentBlocks, Meet::kDevice>, grid));
   ONSAS_HIP_TRY(c, hipGetLastError());
   return ONSAS_OK;
 }
@@ -774,19 +771,27 @@ bool pcg_resident_fits(const Ctx* c) {
          resident_shape(c).grid <= kMaxGridWg;
 }
 
-void pcg_resident_setup(Ctx* c) {
+int pcg_resident_setup(Ctx* c) {
   const char* e = std::getenv("ONSAS_PCG_RESIDENT");
   c->pcg_resident = pcg_resident_fits(c) && !(e && e[0] == '0');
+  if (const char* x = std::getenv("ONSAS_RESIDENT_XCD")) c->one_xcd = x[0] != '0';
   if (const char* t = std::getenv("ONSAS_RESIDENT_TICKS")) c->gslot_ticks = std::atoll(t);
+  if (!c->pcg_resident) return ONSAS_OK;
+  const size_t bytes = share_words(c) * sizeof(unsigned long long);
+  ONSAS_HIP_TRY(c, hipMalloc((void**)&c->d_share, bytes));
+  ONSAS_HIP_TRY(c, hipMemset(c->d_share, 0, bytes));
+  return ONSAS_OK;
 }
 
-// before the epochs wrap: clear the slots' marks and begin again
+// before the epochs wrap: clear the marks and begin again
 static int renew_epochs(Ctx* c) {
   if (c->gslot_epoch <= 0xf0000000u) return ONSAS_OK;
   ONSAS_HIP_TRY(c, hipMemsetAsync(c->d_gslots, 0,
                                   kGridSlotWords * sizeof(unsigned long long), c->stream));
+  ONSAS_HIP_TRY(c, hipMemsetAsync(c->d_share, 0, share_words(c) * sizeof(unsigned long long),
+                                  c->stream));
   if (c->d_gmslots)
-    ONSAS_HIP_TRY(c, hipMemsetAsync(c->d_gmslots, 0, 2 * (size_t)kMaxGridWg * kGmresSlot *
+    ONSAS_HIP_TRY(c, hipMemsetAsync(c->d_gmslots, 0, 4 * (size_t)kMaxGridWg * kGmresSlot *
                                                          sizeof(unsigned long long), c->stream));
   c->gslot_epoch = 1;
   return ONSAS_OK;
@@ -804,12 +809,15 @@ static int resident_run(Ctx* c, const double* b, const double* fint, const void*
                                                  : resident_t<float>(c, b, fint, x0, warm));
   ONSAS_HIP_TRY(c, hipStreamSynchronize(s));
   const PcgState& ps = c->h_sc->pcg;
+  if (ps.aborted == kNotOneXcd) {  // before anything was done
+    c->one_xcd = false;
+    c->gslot_epoch += 2;
+    return resident_run(c, b, fint, x0, warm, ran, iters, relres, converged, breakdown);
+  }
   *ran = ps.done && !ps.aborted;
-  c->gslot_epoch += (*ran ? (uint32_t)ps.k : (uint32_t)pcg_maxiter(c)) + 4;
+  c->gslot_epoch += (*ran ? (uint32_t)ps.k : (uint32_t)pcg_maxiter(c)) + 5;
   if (!*ran) {
     c->pcg_resident = false;
-    for (void* v : {c->d_pp0, c->d_pp1})  // the launch may have left its marks there
-      ONSAS_HIP_TRY(c, hipMemsetAsync(v, 0, c->kt * 3 * (size_t)c->nn, s));
     return ONSAS_OK;
   }
   pcg_result(ps, iters, relres, converged, breakdown);
@@ -856,7 +864,7 @@ int launch_gmres_resident(Ctx* c, const double* b_dev, int m, int maxiter, doubl
       (c->nn + R - 1) / R > kMaxGridWg || gmres_lds(m, R, c->kt) > 150 * 1024)
     return ONSAS_OK;
   hipStream_t s = c->stream;
-  const size_t bytes = 2 * (size_t)kMaxGridWg * kGmresSlot * sizeof(unsigned long long);
+  const size_t bytes = 4 * (size_t)kMaxGridWg * kGmresSlot * sizeof(unsigned long long);
   if (!c->d_gmslots) {
     ONSAS_HIP_TRY(c, hipMalloc((void**)&c->d_gmslots, bytes));
     ONSAS_HIP_TRY(c, hipMemsetAsync(c->d_gmslots, 0, bytes, s));
@@ -873,12 +881,15 @@ int launch_gmres_resident(Ctx* c, const double* b_dev, int m, int maxiter, doubl
                                   hipMemcpyDeviceToHost, s));
   ONSAS_HIP_TRY(c, hipStreamSynchronize(s));
   const PcgState& ps = c->h_sc->pcg;
-  // an iteration takes at most 3 epochs, a restart 2
-  c->gslot_epoch += (ps.aborted ? 5u * ((uint32_t)maxiter + 2) : (uint32_t)ps.k) + 2;
+  if (ps.aborted == kNotOneXcd) {  // before anything was done
+    c->one_xcd = false;
+    c->gslot_epoch += 2;
+    return launch_gmres_resident(c, b_dev, m, maxiter, rtol, ran, iters, relres, converged);
+  }
+  // an iteration takes at most 3 epochs, a restart 3
+  c->gslot_epoch += (ps.aborted ? 6u * ((uint32_t)maxiter + 2) : (uint32_t)ps.k) + 4;
   if (ps.aborted) {
     c->pcg_resident = false;
-    for (void* v : {c->d_pp0, c->d_pp1})  // the launch may have left its marks there
-      ONSAS_HIP_TRY(c, hipMemsetAsync(v, 0, c->kt * 3 * (size_t)c->nn, s));
     return ONSAS_OK;
   }
   *ran = true;

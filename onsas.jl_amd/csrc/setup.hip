@@ -494,7 +494,7 @@ int finalize_model(Ctx* c) {
     ONSAS_TRY(dev_upload(c, &c->d_sell_col, scol.data(), scol.size()));
     ONSAS_TRY(dev_alloc(c, &c->d_Ksell, c->kt * 9 * (size_t)c->nsell));
   }
-  pcg_resident_setup(c);
+  ONSAS_TRY(pcg_resident_setup(c));
   if (c->gather) ONSAS_TRY(build_gather(c, slots_h, rstride));
 
   if (c->gather) ONSAS_TRY(launch_gather_init(c));

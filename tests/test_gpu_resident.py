@@ -207,3 +207,23 @@ def test_resident_newton_expired_wait(monkeypatch, prec):
     for a, b in zip(log, logg):
         assert _stat(a, "r_norm") == _stat(b, "r_norm")
         assert _stat(a, "lin_iters") == _stat(b, "lin_iters")
+
+
+@pytest.mark.parametrize("kind", [_capi.LINSOLVE_PCG, _capi.LINSOLVE_GMRES])
+@pytest.mark.parametrize("prec", [_capi.PRECISION_MIXED, _capi.PRECISION_FP64])
+@pytest.mark.parametrize("model", ["8x6x3", "10x10x10", "16x15x15", "21x20x19"])
+def test_resident_across_the_device(monkeypatch, model, prec, kind):
+    """The same solves by workgroups that meet in device memory, not in one XCD's L2
+    (the only way of the largest model, whose workgroups one XCD does not hold)."""
+    print(f"[gpu] resident solver {kind} {model} precision {prec}, across the device", flush=True)
+    rtol = 1e-3 if prec == _capi.PRECISION_MIXED else 1e-10
+    if kind == _capi.LINSOLVE_GMRES:
+        if model in ("16x15x15", "21x20x19"):
+            pytest.skip("a restarted GMRES of this size stagnates on either path")
+        rtol = max(rtol, 1e-9)
+    it, res, bound = _solve(MODELS[model], prec, rtol, kind)
+    assert res <= bound
+    monkeypatch.setenv("ONSAS_RESIDENT_XCD", "0")
+    itd, resd, bound = _solve(MODELS[model], prec, rtol, kind)
+    assert resd <= bound
+    assert abs(it - itd) <= 2 + itd // 20
