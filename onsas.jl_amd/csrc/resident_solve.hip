@@ -21,6 +21,9 @@
 // with p.q and (r.z, r.r) as two sums, z safe to read only after the second, a tree per
 // sum and 4- and 8-byte loads it was 4.6 and 2.6 us.  Polling by every wave of a
 // workgroup instead of one costs 1 us.
+#include <unistd.h>
+
+#include <atomic>
 #include <cmath>
 #include <cstdlib>
 #include <type_traits>
@@ -50,7 +53,7 @@ struct ResidentArgs {
   Scalars* host;       // pinned host: the results
   unsigned long long* slots;  // four regions of 8 words per workgroup
   uint32_t base;              // epochs base + 1, base + 2, ... are new to the slots and z
-  int nwg;                    // workgroups (of kXcd launches every 8th)
+  int nwg, xcd;               // workgroups; of kXcd launches every 8th, from xcd on
   long long limit;
   int64_t nn;
   int maxiter;
@@ -90,13 +93,14 @@ constexpr int xcd_waves(size_t kt) { return kt == 4 ? 3 : 2; }
 // another still reads sum k.  z has one buffer: the sum before its next hand-over is
 // complete only when every workgroup has made its product.
 //
-// kXcd: every 8th workgroup takes part.  Consecutive workgroups go round the 8 XCDs, so
+// kXcd: every 8th workgroup takes part, from the context's own first one on (contexts
+// that solve at the same time would hold each other's places on a shared XCD).  Consecutive workgroups go round the 8 XCDs, so
 // these share one, which a first sum across the device confirms (if not, nothing has
 // been done and the host launches the other kernel); they then meet in its L2.
 template <typename KT, int L, int NB, int T, bool ONE, Meet M>
 __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs<KT> a) {
   constexpr int kSpread = M == Meet::kXcd ? 8 : 1;
-  if (blockIdx.x % kSpread) return;
+  if (M == Meet::kXcd && (int)(blockIdx.x % kSpread) != a.xcd) return;
   const int wg = (int)(blockIdx.x / kSpread);
   __shared__ double sh[4 * (T / 64) + 5];
   __shared__ __align__(16) KT shz[ONE ? 4 * (T / L) : 4];  // a node's z and a pad: 16-byte reads
@@ -356,7 +360,7 @@ struct GmresArgs {
   PcgState* st;
   unsigned long long* slots;  // four regions of kMaxGridWg slots
   uint32_t base;
-  int nwg, spread;
+  int nwg, xcd;
   long long limit;
   int64_t nn;
   int m, maxiter;
@@ -376,7 +380,7 @@ template <typename KT, int L, int NB, Meet M>
 __global__ __launch_bounds__(kGmresThreads) void k_gmres_resident(GmresArgs<KT> a) {
   constexpr int T = kGmresThreads, R = T / L, DN = 3 * R, S = DN + 4;
   constexpr int kSpread = M == Meet::kXcd ? 8 : 1;
-  if (blockIdx.x % kSpread) return;
+  if (M == Meet::kXcd && (int)(blockIdx.x % kSpread) != a.xcd) return;
   const int wg = (int)(blockIdx.x / kSpread);
   extern __shared__ double lds[];
   __shared__ int late;  // a wait for t or x has expired
@@ -665,7 +669,7 @@ inline size_t share_words(const Ctx* c) { return (size_t)c->nn * c->kt / 2; }  /
 
 // A Newton step's launch stamps the step's timing events.
 template <typename KT, int L>
-void run_resident(Ctx* c, const ResidentArgs<KT>& a, const ResidentShape& sh) {
+void run_resident(Ctx* c, const ResidentArgs<KT>& a, const ResidentShape& sh, bool xcd) {
   constexpr int T1 = resident_one_threads(sizeof(KT)), T = kResidentThreads;
   constexpr int NB = kResidentBlocks;
   constexpr Meet D = Meet::kDevice, X = Meet::kXcd;
@@ -677,7 +681,7 @@ void run_resident(Ctx* c, const ResidentArgs<KT>& a, const ResidentShape& sh) {
     go(k_pcg_resident<KT, L, NB, 512, true, D>, 512, 1);
   else if (sh.grid == 1)
     go(k_pcg_resident<KT, L, NB, T1, true, D>, T1, 1);
-  else if (sh.threads == T && on_one_xcd(c, sh.grid, xcd_waves(sizeof(KT))))
+  else if (xcd)
     go(k_pcg_resident<KT, L, NB, T, false, X>, T, 8 * sh.grid);
   else if (sh.threads == T)
     go(k_pcg_resident<KT, L, NB, T, false, D>, T, sh.grid);
@@ -686,7 +690,7 @@ void run_resident(Ctx* c, const ResidentArgs<KT>& a, const ResidentShape& sh) {
 }
 
 template <typename KT>
-int resident_t(Ctx* c, const double* b, const double* fint, const void* x0, void* warm) {
+int resident_t(Ctx* c, const double* b, const double* fint, const void* x0, void* warm, bool* xcd) {
   ResidentArgs<KT> a{};
   a.sell_ptr = c->d_sell_ptr;
   a.slice_rounds = c->d_slice_rounds;
@@ -712,17 +716,19 @@ int resident_t(Ctx* c, const double* b, const double* fint, const void* x0, void
   a.limit = c->gslot_ticks;
   a.nn = c->nn;
   const ResidentShape sh = resident_shape(c);
+  *xcd = sh.grid > 1 && sh.threads == kResidentThreads && on_one_xcd(c, sh.grid, xcd_waves(c->kt));
   a.nwg = (int)sh.grid;
+  a.xcd = c->xcd;
   if (lanes_per_row(c) == 4)
-    run_resident<KT, 4>(c, a, sh);
+    run_resident<KT, 4>(c, a, sh, *xcd);
   else
-    run_resident<KT, 8>(c, a, sh);
+    run_resident<KT, 8>(c, a, sh, *xcd);
   ONSAS_HIP_TRY(c, hipGetLastError());
   return ONSAS_OK;
 }
 
 template <typename KT, int L>
-int gmres_t(Ctx* c, const double* b_dev, int m, int maxiter, double rtol) {
+int gmres_t(Ctx* c, const double* b_dev, int m, int maxiter, double rtol, bool* xcd) {
   GmresArgs<KT> a{};
   a.sell_ptr = c->d_sell_ptr;
   a.slice_rounds = c->d_slice_rounds;
@@ -745,6 +751,7 @@ int gmres_t(Ctx* c, const double* b_dev, int m, int maxiter, double rtol) {
   const int R = kGmresThreads / L;
   const int64_t grid = (c->nn + R - 1) / R;
   a.nwg = (int)grid;
+  a.xcd = c->xcd;
   const size_t lds = gmres_lds(m, R, sizeof(KT));
   auto go = [&](auto kern, int64_t n) -> int {
     ONSAS_HIP_TRY(c, hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -753,7 +760,8 @@ int gmres_t(Ctx* c, const double* b_dev, int m, int maxiter, double rtol) {
     return ONSAS_OK;
   };
   // two workgroups a CU where the LDS holds two
-  if (on_one_xcd(c, grid, lds <= 78 * 1024 ? 2 : 1))
+  *xcd = on_one_xcd(c, grid, lds <= 78 * 1024 ? 2 : 1);
+  if (*xcd)
     ONSAS_TRY(go(k_gmres_resident<KT, L, kResidentBlocks, Meet::kXcd>, 8 * grid));
   else
     ONSAS_TRY(go(k_gmres_resident<KT, L, kResidentBlocks, Meet::kDevice>, grid));
@@ -776,10 +784,18 @@ int pcg_resident_setup(Ctx* c) {
   c->pcg_resident = pcg_resident_fits(c) && !(e && e[0] == '0');
   if (const char* x = std::getenv("ONSAS_RESIDENT_XCD")) c->one_xcd = x[0] != '0';
   if (const char* t = std::getenv("ONSAS_RESIDENT_TICKS")) c->gslot_ticks = std::atoll(t);
+  static std::atomic<unsigned> contexts{0};
+  c->xcd = (int)((contexts++ + (unsigned)getpid()) % 8);
   if (!c->pcg_resident) return ONSAS_OK;
   const size_t bytes = share_words(c) * sizeof(unsigned long long);
   ONSAS_HIP_TRY(c, hipMalloc((void**)&c->d_share, bytes));
   ONSAS_HIP_TRY(c, hipMemset(c->d_share, 0, bytes));
+  return ONSAS_OK;
+}
+
+// the abort word of a launch that gave up
+static int clear_abort(Ctx* c) {
+  ONSAS_HIP_TRY(c, hipMemsetAsync(&c->d_sc->pcg.aborted, 0, sizeof(int32_t), c->stream));
   return ONSAS_OK;
 }
 
@@ -797,31 +813,34 @@ static int renew_epochs(Ctx* c) {
   return ONSAS_OK;
 }
 
-// Launches, waits and takes the results; *ran = false once a wait has expired (the
-// GPU was too busy to hold the whole grid): the context keeps to the general
-// kernels from then on.
+// A launch that gave up (a wait expired: the GPU, or the XCD, was too busy to hold the
+// whole grid) or found its workgroups on several XCDs: the next one meets across the
+// device, and after that the context keeps to the general kernels.
+static void resident_failed(Ctx* c, bool xcd) {
+  if (xcd)
+    c->one_xcd = false;
+  else
+    c->pcg_resident = false;
+}
+
+// Launches, waits and takes the results; *ran = false if the launch gave up.
 static int resident_run(Ctx* c, const double* b, const double* fint, const void* x0, void* warm,
                         bool* ran, int* iters, double* relres, int* converged, int* breakdown) {
-  hipStream_t s = c->stream;
   ONSAS_TRY(renew_epochs(c));
   c->h_sc->pcg = PcgState{};
-  ONSAS_TRY(c->precision == ONSAS_PRECISION_FP64 ? resident_t<double>(c, b, fint, x0, warm)
-                                                 : resident_t<float>(c, b, fint, x0, warm));
-  ONSAS_HIP_TRY(c, hipStreamSynchronize(s));
+  bool xcd = false;
+  ONSAS_TRY(c->precision == ONSAS_PRECISION_FP64 ? resident_t<double>(c, b, fint, x0, warm, &xcd)
+                                                 : resident_t<float>(c, b, fint, x0, warm, &xcd));
+  ONSAS_HIP_TRY(c, hipStreamSynchronize(c->stream));
   const PcgState& ps = c->h_sc->pcg;
-  if (ps.aborted == kNotOneXcd) {  // before anything was done
-    c->one_xcd = false;
-    c->gslot_epoch += 2;
-    return resident_run(c, b, fint, x0, warm, ran, iters, relres, converged, breakdown);
-  }
   *ran = ps.done && !ps.aborted;
   c->gslot_epoch += (*ran ? (uint32_t)ps.k : (uint32_t)pcg_maxiter(c)) + 5;
-  if (!*ran) {
-    c->pcg_resident = false;
+  if (*ran) {
+    pcg_result(ps, iters, relres, converged, breakdown);
     return ONSAS_OK;
   }
-  pcg_result(ps, iters, relres, converged, breakdown);
-  return ONSAS_OK;
+  resident_failed(c, xcd);
+  return clear_abort(c);
 }
 
 inline bool pcg_resident_now(const Ctx* c) {
@@ -832,18 +851,21 @@ inline bool pcg_resident_now(const Ctx* c) {
 int launch_pcg_resident(Ctx* c, const double* b_dev, bool* ran, int* iters, double* relres,
                         int* converged, int* breakdown) {
   *ran = false;
-  if (!pcg_resident_now(c)) return ONSAS_OK;
-  return resident_run(c, b_dev, nullptr, nullptr, nullptr, ran, iters, relres, converged, breakdown);
+  while (!*ran && pcg_resident_now(c))
+    ONSAS_TRY(resident_run(c, b_dev, nullptr, nullptr, nullptr, ran, iters, relres, converged,
+                           breakdown));
+  return ONSAS_OK;
 }
 
 int launch_newton_resident(Ctx* c, const void* x0, void* warm, bool* ran, int* iters,
                            double* relres, int* converged, int* breakdown) {
   *ran = false;
-  if (!pcg_resident_now(c) || c->lin.kind == ONSAS_LINSOLVE_GMRES) return ONSAS_OK;
-  const double prev_b2 = c->h_sc->nwt.prev_b2;
-  ONSAS_TRY(resident_run(c, c->d_fext, c->d_fint, x0, warm, ran, iters, relres, converged,
-                         breakdown));
-  if (!*ran) {  // U and the forcing's memory as they were (some workgroups may have got that far)
+  while (!*ran && pcg_resident_now(c) && c->lin.kind != ONSAS_LINSOLVE_GMRES) {
+    const double prev_b2 = c->h_sc->nwt.prev_b2;
+    ONSAS_TRY(resident_run(c, c->d_fext, c->d_fint, x0, warm, ran, iters, relres, converged,
+                           breakdown));
+    if (*ran) break;
+    // U and the forcing's memory as they were (some workgroups may have got that far)
     ONSAS_HIP_TRY(c, hipMemcpyAsync(c->d_U, c->d_Uasm, 3 * c->nn * sizeof(double),
                                     hipMemcpyDeviceToDevice, c->stream));
     c->h_sc->nwt.prev_b2 = prev_b2;
@@ -871,26 +893,23 @@ int launch_gmres_resident(Ctx* c, const double* b_dev, int m, int maxiter, doubl
   }
   ONSAS_TRY(renew_epochs(c));
   ONSAS_HIP_TRY(c, hipMemsetAsync(&c->d_sc->pcg, 0, sizeof(PcgState), s));
+  bool xcd = false;
   if (c->precision == ONSAS_PRECISION_FP64)
-    ONSAS_TRY(L == 4 ? (gmres_t<double, 4>(c, b_dev, m, maxiter, rtol))
-                     : (gmres_t<double, 8>(c, b_dev, m, maxiter, rtol)));
+    ONSAS_TRY(L == 4 ? (gmres_t<double, 4>(c, b_dev, m, maxiter, rtol, &xcd))
+                     : (gmres_t<double, 8>(c, b_dev, m, maxiter, rtol, &xcd)));
   else
-    ONSAS_TRY(L == 4 ? (gmres_t<float, 4>(c, b_dev, m, maxiter, rtol))
-                     : (gmres_t<float, 8>(c, b_dev, m, maxiter, rtol)));
+    ONSAS_TRY(L == 4 ? (gmres_t<float, 4>(c, b_dev, m, maxiter, rtol, &xcd))
+                     : (gmres_t<float, 8>(c, b_dev, m, maxiter, rtol, &xcd)));
   ONSAS_HIP_TRY(c, hipMemcpyAsync(&c->h_sc->pcg, &c->d_sc->pcg, sizeof(PcgState),
                                   hipMemcpyDeviceToHost, s));
   ONSAS_HIP_TRY(c, hipStreamSynchronize(s));
   const PcgState& ps = c->h_sc->pcg;
-  if (ps.aborted == kNotOneXcd) {  // before anything was done
-    c->one_xcd = false;
-    c->gslot_epoch += 2;
-    return launch_gmres_resident(c, b_dev, m, maxiter, rtol, ran, iters, relres, converged);
-  }
   // an iteration takes at most 3 epochs, a restart 3
   c->gslot_epoch += (ps.aborted ? 6u * ((uint32_t)maxiter + 2) : (uint32_t)ps.k) + 4;
   if (ps.aborted) {
-    c->pcg_resident = false;
-    return ONSAS_OK;
+    resident_failed(c, xcd);
+    ONSAS_TRY(clear_abort(c));
+    return launch_gmres_resident(c, b_dev, m, maxiter, rtol, ran, iters, relres, converged);
   }
   *ran = true;
   *iters = ps.iters;

@@ -227,3 +227,17 @@ def test_resident_across_the_device(monkeypatch, model, prec, kind):
     itd, resd, bound = _solve(MODELS[model], prec, rtol, kind)
     assert resd <= bound
     assert abs(it - itd) <= 2 + itd // 20
+
+
+def test_resident_contexts_at_the_same_time():
+    """Ten contexts solving on threads of their own (more than there are XCDs): whichever
+    way a solve ends up taking, it meets its bound."""
+    from concurrent.futures import ThreadPoolExecutor
+    print("[gpu] resident solves of ten contexts at a time", flush=True)
+    kinds = [(_capi.PRECISION_FP64, 1e-10), (_capi.PRECISION_MIXED, 1e-3)]
+    with ThreadPoolExecutor(10) as pool:
+        runs = [pool.submit(_solve, MODELS["16x15x15" if i % 3 else "10x10x10"], *kinds[i % 2])
+                for i in range(10)]
+        for f in runs:
+            _, res, bound = f.result()
+            assert res <= bound
