@@ -383,7 +383,7 @@ struct Ctx {
   int gm_m = 0;
 
   // timers
-  hipEvent_t ev[10] = {};  // 0/3 assembly, 1/8/2 element+gather passes, 4..7 Newton step
+  hipEvent_t ev[10] = {};  // 0/3 scatter assembly, 1/8/2 its passes or the gather's, 4..7 Newton step
   hipEvent_t ev_spmv[2 * 32] = {};  // brackets of the sampled SpMV launches
   onsas_timings tm{};
   double last_assemble_ms = 0;
