@@ -1270,24 +1270,57 @@ __global__ __launch_bounds__(256) void k_dense_apply(const KT* __restrict__ Ainv
   if (l == 0) x[r] = s;
 }
 
-// partial sums of v.v (power iteration), grid-stride, one partial per block
+// Power iteration, the norms' part: partial sums of w.w and, 256 on, of v.v, one a
+// block (256 blocks).
 template <typename KT>
-__global__ __launch_bounds__(256) void k_norm2(const KT* __restrict__ v, int64_t n,
-                                               double* __restrict__ part) {
-  __shared__ double sh[4];
-  double s = 0;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
-    s += (double)v[i] * (double)v[i];
+__global__ __launch_bounds__(256) void k_power_norms(const KT* __restrict__ w,
+                                                     const KT* __restrict__ v, int64_t n,
+                                                     double* __restrict__ part) {
+  __shared__ double sh[8];
+  double s = 0, t = 0;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+    s += (double)w[i] * (double)w[i];
+    t += (double)v[i] * (double)v[i];
+  }
   s = wave_sum(s);
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+  t = wave_sum(t);
+  if ((threadIdx.x & 63) == 0) {
+    sh[threadIdx.x >> 6] = s;
+    sh[4 + (threadIdx.x >> 6)] = t;
+  }
   __syncthreads();
-  if (threadIdx.x == 0) part[blockIdx.x] = sh[0] + sh[1] + sh[2] + sh[3];
+  if (threadIdx.x == 0) {
+    part[blockIdx.x] = sh[0] + sh[1] + sh[2] + sh[3];
+    part[256 + blockIdx.x] = sh[4] + sh[5] + sh[6] + sh[7];
+  }
 }
 
-// v = a w
+// ... and the step's: lambda = |w| / |v| and v = w / |w|; nothing where a norm is zero
+// or not a number (and then not in the steps after it either; `before` is the estimate
+// that stays, from the first step's launch).  Every block sums the partials for itself,
+// so that the host does not wait for the norms in between (55 us a step).
 template <typename KT>
-__global__ void k_scaled_copy(const KT* __restrict__ w, KT* __restrict__ v, int64_t n, KT a) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(256) void k_power_step(const KT* __restrict__ w, KT* __restrict__ v,
+                                                    int64_t n, const double* __restrict__ part,
+                                                    double* __restrict__ lam, double before) {
+  __shared__ double sh[8];
+  const double s = wave_sum(part[threadIdx.x]), t = wave_sum(part[256 + threadIdx.x]);
+  if ((threadIdx.x & 63) == 0) {
+    sh[threadIdx.x >> 6] = s;
+    sh[4 + (threadIdx.x >> 6)] = t;
+  }
+  __syncthreads();
+  const double nw = sh[0] + sh[1] + sh[2] + sh[3], nv = sh[4] + sh[5] + sh[6] + sh[7];
+  const bool ok = nw > 0 && nv > 0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (ok)
+      *lam = sqrt(nw / nv);
+    else if (before > 0)
+      *lam = before;
+  }
+  if (!ok) return;
+  const KT a = (KT)(1.0 / sqrt(nw));
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i < n) v[i] = a * w[i];
 }
 
@@ -1640,8 +1673,8 @@ void op_cheb(Ctx* c, int l, const KT* v, const KT* b, KT* r_out, double c1, doub
   }
 }
 
-// lambda_max(D^-1 A) of level l by power iteration (host-driven), from a hashed
-// start vector or from the last iterate
+// lambda_max(D^-1 A) of level l by power iteration, from a hashed start vector or
+// from the last iterate; the host waits once, for the estimate
 template <typename KT>
 int estimate_lambda(Ctx* c, int l, int iters, bool fresh) {
   Amg& A = c->amg;
@@ -1650,29 +1683,21 @@ int estimate_lambda(Ctx* c, int l, int iters, bool fresh) {
   const int64_t nd = (int64_t)L.bs * L.n;
   KT* v = (KT*)L.d_ev;
   KT* w = (KT*)L.d_d1;
+  double* lam = A.d_part + 512;
   if (fresh)
     hipLaunchKernelGGL(k_fill_hash<KT>, dim3(nblocks(nd, 256)), dim3(256), 0, s, v, nd,
                        l == 0 ? c->d_fixmask : nullptr, L.bs);
-  std::vector<double> h(512);
-  double lam = L.lam > 0 ? L.lam : 1.0;
   for (int it = 0; it < iters; ++it) {
     op_cheb<KT>(c, l, v, nullptr, nullptr, 0.0, 1.0, w, nullptr, nullptr, nullptr);  // w = -D^-1 A v
-    hipLaunchKernelGGL(k_norm2<KT>, dim3(256), dim3(256), 0, s, w, nd, A.d_part);
-    hipLaunchKernelGGL(k_norm2<KT>, dim3(256), dim3(256), 0, s, v, nd, A.d_part + 256);
-    ONSAS_HIP_TRY(c, hipMemcpyAsync(h.data(), A.d_part, 512 * sizeof(double), hipMemcpyDeviceToHost, s));
-    ONSAS_HIP_TRY(c, hipStreamSynchronize(s));
-    double nw = 0, nv = 0;
-    for (int k = 0; k < 256; ++k) {
-      nw += h[k];
-      nv += h[256 + k];
-    }
-    if (!(nw > 0) || !(nv > 0)) break;
-    lam = std::sqrt(nw / nv);
-    hipLaunchKernelGGL(k_scaled_copy<KT>, dim3(nblocks(nd, 256)), dim3(256), 0, s, w, v, nd,
-                       (KT)(1.0 / std::sqrt(nw)));
+    hipLaunchKernelGGL(k_power_norms<KT>, dim3(256), dim3(256), 0, s, w, v, nd, A.d_part);
+    hipLaunchKernelGGL(k_power_step<KT>, dim3(nblocks(nd, 256)), dim3(256), 0, s, w, v, nd, A.d_part,
+                       lam, it == 0 ? (L.lam > 0 ? L.lam : 1.0) : 0.0);
   }
   ONSAS_HIP_TRY(c, hipGetLastError());
-  L.lam = lam;
+  double h = 0;
+  ONSAS_HIP_TRY(c, hipMemcpyAsync(&h, lam, sizeof h, hipMemcpyDeviceToHost, s));
+  ONSAS_HIP_TRY(c, hipStreamSynchronize(s));
+  L.lam = h;
   return ONSAS_OK;
 }
 

@@ -1215,13 +1215,18 @@ int pcg_solve_t(Ctx* c, const double* b_dev, bool forcing, const void* x0, int e
   const bool sample = !use_graph || (c->pcg_solves++ % kSampleEvery) == 0;
   if (use_graph) {
     ONSAS_TRY(build_pcg_graph<KT>(c, 0, kFirstIters));
-    ONSAS_TRY(build_pcg_graph<KT>(c, 1, chunk_iters));
+    if (!amg) ONSAS_TRY(build_pcg_graph<KT>(c, 1, chunk_iters));
     ONSAS_TRY(build_pcg_graph<KT>(c, 2, 4));
   }
-  // n (even) more iterations: chunk_iters at a time, then 4, then 2
+  // n (even) more iterations: chunk_iters at a time, then 4, then 2.  Multigrid keeps
+  // to the short graphs: every numerics pass makes them stale (the smoothing
+  // coefficients are in their nodes), and capturing 16 iterations of 12 kernels each
+  // time costs more than it saves: with one host wait per level in the power iteration
+  // instead of one per step, 26.3 / 20.8 / 13.3 -> 25.8 / 20.5 / 13.0 ms (FP64 box of
+  // 8,640 nodes, 12 x 96 x 48 cylinder, 24^3 identification); 64^3 unchanged.
   auto run_iters = [&](int n) -> int {
     while (n > 0) {
-      const int slot = n >= chunk_iters ? 1 : (n >= 4 ? 2 : 0);
+      const int slot = n >= chunk_iters && !amg ? 1 : (n >= 4 ? 2 : 0);
       const int len = slot == 1 ? chunk_iters : (slot == 2 ? 4 : kFirstIters);
       if (use_graph) {
         ONSAS_HIP_TRY(c, hipGraphLaunch(c->pcg_graph[slot].exec, s));
