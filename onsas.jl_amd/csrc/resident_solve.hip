@@ -163,6 +163,10 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs<KT> a) {
   };
   const int64_t dof = 3 * i + ph;
   const bool newton = a.fint != nullptr;
+  // read before the first sum: the first workgroup overwrites it as early as after a
+  // breakdown in iteration 0
+  double before_b2 = read_lane(a.tol.forcing ? a.sc->nwt.prev_b2 : 0.0, 0);
+  asm volatile("" : "+s"(before_b2));
   KT xs = 0, rs = 0, zs = 0, ps = 0, qs = 0, d0 = 0, d1 = 0, d2 = 0, bk = 0;
   double u = 0, sm[4] = {0, 0, 0, 0};
   bool freed = false;
@@ -262,7 +266,7 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs<KT> a) {
     if (k == 0) {
       bb = sm[3];
       sm[3] = 0;
-      eta = inner_eta(a.tol, bb, f2, a.tol.forcing ? a.sc->nwt.prev_b2 : 0.0);
+      eta = inner_eta(a.tol, bb, f2, before_b2);
       tol2 = eta * eta * bb;
     }
     rzp = rz;

@@ -241,3 +241,33 @@ def test_resident_contexts_at_the_same_time():
         for f in runs:
             _, res, bound = f.result()
             assert res <= bound
+
+
+@pytest.mark.parametrize("prec", [_capi.PRECISION_MIXED, _capi.PRECISION_FP64])
+def test_resident_newton_breakdown_across_workgroups(monkeypatch, prec):
+    """PCG only on a negative definite tangent of many workgroups, with forcing: every one
+    of them leaves the first iteration the same way, the step is an error as on the
+    general path, and U stays."""
+    print(f"[gpu] resident newton, breakdown of many workgroups, precision {prec}", flush=True)
+    sm = meshes.cube(10, jitter=0.05, seed=4)
+    for resident in ("1", "0"):
+        monkeypatch.setenv("ONSAS_PCG_RESIDENT", resident)
+        c = Context(prec)
+        try:
+            c.set_nodes(sm.coords)
+            c.add_tet_group(sm.tets, _capi.MAT_NEOHOOKEAN, (-8.3e5, -3.8e5))
+            c.set_fixed_dofs((3 * sm.node_sets["x0"][:, None] + np.arange(3)).reshape(-1))
+            c.finalize()
+            c.set_linear_solver(_capi.LINSOLVE_PCG, rtol=1e-6, maxiter=20000, forcing=True,
+                                newton_tol=1e-8)
+            U = 1e-3 * np.random.default_rng(1).normal(size=3 * sm.nn)
+            f = np.ones(3 * sm.nn)
+            for _ in range(3):
+                c.set_U(U)
+                c.set_loads(nodal=f)
+                c.assemble()
+                with pytest.raises(_capi.OnsasError, match="breakdown"):
+                    c.newton_step()
+                assert np.array_equal(c.get_U(), U)
+        finally:
+            c.close()
