@@ -9,12 +9,15 @@
 // registers (L lanes a row, NB blocks a lane), p, q, r, x and z of a row in its
 // lanes.  What is left is the latency of one workgroup hearing from the others,
 // so an iteration does it twice only, once for the neighbours' z and once for one
-// sum of four values (grid_exchange.hpp):
+// sum of four values (grid_exchange.hpp), as in the single-reduction form of the
+// method (A. T. Chronopoulos and C. W. Gear, J. Comput. Appl. Math. 25, 1989):
 //   w = K z;  r.z, r.r, z.w and z.q + p.w, with p and q of the iteration before
 //   p <- z + beta p, q <- w + beta q;  p.q <- z.w + beta (z.q + p.w) + beta^2 p.q
-// The last line is p.q written out (no conjugacy is assumed), so the recurrences,
-// the stop and breakdown rules and the scalars are those of k_pcg_A / k_pcg_B and
-// only the rounding of p.q differs.  z needs no sum to be safe to read: a node that
+// The last line is p.q written out (no conjugacy is assumed), so the recurrences and
+// the stop and breakdown rules are those of k_pcg_A / k_pcg_B.  It does not see the
+// rounding of p and q and hands its error on, times beta^2: an error estimate goes
+// with it (kPqError), and p.q is summed from p and q where that has grown, and before
+// every breakdown.  z needs no sum to be safe to read: a node that
 // is not there yet carries an old epoch.
 // An iteration takes 2.3 us at 1,680 nodes (27 workgroups, met in one XCD), 1.1 us at
 // 125 nodes (one workgroup, z and the sums in LDS).  Met in device memory it is 3.4 us;
@@ -64,6 +67,21 @@ struct ResidentArgs {
   KT* warm;            // takes a copy of x, or null
   double *res, *U;
 };
+
+// The estimate of p.q's error is 2 u (z.w + |beta (z.q + p.w)| + beta^2 p.q), u the unit
+// of KT, and beta^2 times the estimate before; past kPqError u p.q a sum of its own takes
+// the place of the recurrence (an exchange: 2 of the 225 iterations of a 13 x 9 x 11 box,
+// none of 69 at 4 x 4 x 4, every 30th on a flat box, every 5th to 16th where stiffnesses
+// spread over two to seven decades).  Of chains of 20 bars over 2 / 4 / 6 / 7 decades in
+// FP32 (a host model, 192 each) the largest error of p.q is then 29 / 100 / 480 / 1,100 u,
+// and the iterations are the direct sum's within 2 %; without it 67 / 7,200 / 3e5 / 5e7 u,
+// up to a quarter more iterations, and breakdowns of definite tangents.  With 64 u 6 / 32 /
+// 210 / 670 u for about twice as many sums.  The estimate is made beside the division that
+// alpha waits for; it and its sums take 1 to 3 % of the solves' time, a fifth sum in every
+// exchange took 8 to 10 %.
+constexpr double kPqError = 256;
+template <typename KT>
+constexpr double kUnit = sizeof(KT) == 4 ? 0x1p-24 : 0x1p-53;
 
 // PcgState::aborted of a launch whose workgroups did not share one XCD
 constexpr int kNotOneXcd = 2;
@@ -242,7 +260,7 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs<KT> a) {
   };
   next_z();
 
-  double rz = 0, rr = 0, rzp = 0, pq = 0, bb = 0, eta = 0, tol2 = 0;
+  double rz = 0, rr = 0, rzp = 0, pq = 0, pqe = 0, bb = 0, eta = 0, tol2 = 0;
   int k = 0, conv = 0, brk = 0;
   for (;; ++k) {
     KT zj[NB][3];
@@ -275,15 +293,29 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs<KT> a) {
     conv = rr <= tol2;
     if (conv || k >= a.maxiter) break;
     const KT beta = (KT)(k > 0 ? rz / rzp : 0.0);
-    pq = sm[2] + (double)beta * (sm[3] + (double)beta * pq);
-    if (!(pq > 0.0) || !isfinite(pq) || !isfinite(rz)) {
-      brk = 1;
-      break;
-    }
-    const KT alpha = (KT)(rz / pq);
+    const double bt = (double)beta, b2 = bt * bt, b2pq = b2 * pq;
+    pq = sm[2] + (bt * sm[3] + b2pq);
+    KT alpha = (KT)(rz / pq);
+    pqe = b2 * pqe + 2 * kUnit<KT> * (fabs(sm[2]) + fabs(bt * sm[3]) + b2pq);
     if (own) {
       ps = zs + beta * ps;
       qs = w + beta * qs;
+    }
+    // (the same answer in every workgroup; pq > 0 otherwise)
+    if (!(pqe <= kPqError * kUnit<KT> * pq) || !isfinite(pq) || !isfinite(rz)) {
+      sm[0] = own ? (double)ps * (double)qs : 0.0;
+      sm[1] = sm[2] = sm[3] = 0;
+      if (ONE) __syncthreads();  // the last sums have been read
+      if (!sums(sm, here)) return;
+      pq = sm[0];
+      pqe = 0;
+      if (!(pq > 0.0) || !isfinite(pq) || !isfinite(rz)) {
+        brk = 1;
+        break;
+      }
+      alpha = (KT)(rz / pq);
+    }
+    if (own) {
       xs += alpha * ps;
       rs -= alpha * qs;
     }
@@ -310,7 +342,7 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs<KT> a) {
     PcgState* st = &a.host->pcg;
     host_store(&st->bb, bb);
     host_store(&st->rr_last, rr);
-    host_store(&st->k, k);
+    host_store(&st->k, (int32_t)(ep - a.base));  // epochs used
     host_store(&st->breakdown, brk);
     host_store(&st->breakdown_k, brk ? k : -1);
     host_store(&st->iters, k);
@@ -838,7 +870,8 @@ static int resident_run(Ctx* c, const double* b, const double* fint, const void*
   ONSAS_HIP_TRY(c, hipStreamSynchronize(c->stream));
   const PcgState& ps = c->h_sc->pcg;
   *ran = ps.done && !ps.aborted;
-  c->gslot_epoch += (*ran ? (uint32_t)ps.k : (uint32_t)pcg_maxiter(c)) + 5;
+  // an iteration takes at most two epochs
+  c->gslot_epoch += (*ran ? (uint32_t)ps.k : 2 * (uint32_t)pcg_maxiter(c) + 5) + 1;
   if (*ran) {
     pcg_result(ps, iters, relres, converged, breakdown);
     return ONSAS_OK;
