@@ -342,6 +342,16 @@ int onsas_locate_points(onsas_ctx* ctx, int32_t group, int64_t npts, const doubl
 int onsas_get_timings(onsas_ctx* ctx, onsas_timings* t);
 int onsas_reset_timings(onsas_ctx* ctx);
 
+/* Which way the solves of small and mid-size models went (no counterpart in the
+ * reference), counted since onsas_finalize.  Block-Jacobi PCG (with the whole Newton
+ * step around it) and GMRES of such models run as one launch whose workgroups wait for
+ * one another; where the GPU is too busy to hold them all at once a wait expires (0.2 s)
+ * and the solve is taken again on a slower path, with other rounding.  out[0]: launches
+ * that solved in one workgroup, out[1]: whose workgroups met in one XCD's cache, out[2]:
+ * across the device, out[3]: launches that gave up.  Solves in none of them ran on the
+ * general kernels. */
+int onsas_resident_launches(onsas_ctx* ctx, int64_t* out);
+
 /* Test hook: the next fallible call on ctx returns `code` (error-path tests). */
 int onsas_inject_error(onsas_ctx* ctx, int32_t code);
 

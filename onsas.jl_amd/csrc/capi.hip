@@ -6,6 +6,7 @@
 #include <atomic>
 #include <cmath>
 #include <cstring>
+#include <iterator>
 #include <mutex>
 #include <string>
 #include <thread>
@@ -1106,6 +1107,14 @@ int onsas_get_timings(onsas_ctx* ctx, onsas_timings* t) {
     account_assembly(c);
   }
   *t = c->tm;
+  return ONSAS_OK;
+}
+
+int onsas_resident_launches(onsas_ctx* ctx, int64_t* out) {
+  Ctx* c = C(ctx);
+  ONSAS_TRY(check_ready(c));
+  if (!out) return set_err(c, ONSAS_ERR_ARG, "NULL output");
+  std::copy(std::begin(c->resident_launches), std::end(c->resident_launches), out);
   return ONSAS_OK;
 }
 

@@ -372,6 +372,8 @@ struct Ctx {
   unsigned long long* d_share = nullptr;    // a vector handed from workgroup to workgroup
   uint32_t gslot_epoch = 1;
   long long gslot_ticks = 20000000;  // 0.2 s
+  // launches that solved: one workgroup, met in one XCD, across the device; that gave up
+  int64_t resident_launches[4] = {0, 0, 0, 0};
 
   // aggregation multigrid preconditioner (built on its first use)
   Amg amg;

@@ -680,6 +680,9 @@ constexpr int kResidentBlocks = 4;  // blocks a lane keeps in registers
 constexpr int kResidentThreads = 256;
 constexpr int resident_one_threads(size_t kt) { return kt == 4 ? 1024 : 512; }
 
+// where a launch's workgroups meet (an index of Ctx::resident_launches)
+enum Place { kOneWorkgroup, kOneXcd, kAcrossDevice, kGaveUp };
+
 struct ResidentShape {
   int threads;
   int64_t grid;
@@ -726,7 +729,7 @@ void run_resident(Ctx* c, const ResidentArgs<KT>& a, const ResidentShape& sh, bo
 }
 
 template <typename KT>
-int resident_t(Ctx* c, const double* b, const double* fint, const void* x0, void* warm, bool* xcd) {
+int resident_t(Ctx* c, const double* b, const double* fint, const void* x0, void* warm, Place* at) {
   ResidentArgs<KT> a{};
   a.sell_ptr = c->d_sell_ptr;
   a.slice_rounds = c->d_slice_rounds;
@@ -752,19 +755,21 @@ int resident_t(Ctx* c, const double* b, const double* fint, const void* x0, void
   a.limit = c->gslot_ticks;
   a.nn = c->nn;
   const ResidentShape sh = resident_shape(c);
-  *xcd = sh.grid > 1 && sh.threads == kResidentThreads && on_one_xcd(c, sh.grid, xcd_waves(c->kt));
+  const bool xcd =
+      sh.grid > 1 && sh.threads == kResidentThreads && on_one_xcd(c, sh.grid, xcd_waves(c->kt));
+  *at = sh.grid == 1 ? kOneWorkgroup : xcd ? kOneXcd : kAcrossDevice;
   a.nwg = (int)sh.grid;
   a.xcd = c->xcd;
   if (lanes_per_row(c) == 4)
-    run_resident<KT, 4>(c, a, sh, *xcd);
+    run_resident<KT, 4>(c, a, sh, xcd);
   else
-    run_resident<KT, 8>(c, a, sh, *xcd);
+    run_resident<KT, 8>(c, a, sh, xcd);
   ONSAS_HIP_TRY(c, hipGetLastError());
   return ONSAS_OK;
 }
 
 template <typename KT, int L>
-int gmres_t(Ctx* c, const double* b_dev, int m, int maxiter, double rtol, bool* xcd) {
+int gmres_t(Ctx* c, const double* b_dev, int m, int maxiter, double rtol, Place* at) {
   GmresArgs<KT> a{};
   a.sell_ptr = c->d_sell_ptr;
   a.slice_rounds = c->d_slice_rounds;
@@ -796,8 +801,9 @@ int gmres_t(Ctx* c, const double* b_dev, int m, int maxiter, double rtol, bool* 
     return ONSAS_OK;
   };
   // two workgroups a CU where the LDS holds two
-  *xcd = on_one_xcd(c, grid, lds <= 78 * 1024 ? 2 : 1);
-  if (*xcd)
+  const bool xcd = on_one_xcd(c, grid, lds <= 78 * 1024 ? 2 : 1);
+  *at = xcd ? kOneXcd : kAcrossDevice;
+  if (xcd)
     ONSAS_TRY(go(k_gmres_resident<KT, L, kResidentBlocks, Meet::kXcd>, 8 * grid));
   else
     ONSAS_TRY(go(k_gmres_resident<KT, L, kResidentBlocks, Meet::kDevice>, grid));
@@ -852,8 +858,9 @@ static int renew_epochs(Ctx* c) {
 // A launch that gave up (a wait expired: the GPU, or the XCD, was too busy to hold the
 // whole grid) or found its workgroups on several XCDs: the next one meets across the
 // device, and after that the context keeps to the general kernels.
-static void resident_failed(Ctx* c, bool xcd) {
-  if (xcd)
+static void resident_failed(Ctx* c, Place at) {
+  c->resident_launches[kGaveUp]++;
+  if (at == kOneXcd)
     c->one_xcd = false;
   else
     c->pcg_resident = false;
@@ -864,19 +871,20 @@ static int resident_run(Ctx* c, const double* b, const double* fint, const void*
                         bool* ran, int* iters, double* relres, int* converged, int* breakdown) {
   ONSAS_TRY(renew_epochs(c));
   c->h_sc->pcg = PcgState{};
-  bool xcd = false;
-  ONSAS_TRY(c->precision == ONSAS_PRECISION_FP64 ? resident_t<double>(c, b, fint, x0, warm, &xcd)
-                                                 : resident_t<float>(c, b, fint, x0, warm, &xcd));
+  Place at = kOneWorkgroup;
+  ONSAS_TRY(c->precision == ONSAS_PRECISION_FP64 ? resident_t<double>(c, b, fint, x0, warm, &at)
+                                                 : resident_t<float>(c, b, fint, x0, warm, &at));
   ONSAS_HIP_TRY(c, hipStreamSynchronize(c->stream));
   const PcgState& ps = c->h_sc->pcg;
   *ran = ps.done && !ps.aborted;
   // an iteration takes at most two epochs
   c->gslot_epoch += (*ran ? (uint32_t)ps.k : 2 * (uint32_t)pcg_maxiter(c) + 5) + 1;
   if (*ran) {
+    c->resident_launches[at]++;
     pcg_result(ps, iters, relres, converged, breakdown);
     return ONSAS_OK;
   }
-  resident_failed(c, xcd);
+  resident_failed(c, at);
   return clear_abort(c);
 }
 
@@ -930,13 +938,13 @@ int launch_gmres_resident(Ctx* c, const double* b_dev, int m, int maxiter, doubl
   }
   ONSAS_TRY(renew_epochs(c));
   ONSAS_HIP_TRY(c, hipMemsetAsync(&c->d_sc->pcg, 0, sizeof(PcgState), s));
-  bool xcd = false;
+  Place at = kOneXcd;
   if (c->precision == ONSAS_PRECISION_FP64)
-    ONSAS_TRY(L == 4 ? (gmres_t<double, 4>(c, b_dev, m, maxiter, rtol, &xcd))
-                     : (gmres_t<double, 8>(c, b_dev, m, maxiter, rtol, &xcd)));
+    ONSAS_TRY(L == 4 ? (gmres_t<double, 4>(c, b_dev, m, maxiter, rtol, &at))
+                     : (gmres_t<double, 8>(c, b_dev, m, maxiter, rtol, &at)));
   else
-    ONSAS_TRY(L == 4 ? (gmres_t<float, 4>(c, b_dev, m, maxiter, rtol, &xcd))
-                     : (gmres_t<float, 8>(c, b_dev, m, maxiter, rtol, &xcd)));
+    ONSAS_TRY(L == 4 ? (gmres_t<float, 4>(c, b_dev, m, maxiter, rtol, &at))
+                     : (gmres_t<float, 8>(c, b_dev, m, maxiter, rtol, &at)));
   ONSAS_HIP_TRY(c, hipMemcpyAsync(&c->h_sc->pcg, &c->d_sc->pcg, sizeof(PcgState),
                                   hipMemcpyDeviceToHost, s));
   ONSAS_HIP_TRY(c, hipStreamSynchronize(s));
@@ -944,10 +952,11 @@ int launch_gmres_resident(Ctx* c, const double* b_dev, int m, int maxiter, doubl
   // an iteration takes at most 3 epochs, a restart 3
   c->gslot_epoch += (ps.aborted ? 6u * ((uint32_t)maxiter + 2) : (uint32_t)ps.k) + 4;
   if (ps.aborted) {
-    resident_failed(c, xcd);
+    resident_failed(c, at);
     ONSAS_TRY(clear_abort(c));
     return launch_gmres_resident(c, b_dev, m, maxiter, rtol, ran, iters, relres, converged);
   }
+  c->resident_launches[at]++;
   *ran = true;
   *iters = ps.iters;
   *relres = ps.bb > 0 ? std::sqrt(ps.rr_last / ps.bb) : 0.0;

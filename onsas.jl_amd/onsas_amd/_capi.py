@@ -40,7 +40,7 @@ EXPORTED = (
     "onsas_linear_solve", "onsas_adjoint_shear", "onsas_set_shear_moduli", "onsas_locate_points",
     "onsas_get_timings", "onsas_reset_timings", "onsas_inject_error", "onsas_amg_levels",
     "onsas_amg_level_info", "onsas_amg_get_operator", "onsas_amg_get_prolongator",
-    "onsas_time_cycle_products", "onsas_time_level_products",
+    "onsas_time_cycle_products", "onsas_time_level_products", "onsas_resident_launches",
 )
 
 
@@ -132,6 +132,7 @@ def load():
         "onsas_locate_points": ([_vp, C.c_int32, C.c_int64, _vp, _vp, _vp, _vp, _vp], C.c_int),
         "onsas_get_timings": ([_vp, C.POINTER(Timings)], C.c_int),
         "onsas_reset_timings": ([_vp], C.c_int),
+        "onsas_resident_launches": ([_vp, _i64p], C.c_int),
         "onsas_inject_error": ([_vp, C.c_int32], C.c_int),
         "onsas_amg_levels": ([_vp, _i32p], C.c_int),
         "onsas_amg_level_info": ([_vp, C.c_int32, _i64p, _i32p, _i64p, _i64p, _dp], C.c_int),
@@ -454,6 +455,13 @@ class Context:
 
     def reset_timings(self):
         self._check(self.L.onsas_reset_timings(self.h))
+
+    def resident_launches(self):
+        """Solves that ran as one launch, by where its workgroups met, and launches that gave
+        up (their solves were taken again on a slower path)."""
+        out = (C.c_int64 * 4)()
+        self._check(self.L.onsas_resident_launches(self.h, out))
+        return dict(zip(("one_workgroup", "one_xcd", "across_device", "gave_up"), out))
 
     def inject_error(self, code):
         self._check(self.L.onsas_inject_error(self.h, int(code)))
