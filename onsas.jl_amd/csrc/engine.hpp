@@ -367,6 +367,8 @@ struct Ctx {
   bool pcg_resident = false;  // ONSAS_PCG_RESIDENT=0 turns it off (read at finalize)
   bool one_xcd = true;        // resident launches may meet in one XCD (ONSAS_RESIDENT_XCD=0: not)
   int xcd = 0;                // ... in the one that holds this residue of the workgroup ids
+  int cus = 0;                // CUs of the device
+  bool pcg_xcd = false, pcg_device = false;  // ... where the PCG's workgroups are resident at once
   unsigned long long* d_gslots = nullptr;    // the tail of d_part's allocation
   unsigned long long* d_gmslots = nullptr;  // the same for GMRES (on its first use)
   unsigned long long* d_share = nullptr;    // a vector handed from workgroup to workgroup

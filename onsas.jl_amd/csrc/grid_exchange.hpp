@@ -1,8 +1,9 @@
 // grid_exchange.hpp -- sums and vectors shared by the workgroups of one resident
 // launch (the solver kernels that run a whole solve in one launch).  gfx950.
 //
-// Every workgroup of such a launch is resident at once (the host keeps the grid
-// far below the 256 CUs), so workgroups may wait for one another.  A grid-wide
+// Every workgroup of such a launch is resident at once (the host holds the grid to what
+// the device reports for the kernel: resident_rule.hpp), so workgroups may wait for one
+// another.  A grid-wide
 // sum is one exchange: each workgroup writes its partial into its own slot and
 // polls the slots of all others.  The slot words are 8 bytes, (epoch << 32) |
 // half of the double, so a word carries its own "ready" mark and the sum is

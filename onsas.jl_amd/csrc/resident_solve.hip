@@ -35,6 +35,7 @@
 
 #include "engine.hpp"
 #include "grid_exchange.hpp"
+#include "resident_rule.hpp"
 
 namespace onsas {
 
@@ -91,9 +92,6 @@ template <typename T>
 __device__ inline void host_store(T* p, T v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
-
-// Waves a SIMD that the registers of k_pcg_resident leave (up to 168 and 256 of them).
-constexpr int xcd_waves(size_t kt) { return kt == 4 ? 3 : 2; }
 
 // L lanes a block row (lane ph takes the row's slots ph, ph + L, ...: at most
 // NB), T threads a workgroup.  Lanes 0, 1, 2 of a row hold the row's three
@@ -697,35 +695,66 @@ inline ResidentShape resident_shape(const Ctx* c) {
 }
 
 // Every 8th workgroup of a launch shares an XCD: 32 CUs, on which 64 workgroups of 256
-// threads are resident together with two waves a SIMD, and 96 with three.  That many
-// do better there, met in its L2, than spread over the device: FP32 1,680 / 4,096 /
-// 5,832 nodes 10.3 / 7.6 / 9.8 ms against 14.1 / 9.6 / 12.6 ms, FP64 2,080 / 3,375
-// nodes 2.8 / 9.4 ms against 3.8 / 11.2 ms, GMRES at 720 nodes 14.4 ms against 17.3 ms.
-inline bool on_one_xcd(const Ctx* c, int64_t grid, int waves) {
-  return c->one_xcd && grid <= 32 * waves;
+// threads are resident together with two waves a SIMD (FP64), and 96 with three (FP32).
+// That many do better there, met in its L2, than spread over the device: FP32 1,680 /
+// 4,096 / 5,832 nodes 10.3 / 7.6 / 9.8 ms against 14.1 / 9.6 / 12.6 ms, FP64 2,080 /
+// 3,375 nodes 2.8 / 9.4 ms against 3.8 / 11.2 ms, GMRES at 720 nodes 14.4 ms against
+// 17.3 ms.
+inline bool on_one_xcd(const Ctx* c, int64_t grid, int blocks) {
+  return c->one_xcd && fits_one_xcd(grid, blocks, c->cus);
+}
+
+// workgroups of `kern` that a CU takes
+template <typename... A>
+int blocks_per_cu(Ctx* c, void (*kern)(A...), int threads, size_t lds, int* blocks) {
+  ONSAS_HIP_TRY(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                       blocks, reinterpret_cast<const void*>(kern), threads, lds));
+  return ONSAS_OK;
 }
 inline size_t share_words(const Ctx* c) { return (size_t)c->nn * c->kt / 2; }  // kShareBytes a node
 
-// A Newton step's launch stamps the step's timing events.
-template <typename KT, int L>
-void run_resident(Ctx* c, const ResidentArgs<KT>& a, const ResidentShape& sh, bool xcd) {
+// f(kernel of a shape, its threads, its grid)
+template <typename KT, int L, typename F>
+int with_pcg_kernel(const ResidentShape& sh, bool xcd, F f) {
   constexpr int T1 = resident_one_threads(sizeof(KT)), T = kResidentThreads;
   constexpr int NB = kResidentBlocks;
   constexpr Meet D = Meet::kDevice, X = Meet::kXcd;
-  const hipEvent_t e0 = a.fint ? c->ev[4] : nullptr, e1 = a.fint ? c->ev[7] : nullptr;
-  auto go = [&](auto kern, int threads, int64_t grid) {
-    hipExtLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(threads), 0, c->stream, e0, e1, 0, a);
+  if (sh.grid == 1 && sh.threads == 512) return f(k_pcg_resident<KT, L, NB, 512, true, D>, 512, 1);
+  if (sh.grid == 1) return f(k_pcg_resident<KT, L, NB, T1, true, D>, T1, 1);
+  if (xcd) return f(k_pcg_resident<KT, L, NB, T, false, X>, T, 8 * sh.grid);
+  if (sh.threads == T) return f(k_pcg_resident<KT, L, NB, T, false, D>, T, sh.grid);
+  return f(k_pcg_resident<KT, L, NB, 2 * T, false, D>, 2 * T, sh.grid);
+}
+
+// Where the model's PCG may meet, from what the device takes of its kernels.
+template <typename KT, int L>
+int pcg_places(Ctx* c) {
+  const ResidentShape sh = resident_shape(c);
+  auto blocks = [&](bool xcd, int* n) -> int {
+    return with_pcg_kernel<KT, L>(sh, xcd, [&](auto kern, int threads, int64_t) {
+      return blocks_per_cu(c, kern, threads, 0, n);
+    });
   };
-  if (sh.grid == 1 && sh.threads == 512)
-    go(k_pcg_resident<KT, L, NB, 512, true, D>, 512, 1);
-  else if (sh.grid == 1)
-    go(k_pcg_resident<KT, L, NB, T1, true, D>, T1, 1);
-  else if (xcd)
-    go(k_pcg_resident<KT, L, NB, T, false, X>, T, 8 * sh.grid);
-  else if (sh.threads == T)
-    go(k_pcg_resident<KT, L, NB, T, false, D>, T, sh.grid);
-  else
-    go(k_pcg_resident<KT, L, NB, 2 * T, false, D>, 2 * T, sh.grid);
+  int n = 0;
+  ONSAS_TRY(blocks(false, &n));
+  c->pcg_device = fits_device(sh.grid, n, c->cus);
+  c->pcg_xcd = false;
+  if (sh.grid > 1 && sh.threads == kResidentThreads) {
+    ONSAS_TRY(blocks(true, &n));
+    c->pcg_xcd = fits_one_xcd(sh.grid, n, c->cus);
+  }
+  return ONSAS_OK;
+}
+
+// A Newton step's launch stamps the step's timing events.
+template <typename KT, int L>
+int run_resident(Ctx* c, const ResidentArgs<KT>& a, const ResidentShape& sh, bool xcd) {
+  const hipEvent_t e0 = a.fint ? c->ev[4] : nullptr, e1 = a.fint ? c->ev[7] : nullptr;
+  return with_pcg_kernel<KT, L>(sh, xcd, [&](auto kern, int threads, int64_t grid) -> int {
+    hipExtLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(threads), 0, c->stream, e0, e1, 0, a);
+    ONSAS_HIP_TRY(c, hipGetLastError());
+    return ONSAS_OK;
+  });
 }
 
 template <typename KT>
@@ -755,17 +784,12 @@ int resident_t(Ctx* c, const double* b, const double* fint, const void* x0, void
   a.limit = c->gslot_ticks;
   a.nn = c->nn;
   const ResidentShape sh = resident_shape(c);
-  const bool xcd =
-      sh.grid > 1 && sh.threads == kResidentThreads && on_one_xcd(c, sh.grid, xcd_waves(c->kt));
+  const bool xcd = c->one_xcd && c->pcg_xcd;
   *at = sh.grid == 1 ? kOneWorkgroup : xcd ? kOneXcd : kAcrossDevice;
   a.nwg = (int)sh.grid;
   a.xcd = c->xcd;
-  if (lanes_per_row(c) == 4)
-    run_resident<KT, 4>(c, a, sh, xcd);
-  else
-    run_resident<KT, 8>(c, a, sh, xcd);
-  ONSAS_HIP_TRY(c, hipGetLastError());
-  return ONSAS_OK;
+  return lanes_per_row(c) == 4 ? run_resident<KT, 4>(c, a, sh, xcd)
+                               : run_resident<KT, 8>(c, a, sh, xcd);
 }
 
 template <typename KT, int L>
@@ -794,21 +818,26 @@ int gmres_t(Ctx* c, const double* b_dev, int m, int maxiter, double rtol, Place*
   a.nwg = (int)grid;
   a.xcd = c->xcd;
   const size_t lds = gmres_lds(m, R, sizeof(KT));
-  auto go = [&](auto kern, int64_t n) -> int {
+  // *at = kGaveUp: the device does not take the grid, and nothing has been launched
+  auto blocks = [&](auto kern, int* n) -> int {
     ONSAS_HIP_TRY(c, hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    return blocks_per_cu(c, kern, kGmresThreads, lds, n);
+  };
+  auto go = [&](auto kern, int64_t n) -> int {
     hipLaunchKernelGGL(kern, dim3((unsigned)n), dim3(kGmresThreads), lds, c->stream, a);
+    ONSAS_HIP_TRY(c, hipGetLastError());
     return ONSAS_OK;
   };
-  // two workgroups a CU where the LDS holds two
-  const bool xcd = on_one_xcd(c, grid, lds <= 78 * 1024 ? 2 : 1);
-  *at = xcd ? kOneXcd : kAcrossDevice;
-  if (xcd)
-    ONSAS_TRY(go(k_gmres_resident<KT, L, kResidentBlocks, Meet::kXcd>, 8 * grid));
-  else
-    ONSAS_TRY(go(k_gmres_resident<KT, L, kResidentBlocks, Meet::kDevice>, grid));
-  ONSAS_HIP_TRY(c, hipGetLastError());
-  return ONSAS_OK;
+  int n = 0;
+  ONSAS_TRY(blocks(k_gmres_resident<KT, L, kResidentBlocks, Meet::kXcd>, &n));
+  if (on_one_xcd(c, grid, n)) {
+    *at = kOneXcd;
+    return go(k_gmres_resident<KT, L, kResidentBlocks, Meet::kXcd>, 8 * grid);
+  }
+  ONSAS_TRY(blocks(k_gmres_resident<KT, L, kResidentBlocks, Meet::kDevice>, &n));
+  *at = fits_device(grid, n, c->cus) ? kAcrossDevice : kGaveUp;
+  return *at == kGaveUp ? ONSAS_OK : go(k_gmres_resident<KT, L, kResidentBlocks, Meet::kDevice>, grid);
 }
 
 }  // namespace
@@ -829,6 +858,12 @@ int pcg_resident_setup(Ctx* c) {
   static std::atomic<unsigned> contexts{0};
   c->xcd = (int)((contexts++ + (unsigned)getpid()) % 8);
   if (!c->pcg_resident) return ONSAS_OK;
+  ONSAS_HIP_TRY(c, hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, c->device));
+  const bool f64 = c->precision == ONSAS_PRECISION_FP64;
+  if (lanes_per_row(c) == 4)
+    ONSAS_TRY(f64 ? (pcg_places<double, 4>(c)) : (pcg_places<float, 4>(c)));
+  else
+    ONSAS_TRY(f64 ? (pcg_places<double, 8>(c)) : (pcg_places<float, 8>(c)));
   const size_t bytes = share_words(c) * sizeof(unsigned long long);
   ONSAS_HIP_TRY(c, hipMalloc((void**)&c->d_share, bytes));
   ONSAS_HIP_TRY(c, hipMemset(c->d_share, 0, bytes));
@@ -889,7 +924,8 @@ static int resident_run(Ctx* c, const double* b, const double* fint, const void*
 }
 
 inline bool pcg_resident_now(const Ctx* c) {
-  return c->pcg_resident && c->lin.precond != ONSAS_PRECOND_AMG &&
+  return c->pcg_resident && (c->pcg_device || (c->one_xcd && c->pcg_xcd)) &&
+         c->lin.precond != ONSAS_PRECOND_AMG &&
          pcg_maxiter(c) <= kMaxResidentIters;
 }
 
@@ -945,6 +981,7 @@ int launch_gmres_resident(Ctx* c, const double* b_dev, int m, int maxiter, doubl
   else
     ONSAS_TRY(L == 4 ? (gmres_t<float, 4>(c, b_dev, m, maxiter, rtol, &at))
                      : (gmres_t<float, 8>(c, b_dev, m, maxiter, rtol, &at)));
+  if (at == kGaveUp) return ONSAS_OK;
   ONSAS_HIP_TRY(c, hipMemcpyAsync(&c->h_sc->pcg, &c->d_sc->pcg, sizeof(PcgState),
                                   hipMemcpyDeviceToHost, s));
   ONSAS_HIP_TRY(c, hipStreamSynchronize(s));
