@@ -11,8 +11,8 @@
 // so all of them take the same branches and a solve is bit-identical from run
 // to run.  A sum alone, measured on one MI355X: 1.2 us for 2 workgroups, 1.9 us for
 // 32, 2.4 us for 64 and 3.3 us for 128 across the device, against 4 to 8 us for a
-// kernel boundary with its drain, launch and first loads.  Vectors are handed over in
-// the same way, every component in words of its own, so nothing else orders the
+// kernel boundary with its drain, launch and first loads.  Vectors are handed over a
+// node at a time with a mark of their own (share_node), so nothing else orders the
 // workgroups' memory and the read-only data stays cached.
 //
 // Waits are bounded: a workgroup that polls past `limit` clock ticks (or sees
@@ -24,6 +24,7 @@
 
 #include <cstdint>
 
+#include "share_mark.hpp"
 #include "wave_ops.hpp"
 
 namespace onsas {
@@ -137,11 +138,13 @@ __device__ inline unsigned long long value_word(double p, uint32_t epoch, bool l
   return ((unsigned long long)epoch << 32) | (low ? (b & 0xffffffffull) : (b >> 32));
 }
 
-// A node of a vector that its neighbours read: 16 bytes, its three components and the
-// epoch (FP64: twice 16 bytes, each with 12 bytes of the components and the epoch).
-// An aligned 16-byte store or load of a lane is one request to one cache line and so
-// is seen whole (1.2e8 reads of words being written showed no mixture, in either
-// meeting place).  A sum between the readers' use and the next hand-over makes sure
+// A node of a vector that its neighbours read: 16 bytes, its three components and a
+// mark (FP64: twice 16 bytes, each with 12 bytes of the components and a mark).  No
+// memory model says that an aligned 16-byte store or load of a lane is seen whole; it is
+// one request to one cache line, and no mixture has been seen.  The mark does not rest on
+// that: it is made of the epoch and the other three words (share_mark.hpp).  Against the
+// epoch alone that is 2 % of an FP64 solve of 2,080 nodes and nothing in FP32; a test of
+// one word after the other under branches took 10 % of it.  A sum between the readers' use and the next hand-over makes sure
 // that nothing is overwritten before all have read it.
 template <typename KT>
 constexpr uint32_t kShareBytes = 4 * sizeof(KT);  // per node
@@ -159,16 +162,17 @@ template <Meet M>
 __device__ inline void share_node(SharedBuf z, uint32_t i, int part, float a, float b, float c,
                                   uint32_t epoch) {
   (void)part;
-  shared_store<M>(z, kShareBytes<float> * i,
-                  u32x4{__float_as_uint(a), __float_as_uint(b), __float_as_uint(c), epoch});
+  const uint32_t x = __float_as_uint(a), y = __float_as_uint(b), w = __float_as_uint(c);
+  shared_store<M>(z, kShareBytes<float> * i, u32x4{x, y, w, share_mark(x, y, w, epoch)});
 }
 template <Meet M>
 __device__ inline void share_node(SharedBuf z, uint32_t i, int part, double a, double b, double c,
                                   uint32_t epoch) {
   const double x = part ? c : a;
+  const uint32_t l = (uint32_t)__double2loint(x), h = (uint32_t)__double2hiint(x),
+                 o = (uint32_t)(part ? __double2hiint(b) : __double2loint(b));
   shared_store<M>(z, kShareBytes<double> * i + 16u * part,
-                  u32x4{(uint32_t)__double2loint(x), (uint32_t)__double2hiint(x),
-                        (uint32_t)(part ? __double2hiint(b) : __double2loint(b)), epoch});
+                  u32x4{l, h, o, share_mark(l, h, o, epoch)});
 }
 // The three components of the nodes at the byte offsets off, once they carry the
 // epoch; false once the launch is aborted.
@@ -178,14 +182,16 @@ __device__ inline bool gather_shared(SharedBuf z, const uint32_t (&off)[N], uint
   constexpr int P = kShareLanes<KT>;
   return poll(gs, [&] {
     u32x4 w[N][P];
-    bool ready = true;
+    uint32_t off_mark = 0;  // zero once every mark is the epoch's (no branch a word)
 #pragma unroll
     for (int q = 0; q < N; ++q)
 #pragma unroll
       for (int p = 0; p < P; ++p) w[q][p] = shared_load<M>(z, off[q] + 16u * p);
 #pragma unroll
     for (int q = 0; q < N; ++q) {
-      ready = ready && w[q][0][3] == epoch && w[q][P - 1][3] == epoch;
+#pragma unroll
+      for (int p = 0; p < P; ++p)
+        off_mark |= w[q][p][3] ^ share_mark(w[q][p][0], w[q][p][1], w[q][p][2], epoch);
       if constexpr (P == 1) {
 #pragma unroll
         for (int c = 0; c < 3; ++c) zj[q][c] = __uint_as_float(w[q][0][c]);
@@ -195,7 +201,7 @@ __device__ inline bool gather_shared(SharedBuf z, const uint32_t (&off)[N], uint
         zj[q][2] = __hiloint2double((int)w[q][1][1], (int)w[q][1][0]);
       }
     }
-    return ready;
+    return off_mark == 0;
   });
 }
 
