@@ -374,6 +374,12 @@ struct Ctx {
   unsigned long long* d_share = nullptr;    // a vector handed from workgroup to workgroup
   uint32_t gslot_epoch = 1;
   long long gslot_ticks = 20000000;  // 0.2 s
+  long long first_ticks = 0;         // ... of the first launches
+  int first_launches = 0;
+  // after a launch that gave up: what the context may go back to, solves until it tries,
+  // and the next such rest
+  bool may_pcg_resident = false, may_one_xcd = true;
+  int resident_rest = 0, resident_pause = 0;
   // launches that solved: one workgroup, met in one XCD, across the device; that gave up
   int64_t resident_launches[4] = {0, 0, 0, 0};
 

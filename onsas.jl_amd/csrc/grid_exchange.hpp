@@ -9,15 +9,17 @@
 // half of the double, so a word carries its own "ready" mark and the sum is
 // exact; the partials are added by a fixed tree, the same in every workgroup,
 // so all of them take the same branches and a solve is bit-identical from run
-// to run.  A sum alone, measured on one MI355X: 1.2 us for 2 workgroups, 1.9 us for
+// to run, in either meeting place, as long as no wait expires (the general kernels
+// add in another order).  A sum alone, measured on one MI355X: 1.2 us for 2 workgroups, 1.9 us for
 // 32, 2.4 us for 64 and 3.3 us for 128 across the device, against 4 to 8 us for a
 // kernel boundary with its drain, launch and first loads.  Vectors are handed over a
 // node at a time with a mark of their own (share_node), so nothing else orders the
 // workgroups' memory and the read-only data stays cached.
 //
 // Waits are bounded: a workgroup that polls past `limit` clock ticks (or sees
-// another's abort) raises the abort word and the launch drains; the host then
-// solves with the one-kernel-per-step path.
+// another's abort) raises the abort word and the launch drains; the host then takes the
+// solve again across the device, or on the general kernels, and comes back to the fastest
+// path some solves later.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -29,6 +29,7 @@
 #include <atomic>
 #include <cmath>
 #include <cstdlib>
+#include <cstring>
 #include <type_traits>
 
 #include <hip/hip_ext.h>
@@ -746,6 +747,13 @@ int pcg_places(Ctx* c) {
   return ONSAS_OK;
 }
 
+// the longest wait of the next launch
+inline long long wait_ticks(Ctx* c) {
+  if (c->first_launches == 0) return c->gslot_ticks;
+  --c->first_launches;
+  return c->first_ticks;
+}
+
 // A Newton step's launch stamps the step's timing events.
 template <typename KT, int L>
 int run_resident(Ctx* c, const ResidentArgs<KT>& a, const ResidentShape& sh, bool xcd) {
@@ -781,7 +789,7 @@ int resident_t(Ctx* c, const double* b, const double* fint, const void* x0, void
   a.res = c->d_res;
   a.U = c->d_U;
   a.base = c->gslot_epoch;
-  a.limit = c->gslot_ticks;
+  a.limit = wait_ticks(c);
   a.nn = c->nn;
   const ResidentShape sh = resident_shape(c);
   const bool xcd = c->one_xcd && c->pcg_xcd;
@@ -808,7 +816,7 @@ int gmres_t(Ctx* c, const double* b_dev, int m, int maxiter, double rtol, Place*
   a.st = &c->d_sc->pcg;
   a.slots = c->d_gmslots;
   a.base = c->gslot_epoch;
-  a.limit = c->gslot_ticks;
+  a.limit = wait_ticks(c);
   a.nn = c->nn;
   a.m = m;
   a.maxiter = maxiter;
@@ -842,6 +850,12 @@ int gmres_t(Ctx* c, const double* b_dev, int m, int maxiter, double rtol, Place*
 
 }  // namespace
 
+// Solves that a context takes on the slower path before it tries again, doubled by every
+// launch that gives up and back to the first by one that solves: an expired wait is 0.2 s,
+// some tens of general solves, so a GPU that stays busy costs a vanishing share of it and
+// one that was busy once costs a model this many slower solves.
+constexpr int kFirstRest = 64, kLongestRest = 1 << 16;
+
 // Whether a block-Jacobi PCG of this model runs as one launch: rows short enough
 // for the lanes' registers and a grid of at most kMaxGridWg workgroups (16,384
 // rows of up to 16 blocks, 8,192 of up to 32).
@@ -852,9 +866,16 @@ bool pcg_resident_fits(const Ctx* c) {
 
 int pcg_resident_setup(Ctx* c) {
   const char* e = std::getenv("ONSAS_PCG_RESIDENT");
-  c->pcg_resident = pcg_resident_fits(c) && !(e && e[0] == '0');
-  if (const char* x = std::getenv("ONSAS_RESIDENT_XCD")) c->one_xcd = x[0] != '0';
-  if (const char* t = std::getenv("ONSAS_RESIDENT_TICKS")) c->gslot_ticks = std::atoll(t);
+  c->pcg_resident = c->may_pcg_resident = pcg_resident_fits(c) && !(e && e[0] == '0');
+  if (const char* x = std::getenv("ONSAS_RESIDENT_XCD")) c->one_xcd = c->may_one_xcd = x[0] != '0';
+  c->resident_rest = 0;
+  c->resident_pause = kFirstRest;
+  // "n" ticks, or "n:m", for the first m launches
+  if (const char* t = std::getenv("ONSAS_RESIDENT_TICKS")) {
+    const char* colon = std::strchr(t, ':');
+    (colon ? c->first_ticks : c->gslot_ticks) = std::atoll(t);
+    c->first_launches = colon ? std::atoi(colon + 1) : 0;
+  }
   static std::atomic<unsigned> contexts{0};
   c->xcd = (int)((contexts++ + (unsigned)getpid()) % 8);
   if (!c->pcg_resident) return ONSAS_OK;
@@ -892,13 +913,25 @@ static int renew_epochs(Ctx* c) {
 
 // A launch that gave up (a wait expired: the GPU, or the XCD, was too busy to hold the
 // whole grid) or found its workgroups on several XCDs: the next one meets across the
-// device, and after that the context keeps to the general kernels.
+// device, and after that the context keeps to the general kernels, for some solves.
 static void resident_failed(Ctx* c, Place at) {
   c->resident_launches[kGaveUp]++;
   if (at == kOneXcd)
     c->one_xcd = false;
   else
     c->pcg_resident = false;
+  c->resident_rest = c->resident_pause;
+  c->resident_pause = std::min(2 * c->resident_pause, kLongestRest);
+}
+static void resident_solved(Ctx* c, Place at) {
+  c->resident_launches[at]++;
+  if (c->resident_rest == 0) c->resident_pause = kFirstRest;
+}
+// before a solve that may be one launch: back to the fastest path once the rest is over
+static void resident_turn(Ctx* c) {
+  if (c->resident_rest == 0 || --c->resident_rest > 0) return;
+  c->one_xcd = c->may_one_xcd;
+  c->pcg_resident = c->may_pcg_resident;
 }
 
 // Launches, waits and takes the results; *ran = false if the launch gave up.
@@ -915,7 +948,7 @@ static int resident_run(Ctx* c, const double* b, const double* fint, const void*
   // an iteration takes at most two epochs
   c->gslot_epoch += (*ran ? (uint32_t)ps.k : 2 * (uint32_t)pcg_maxiter(c) + 5) + 1;
   if (*ran) {
-    c->resident_launches[at]++;
+    resident_solved(c, at);
     pcg_result(ps, iters, relres, converged, breakdown);
     return ONSAS_OK;
   }
@@ -923,15 +956,19 @@ static int resident_run(Ctx* c, const double* b, const double* fint, const void*
   return clear_abort(c);
 }
 
-inline bool pcg_resident_now(const Ctx* c) {
-  return c->pcg_resident && (c->pcg_device || (c->one_xcd && c->pcg_xcd)) &&
-         c->lin.precond != ONSAS_PRECOND_AMG &&
+inline bool pcg_resident_kind(const Ctx* c) {
+  return c->may_pcg_resident && c->lin.precond != ONSAS_PRECOND_AMG &&
          pcg_maxiter(c) <= kMaxResidentIters;
+}
+inline bool pcg_resident_now(const Ctx* c) {
+  return c->pcg_resident && (c->pcg_device || (c->one_xcd && c->pcg_xcd));
 }
 
 int launch_pcg_resident(Ctx* c, const double* b_dev, bool* ran, int* iters, double* relres,
                         int* converged, int* breakdown) {
   *ran = false;
+  if (!pcg_resident_kind(c)) return ONSAS_OK;
+  resident_turn(c);
   while (!*ran && pcg_resident_now(c))
     ONSAS_TRY(resident_run(c, b_dev, nullptr, nullptr, nullptr, ran, iters, relres, converged,
                            breakdown));
@@ -941,7 +978,9 @@ int launch_pcg_resident(Ctx* c, const double* b_dev, bool* ran, int* iters, doub
 int launch_newton_resident(Ctx* c, const void* x0, void* warm, bool* ran, int* iters,
                            double* relres, int* converged, int* breakdown) {
   *ran = false;
-  while (!*ran && pcg_resident_now(c) && c->lin.kind != ONSAS_LINSOLVE_GMRES) {
+  if (!pcg_resident_kind(c) || c->lin.kind == ONSAS_LINSOLVE_GMRES) return ONSAS_OK;
+  resident_turn(c);
+  while (!*ran && pcg_resident_now(c)) {
     const double prev_b2 = c->h_sc->nwt.prev_b2;
     ONSAS_TRY(resident_run(c, c->d_fext, c->d_fint, x0, warm, ran, iters, relres, converged,
                            breakdown));
@@ -963,41 +1002,44 @@ int launch_gmres_resident(Ctx* c, const double* b_dev, int m, int maxiter, doubl
                           int* iters, double* relres, int* converged) {
   *ran = false;
   const int L = lanes_per_row(c), R = kGmresThreads / L;
-  if (!c->pcg_resident || m > kGmresMax || maxiter > kMaxResidentIters ||
+  if (!c->may_pcg_resident || m > kGmresMax || maxiter > kMaxResidentIters ||
       (c->nn + R - 1) / R > kMaxGridWg || gmres_lds(m, R, c->kt) > 150 * 1024)
     return ONSAS_OK;
   hipStream_t s = c->stream;
   const size_t bytes = 4 * (size_t)kMaxGridWg * kGmresSlot * sizeof(unsigned long long);
-  if (!c->d_gmslots) {
-    ONSAS_HIP_TRY(c, hipMalloc((void**)&c->d_gmslots, bytes));
-    ONSAS_HIP_TRY(c, hipMemsetAsync(c->d_gmslots, 0, bytes, s));
+  resident_turn(c);
+  while (!*ran && c->pcg_resident) {
+    if (!c->d_gmslots) {
+      ONSAS_HIP_TRY(c, hipMalloc((void**)&c->d_gmslots, bytes));
+      ONSAS_HIP_TRY(c, hipMemsetAsync(c->d_gmslots, 0, bytes, s));
+    }
+    ONSAS_TRY(renew_epochs(c));
+    ONSAS_HIP_TRY(c, hipMemsetAsync(&c->d_sc->pcg, 0, sizeof(PcgState), s));
+    Place at = kOneXcd;
+    if (c->precision == ONSAS_PRECISION_FP64)
+      ONSAS_TRY(L == 4 ? (gmres_t<double, 4>(c, b_dev, m, maxiter, rtol, &at))
+                       : (gmres_t<double, 8>(c, b_dev, m, maxiter, rtol, &at)));
+    else
+      ONSAS_TRY(L == 4 ? (gmres_t<float, 4>(c, b_dev, m, maxiter, rtol, &at))
+                       : (gmres_t<float, 8>(c, b_dev, m, maxiter, rtol, &at)));
+    if (at == kGaveUp) return ONSAS_OK;
+    ONSAS_HIP_TRY(c, hipMemcpyAsync(&c->h_sc->pcg, &c->d_sc->pcg, sizeof(PcgState),
+                                    hipMemcpyDeviceToHost, s));
+    ONSAS_HIP_TRY(c, hipStreamSynchronize(s));
+    const PcgState& ps = c->h_sc->pcg;
+    *ran = !ps.aborted;
+    // an iteration takes at most 3 epochs, a restart 3
+    c->gslot_epoch += (*ran ? (uint32_t)ps.k : 6u * ((uint32_t)maxiter + 2)) + 4;
+    if (*ran) {
+      resident_solved(c, at);
+      *iters = ps.iters;
+      *relres = ps.bb > 0 ? std::sqrt(ps.rr_last / ps.bb) : 0.0;
+      *converged = ps.converged;
+    } else {
+      resident_failed(c, at);
+      ONSAS_TRY(clear_abort(c));
+    }
   }
-  ONSAS_TRY(renew_epochs(c));
-  ONSAS_HIP_TRY(c, hipMemsetAsync(&c->d_sc->pcg, 0, sizeof(PcgState), s));
-  Place at = kOneXcd;
-  if (c->precision == ONSAS_PRECISION_FP64)
-    ONSAS_TRY(L == 4 ? (gmres_t<double, 4>(c, b_dev, m, maxiter, rtol, &at))
-                     : (gmres_t<double, 8>(c, b_dev, m, maxiter, rtol, &at)));
-  else
-    ONSAS_TRY(L == 4 ? (gmres_t<float, 4>(c, b_dev, m, maxiter, rtol, &at))
-                     : (gmres_t<float, 8>(c, b_dev, m, maxiter, rtol, &at)));
-  if (at == kGaveUp) return ONSAS_OK;
-  ONSAS_HIP_TRY(c, hipMemcpyAsync(&c->h_sc->pcg, &c->d_sc->pcg, sizeof(PcgState),
-                                  hipMemcpyDeviceToHost, s));
-  ONSAS_HIP_TRY(c, hipStreamSynchronize(s));
-  const PcgState& ps = c->h_sc->pcg;
-  // an iteration takes at most 3 epochs, a restart 3
-  c->gslot_epoch += (ps.aborted ? 6u * ((uint32_t)maxiter + 2) : (uint32_t)ps.k) + 4;
-  if (ps.aborted) {
-    resident_failed(c, at);
-    ONSAS_TRY(clear_abort(c));
-    return launch_gmres_resident(c, b_dev, m, maxiter, rtol, ran, iters, relres, converged);
-  }
-  c->resident_launches[at]++;
-  *ran = true;
-  *iters = ps.iters;
-  *relres = ps.bb > 0 ? std::sqrt(ps.rr_last / ps.bb) : 0.0;
-  *converged = ps.converged;
   return ONSAS_OK;
 }
 

@@ -103,3 +103,21 @@ def test_both_meeting_places_give_the_same_bits(monkeypatch, prec):
         at2, x2 = s.run()
     assert (at, at2) == ({"one_xcd": 1}, {"across_device": 1})
     assert np.array_equal(x, x2)
+
+
+@pytest.mark.parametrize("kind", [PCG, GMRES])
+@pytest.mark.parametrize("prec", [MIXED, FP64])
+def test_a_context_comes_back_to_the_fast_path(monkeypatch, prec, kind):
+    """Two launches without patience (one XCD, then the device): the context rests for 128
+    solves on the general kernels and then stays on the fast path.  With one, it meets across
+    the device for 64 solves."""
+    print(f"[gpu] coming back, solver {kind} precision {prec}", flush=True)
+    for launches, rest, meanwhile in ((2, 128, {}), (1, 64, {"across_device": 1})):
+        monkeypatch.setenv("ONSAS_RESIDENT_TICKS", f"-1:{launches}")
+        with Solves("10x10x10", prec, kind) as s:
+            first = s.run()[0]
+            assert first.pop("gave_up") == launches and first == meanwhile
+            for _ in range(rest - 1):
+                assert s.run()[0] == meanwhile
+            for _ in range(2):
+                assert s.run()[0] == {"one_xcd": 1}
