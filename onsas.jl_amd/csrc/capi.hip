@@ -3,13 +3,11 @@
 // one Newton iteration; the numerics live in element_kernels.hip and
 // solver_kernels.hip, the setup in setup.hip.
 #include <algorithm>
-#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <iterator>
 #include <mutex>
 #include <string>
-#include <thread>
 #include <vector>
 
 #include "engine.hpp"
@@ -90,86 +88,27 @@ int upload_state(Ctx* c, double* d_dst, const double* src) {
   return ONSAS_OK;
 }
 
-// Results to host arrays.  The runtime's copy to pageable memory is bound by one
-// thread reading the staging memory the GPU has just written (about 16 GB/s, where
-// the link gives 50): large results go through a pinned ring whose slots
-// kCopyThreads threads empty while the next chunks are on the way.  48 MB of
-// stresses and strains with the assembly that precedes them: 3.15 ms on the
-// runtime's path, 1.83 ms here (1.88 ms with 2 threads, 2.2 to 2.3 ms with 1 MB
-// chunks and 4 to 8 threads, each array for itself).  Below kParallelCopy bytes the
-// runtime's path is the faster one (no threads to start, no ring to make).
-constexpr size_t kParallelCopy = size_t(8) << 20, kCopyChunk = size_t(2) << 20;
-constexpr int kCopyThreads = 4, kCopySlots = Ctx::kCopySlots;
-static_assert(kCopySlots % kCopyThreads == 0, "a slot belongs to one thread");
+// Results to host arrays; returns once every value is in its array.  Large ones go
+// through the ring (copy_ring.hpp), and the runtime's way where there is none to be had.
+// Stresses and strains of 2 / 4 / 6 / 8 / 16 MiB take 0.12 / 0.35 / 0.46 / 0.57 / 1.10 ms
+// the runtime's way and 0.16 / 0.39 / 0.41 / 0.47 / 0.70 ms with the ring (threads to
+// start), a new context's first 9 / 32 MiB 1.6 / 2.4 and 1.3 / 1.5 ms.
+constexpr size_t kParallelCopy = size_t(8) << 20;
 
-struct HostPart {
-  void* dst;
-  const void* d_src;
-  size_t bytes;
-};
-
-// returns once every value is in its array
-int download(Ctx* c, const std::vector<HostPart>& parts) {
+int download(Ctx* c, const std::vector<onsas::CopyPart>& parts) {
   size_t total = 0;
-  for (const HostPart& p : parts) total += p.bytes;
-  auto plain = [&]() -> int {
-    for (const HostPart& p : parts)
-      ONSAS_HIP_TRY(c, hipMemcpyAsync(p.dst, p.d_src, p.bytes, hipMemcpyDeviceToHost, c->stream));
-    ONSAS_HIP_TRY(c, hipStreamSynchronize(c->stream));
-    return ONSAS_OK;
-  };
-  if (total < kParallelCopy) return plain();
-  if (!c->h_ring) {
-    ONSAS_HIP_TRY(c, hipHostMalloc((void**)&c->h_ring, kCopySlots * kCopyChunk, hipHostMallocDefault));
-    for (auto& e : c->ev_ring) ONSAS_HIP_TRY(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  for (const auto& p : parts) total += p.bytes;
+  if (total >= kParallelCopy) {
+    onsas::HipCopy api{c->stream};
+    const auto r = c->ring.copy(api, parts);
+    if (r == c->ring.kDone) return ONSAS_OK;
+    if (r == c->ring.kFailed)
+      return set_err(c, ONSAS_ERR_HIP, std::string("copy to the host failed: ") +
+                                           hipGetErrorString((hipError_t)api.error.load()));
   }
-  std::vector<HostPart> chunks;
-  for (const HostPart& p : parts)
-    for (size_t o = 0; o < p.bytes; o += kCopyChunk)
-      chunks.push_back({(char*)p.dst + o, (const char*)p.d_src + o, std::min(kCopyChunk, p.bytes - o)});
-  const int64_t n = (int64_t)chunks.size();
-  std::atomic<int64_t> issued{0};          // chunks whose transfer is queued
-  std::atomic<int64_t> taken[kCopySlots];  // per slot: chunks copied out of it
-  for (auto& q : taken) q = 0;
-  std::atomic<bool> failed{false};
-  // chunk i lives in slot i % kCopySlots and belongs to thread i % kCopyThreads
-  auto work = [&](int w) {
-    for (int64_t i = w; i < n; i += kCopyThreads) {
-      while (issued.load(std::memory_order_acquire) <= i && !failed) std::this_thread::yield();
-      if (failed) return;
-      const int k = (int)(i % kCopySlots);
-      if (hipEventSynchronize(c->ev_ring[k]) != hipSuccess) {
-        failed = true;
-        return;
-      }
-      std::memcpy(chunks[i].dst, c->h_ring + k * kCopyChunk, chunks[i].bytes);
-      taken[k].fetch_add(1, std::memory_order_release);
-    }
-  };
-  std::vector<std::thread> threads;
-  threads.reserve(kCopyThreads);
-  try {
-    for (int w = 0; w < kCopyThreads; ++w) threads.emplace_back(work, w);
-  } catch (...) {  // no thread to be had: the runtime's path
-    failed = true;
-    for (auto& t : threads) t.join();
-    return plain();
-  }
-  hipError_t e = hipSuccess;
-  for (int64_t i = 0; i < n && e == hipSuccess && !failed; ++i) {
-    const int k = (int)(i % kCopySlots);
-    while (taken[k].load(std::memory_order_acquire) < i / kCopySlots && !failed) std::this_thread::yield();
-    e = hipMemcpyAsync(c->h_ring + k * kCopyChunk, chunks[i].d_src, chunks[i].bytes,
-                       hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess) e = hipEventRecord(c->ev_ring[k], c->stream);
-    if (e == hipSuccess) issued.store(i + 1, std::memory_order_release);
-  }
-  if (e != hipSuccess) failed = true;
-  for (auto& t : threads) t.join();
-  if (failed) {
-    (void)hipStreamSynchronize(c->stream);
-    return set_err(c, ONSAS_ERR_HIP, std::string("copy to the host failed: ") + hipGetErrorString(e));
-  }
+  for (const auto& p : parts)
+    ONSAS_HIP_TRY(c, hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, c->stream));
+  ONSAS_HIP_TRY(c, hipStreamSynchronize(c->stream));
   return ONSAS_OK;
 }
 
@@ -423,9 +362,8 @@ void onsas_destroy(onsas_ctx* ctx) {
   for (auto& e : c->ev_snap_dev)
     if (e) (void)hipEventDestroy(e);
   if (c->h_stage) (void)hipHostFree(c->h_stage);
-  if (c->h_ring) (void)hipHostFree(c->h_ring);
-  for (auto& e : c->ev_ring)
-    if (e) (void)hipEventDestroy(e);
+  onsas::HipCopy api{c->stream};
+  c->ring.destroy(api);
   for (double* h : c->h_snap)
     if (h) (void)hipHostFree(h);
   for (auto& bank : c->d_warm)
@@ -898,7 +836,7 @@ int element_outputs(Ctx* c, int32_t group, const double* U, double* f, double* K
   if (stress) ONSAS_TRY(to_device(c, ds, nullptr, ne * 9));
   if (strain) ONSAS_TRY(to_device(c, de, nullptr, ne * 9));
   ONSAS_TRY(onsas::launch_element_outputs(c, group, U, df.p, dK.p, ds.p, de.p));
-  std::vector<HostPart> parts;
+  std::vector<onsas::CopyPart> parts;
   if (f) parts.push_back({f, df.p, ne * nd * sizeof(double)});
   if (K) parts.push_back({K, dK.p, ne * nd * nd * sizeof(double)});
   if (stress) parts.push_back({stress, ds.p, ne * 9 * sizeof(double)});

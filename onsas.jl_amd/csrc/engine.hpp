@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "../../include/onsas_hip.h"
+#include "copy_ring.hpp"
 #include "grid_exchange.hpp"
 #include "host_setup.hpp"
 #include "inner_tol.hpp"
@@ -47,6 +48,34 @@ enum GroupType { kTet = 0, kTruss = 1 };
 
 // Uniform grid over a tet group's bounding box for point location: bin b
 // lists (in user element order) the elements whose bounding box overlaps it.
+// The copies of a CopyRing, on a stream.  A refusal (of pinned memory, an event) leaves no
+// error behind for the next launch's check to find.
+struct HipCopy {
+  using Event = hipEvent_t;
+  hipStream_t stream;
+  std::atomic<int> error{hipSuccess};  // the first of a copy
+  explicit HipCopy(hipStream_t s) : stream(s) {}
+  bool ok(hipError_t e) {
+    int none = hipSuccess;
+    if (e != hipSuccess) error.compare_exchange_strong(none, e);
+    return e == hipSuccess;
+  }
+  bool had(hipError_t e) {
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e == hipSuccess;
+  }
+  bool pinned(char** p, size_t n) { return had(hipHostMalloc((void**)p, n, hipHostMallocDefault)); }
+  void free_pinned(char* p) { (void)hipHostFree(p); }
+  bool make(Event* e) { return had(hipEventCreateWithFlags(e, hipEventDisableTiming)); }
+  void destroy(Event e) { (void)hipEventDestroy(e); }
+  bool queue(char* pinned, const void* src, size_t n) {
+    return ok(hipMemcpyAsync(pinned, src, n, hipMemcpyDeviceToHost, stream));
+  }
+  bool record(Event e) { return ok(hipEventRecord(e, stream)); }
+  bool wait(Event e) { return ok(hipEventSynchronize(e)); }
+  void drain() { (void)hipStreamSynchronize(stream); }
+};
+
 struct LocateGrid {
   bool built = false;
   double lo[3] = {0, 0, 0}, inv_h[3] = {0, 0, 0};
@@ -303,10 +332,7 @@ struct Ctx {
   Scalars* d_sc = nullptr;
   Scalars* h_sc = nullptr;   // pinned
   double* h_stage = nullptr;  // pinned, 3 nn values: staging of state vector copies
-  // pinned ring of the large downloads (made by the first one), an event per slot
-  static constexpr int kCopySlots = 8;
-  char* h_ring = nullptr;
-  hipEvent_t ev_ring[kCopySlots] = {};
+  CopyRing<HipCopy> ring;     // of the large downloads (made by the first one)
   double* h_snap[2] = {};     // pinned, 3 nn values each: U snapshots (onsas_snapshot_U)
   hipEvent_t ev_snap[2] = {};  // ... their copies' completion
   // A snapshot copies U on the stream into d_snap (device to device, a few
