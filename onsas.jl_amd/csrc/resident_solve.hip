@@ -19,10 +19,15 @@
 // with it (kPqError), and p.q is summed from p and q where that has grown, and before
 // every breakdown.  z needs no sum to be safe to read: a node that
 // is not there yet carries an old epoch.
-// An iteration takes 2.3 us at 1,680 nodes (27 workgroups, met in one XCD), 1.1 us at
-// 125 nodes (one workgroup, z and the sums in LDS).  Met in device memory it is 3.4 us;
-// with p.q and (r.z, r.r) as two sums, z safe to read only after the second, a tree per
-// sum and 4- and 8-byte loads it was 4.6 and 2.6 us.  Polling by every wave of a
+// An iteration takes 2.4 us at 1,680 nodes (27 workgroups, met in one XCD; FP64 2.7 us),
+// 1.0 us at 125 nodes (one workgroup, z and the sums in LDS; FP64 1.2 us).  Met in device
+// memory it is 3.4 us; with p.q and (r.z, r.r) as two sums, z safe to read only after the
+// second, a tree per sum and 4- and 8-byte loads it was 4.6 and 2.6 us.  A pipelined
+// recurrence (P. Ghysels and W. Vanroose, Parallel Comput. 40, 2014) would hide the sum
+// behind the product, but loses the residual: on the host, for a 13 x 9 x 11 box, it
+// stalls at a true residual of 2.5e-2 in FP32 (1e-5 here, rtol 1e-6) and takes 409 for 314
+// iterations to 2e-10 for 8e-13 in FP64 (rtol 1e-12); the residual computed anew every 50
+// iterations mends FP64 and not FP32.  Polling by every wave of a
 // workgroup instead of one costs 1 us.
 #include <unistd.h>
 
@@ -103,8 +108,8 @@ __device__ inline void host_store(T* p, T v) {
 // warm start, stopping tolerance, solve, update of U and norms (k_residual,
 // k_spmv_sell, k_warm_dots, k_warm_init, k_pcg_init_finalize, k_update and
 // k_finalize_newton of the general path, with two copies to the host and one on
-// the device: some 60 us of a step of 195 us at 125 nodes, now 5 us; the step
-// 195 -> 152 us).
+// the device: some 60 us of a step of 195 us at 125 nodes, now 5 us; the step 195 ->
+// 152 us, and 143 us since the assembly stamps its own events).
 //
 // The sums take two slot regions in turn: a workgroup may be in sum k + 1 while
 // another still reads sum k.  z has one buffer: the sum before its next hand-over is
@@ -374,7 +379,9 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs<KT> a) {
 // Gram-Schmidt passes (a value per basis vector, four threads a value).  |w| after
 // the second pass comes with it: |w|^2 before it less the squares of its
 // coefficients, all summed in FP64; where these take most of |w|^2 away it is
-// summed again.  The rotations run while t is under way.  With |w| as an exchange
+// summed again.  It lacks the rounding of the stored w, whose entries' errors average
+// out: basis vectors of three boxes (a host model, 60 each) have a norm within 0.09 u of
+// one in FP32 with either sum, and within 0.10 u instead of 0.08 u in FP64.  The rotations run while t is under way.  With |w| as an exchange
 // of its own and slots polled one after the other an iteration was 14.5 us.
 constexpr int kGmresThreads = 256;
 constexpr int kGmresMax = 60;    // most basis vectors of the resident kernel (four threads each)
@@ -675,7 +682,8 @@ constexpr int kResidentBlocks = 4;  // blocks a lane keeps in registers
 // kernels an iteration; of 4,913 / 6,859 / 8,000 nodes 9.4 / 12.9 / 13.7 ms with 256 (the
 // first in one XCD) and 13.6 / 13.8 / 15.7 ms with 512, which are left for more than
 // kMaxGridWg workgroups of 256.  The single workgroup gathers from LDS: 512 threads, and
-// in FP32 1024 where the rows need them (125 nodes: 1.8 us an iteration against 2.6).
+// in FP32 1024 where the rows need them (125 nodes: 1.0 us an iteration against 2.0 on
+// several workgroups, 252 nodes: 1.7 against 2.2; FP64, 125 nodes: 1.2 against 2.5).
 constexpr int kResidentThreads = 256;
 constexpr int resident_one_threads(size_t kt) { return kt == 4 ? 1024 : 512; }
 
